@@ -14,6 +14,11 @@ namespace gdn {
 // stated.  The backward-only buffers are NULL in a plain forward call.
 struct ChunkWs {
   int32_t* off;     // [N+1] first global chunk of each sequence
+  int32_t* soff;    // [N+1] first segment of each sequence (cu_seqlens and segments)
+  float* segs;      // [segments][Hv][K][V] a segment's own contribution to the state, then
+                    // the state after it
+  u16x8* segm;      // [segments][Hv][hi, lo][K/16][K/32][64] a segment's transfer matrix M
+                    // as bf16 A-operand fragments, M = hi + lo (rows in rho order)
   int32_t* status;  // [1] 0, or the cu_seqlens violation the chunk table found
   float* gate;      // [NC][Hv][64]: G_i, the chunk-local cumulative log-decay
   u16x8* tfrag;     // [NC][Hv][6 slots][64 lanes] fp16 A-operand fragments of Tb,
@@ -191,6 +196,9 @@ inline bool chain_reads_rows(bool bwd, bool l2, int N, int Hv, int V) {
 // Workspace plan (byte offsets into the caller's buffer).
 struct WsPlan {
   size_t off, status, gate, tfrag, pfrag, k16, q16, qn, kn, total;
+  size_t soff, segs, segm;
+  int seg, nseg;   // chunks per segment (0: none), segments of all sequences at most
+  bool whole_head;   // the forward chain takes the whole-head form (gdn_chunk_head.hip)
   bool k16_copy, q16_copy;   // k16 / q16 planned (else the chains read the caller's rows)
   // backward only (0 when not planned)
   size_t tmat, ttfrag, ptfrag, qtfrag, hs, dl, dse, dd;
@@ -198,7 +206,7 @@ struct WsPlan {
 };
 
 WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, bool l2,
-               bool bwd);
+               bool bwd, bool segments = true);
 
 // What a forward launch sequence writes: kForward = o / ht only; kRecompute =
 // the backward's inputs only (prep adds tmat / ttfrag / ptfrag, the chain
@@ -223,6 +231,15 @@ void launch_chain_sw(const uint16_t* v, const uint16_t* qraw, const uint16_t* kr
                      const float* h0, float* ht, uint16_t* o, const int32_t* cu, int N, int T,
                      int total, int Hqk, int Hv, int V, float scale, const ChunkWs& ws,
                      hipStream_t st);
+
+// Forward chain, whole-head form (gdn_chunk_head.hip), in segments where the
+// plan has them: the same results and buffers, K and Q from the caller's rows
+// or (l2) from ws.k16 / ws.q16.
+template <int K, bool SAVE, bool OUT>
+void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, const float* h0,
+                       float* ht, uint16_t* o, const int32_t* cu, int N, int T, int total, int Hqk,
+                       int Hv, int V, float scale, bool l2, const WsPlan& p, const ChunkWs& ws,
+                       hipStream_t st);
 
 // Reverse chain of the backward (gdn_chunk_rev.hip): dS' of every chunk into
 // dse, dd into dd, dh0 (K rows from ws.k16).

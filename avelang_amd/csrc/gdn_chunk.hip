@@ -15,7 +15,7 @@
 //   o     = scale * e^G * (Q S) + P vnew
 //   S     = e^G_L S + K^T (e^(G_L - G) * vnew)
 //
-// Three launches:
+// Three launches (segments of few long chains: five):
 //   chunk_table_kernel  sequence -> first-chunk offsets (varlen plumbing)
 //   chunk_prep_kernel   one workgroup per (chunk, v-head), fully parallel:
 //                       K K^T and Q K^T on MFMA, blocked UT inverse in fp32,
@@ -27,12 +27,17 @@
 //                       sequence's chunks; one wave holds the fp32 state slice
 //                       in VGPRs for the whole sequence, every product is a
 //                       16x16x32 fp16 MFMA, and two more waves stage operands
-//                       and form the output.
+//                       and form the output.  Many chains, or the segments
+//                       of few long ones, take chunk_head_kernel
+//                       (gdn_chunk_head.hip) instead: a workgroup per (sequence
+//                       or segment, v-head); chain_form() has the rule.
 // Precision: every chain product takes fp16 operands rounded from fp32 (one
 // MFMA pass each; fp16's 11-bit significand keeps the final state within
 // ~4e-4 relative Frobenius at any sequence length, against ~3e-3 for single
 // bf16).  Operands stay far inside fp16's range for l2-normalised q / k and
 // v of the magnitudes a layer produces.
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -48,9 +53,11 @@ namespace gdn {
 // outputs are zero-filled by zero_on_violation_kernel.
 __global__ __launch_bounds__(256) void chunk_table_kernel(const int32_t* __restrict__ cu,
                                                           int N, int T, int total,
-                                                          int ncmax, int32_t* __restrict__ off,
+                                                          int ncmax, int seg,
+                                                          int32_t* __restrict__ off,
+                                                          int32_t* __restrict__ soff,
                                                           int32_t* __restrict__ status) {
-  __shared__ int part[257];
+  __shared__ int part[257], spart[257];
   __shared__ int bad;
   const int tid = threadIdx.x;
   const int per = (N + 255) / 256;
@@ -61,32 +68,49 @@ __global__ __launch_bounds__(256) void chunk_table_kernel(const int32_t* __restr
     if (cu[n + 1] < cu[n]) atomicMax(&bad, 2);
   __syncthreads();
   if (bad) {
-    for (int n = tid; n <= N; n += 256) off[n] = 0;
+    for (int n = tid; n <= N; n += 256) {
+      off[n] = 0;
+      if (seg) soff[n] = n;
+    }
     if (tid == 0) *status = bad;
     return;
   }
   if (tid == 0) *status = 0;
-  int sum = 0;
+  // (with segments of `seg` chunks also their first-segment offsets, at
+  // least one segment per sequence)
+  int sum = 0, ssum = 0;
   for (int n = a; n < b; ++n) {
     int s, e;
     seq_bounds(cu, n, T, total, s, e);
-    sum += (e - s + kChunk - 1) / kChunk;
+    const int nc = (e - s + kChunk - 1) / kChunk;
+    sum += nc;
+    if (seg) ssum += max(1, (nc + seg - 1) / seg);
   }
   part[tid + 1] = sum;
+  spart[tid + 1] = ssum;
   __syncthreads();
   if (tid == 0) {
-    part[0] = 0;
-    for (int i = 1; i <= 256; ++i) part[i] += part[i - 1];
+    part[0] = spart[0] = 0;
+    for (int i = 1; i <= 256; ++i) {
+      part[i] += part[i - 1];
+      spart[i] += spart[i - 1];
+    }
   }
   __syncthreads();
-  int run = part[tid];
+  int run = part[tid], srun = spart[tid];
   for (int n = a; n < b; ++n) {
     off[n] = min(run, ncmax);
+    if (seg) soff[n] = srun;
     int s, e;
     seq_bounds(cu, n, T, total, s, e);
-    run += (e - s + kChunk - 1) / kChunk;
+    const int nc = (e - s + kChunk - 1) / kChunk;
+    run += nc;
+    if (seg) srun += max(1, (nc + seg - 1) / seg);
   }
-  if (tid == 255) off[N] = min(part[256], ncmax);
+  if (tid == 255) {
+    off[N] = min(part[256], ncmax);
+    if (seg) soff[N] = spart[256];
+  }
 }
 
 __global__ __launch_bounds__(256) void zero_on_violation_kernel(const int32_t* __restrict__ status,
@@ -506,12 +530,59 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(
 // ------------------------------------------------------------- host ----
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// The forward chain's form for W = N Hv chains of about nct chunks each, and
+// for the whole-head form the chunks per segment (0: whole sequences).
+//
+// The state-wave form (a workgroup per 16 value columns) goes through a chunk
+// in ~0.86 us while W x 8 workgroups leave compute units free, the whole-head
+// form in ~1.9 us with an eighth of the operand traffic.  So the latter pays
+//  - unsegmented once W fills half the GPU: W = 128 (4 x 32 heads of T = 4096)
+//    276 -> 237 us per prefill, W = 256 (8 x 32 of 2048) 282 -> 187, 64 packed
+//    sequences x 32 heads 2298 -> 1490; at W = 64 it loses (128 -> 159).  With
+//    64-wide heads from W = 256 on (143 -> 107; at 128 64 -> 72);
+//  - in segments for few long chains, whose segments' two passes run in
+//    parallel: W = 4, T = 4096 62 -> 53, 16384 219 -> 88; W = 8, 8192
+//    120 -> 77; W = 16, 8192 127 -> 101; W = 32, 16384 390 -> 283; at
+//    W = 32, T = 8192 it loses (142 -> 150), at T = 2048 everywhere (W = 4
+//    36 -> 43).  64-wide heads: W = 16, 4096 58 -> 41; W = 32, 8192 101 -> 83.
+// The segment count balances the passes over a segment (~3.8 us per chunk)
+// against the serial combine (~1.1 us per segment) and fills the GPU at most
+// once.  With cu_seqlens nct is the mean; an unsegmented form still cuts a
+// sequence much longer than that, which would otherwise run on its own.
+static void chain_form(long long ncmax, long long nctotal, int N, int Hv, int K, int V,
+                       bool has_cu, bool segments, WsPlan& p) {
+  p.seg = 0;
+  p.whole_head = false;
+  if (N <= 0 || ncmax <= 0) return;
+  const long long W = (long long)N * Hv, cus = device_cus();
+  const long long nct = std::max(1LL, ncmax / N);
+  const bool square = K == V && segments;
+  if (square && 2 * W <= cus && nct >= std::max(64LL, (K == 128 ? 6 : 4) * W)) {
+    const double ns = std::min((double)cus / W, 1.9 * std::sqrt((double)nct));
+    p.seg = (int)std::ceil(nct / ns);
+    p.whole_head = true;
+    return;
+  }
+  p.whole_head = W >= (K == 128 && V == 128 ? cus / 2 : cus);
+  if (p.whole_head && square && has_cu) {
+    const long long seg = std::max(32LL, 4 * nct);
+    if (nctotal > 2 * seg) p.seg = (int)seg;
+  }
+}
+
 WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, bool l2,
-               bool bwd) {
+               bool bwd, bool segments) {
   WsPlan p{};
   const long long total = (long long)B * T;
   p.ncmax = has_cu ? (total + 63LL * N) / 64 : (long long)B * ((T + 63) / 64);
   const size_t nch = (size_t)p.ncmax * Hv;   // (chunk, v-head) pairs
+  if (bwd) {   // a training forward takes the plain forward's form, so that o is the same
+    const WsPlan f = plan_ws(B, T, Hqk, Hv, K, V, N, has_cu, l2, false);
+    p.whole_head = f.whole_head;
+    p.seg = f.seg;
+  } else {
+    chain_form(p.ncmax, (total + 63) / 64, N, Hv, K, V, has_cu, segments, p);
+  }
   size_t at = 0;
   auto take = [&](size_t bytes) {
     const size_t here = at;
@@ -524,10 +595,10 @@ WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, 
   p.tfrag = take(nch * 6 * 64 * 16);
   p.pfrag = take(nch * 6 * 64 * 16);
   // the fp16 K / Q copies, where the chains do not read the caller's rows:
-  // Q only with use_qk_l2norm (normalised), K also for the backward and for
-  // two V tiles per workgroup
+  // Q only with use_qk_l2norm (normalised), K also for the backward's reverse
+  // chain and for two V tiles per workgroup of the state-wave form
   const size_t nqk = (size_t)p.ncmax * Hqk;   // (chunk, qk-head) pairs
-  p.k16_copy = !chain_reads_rows(bwd, l2, N, Hv, V);
+  p.k16_copy = bwd || l2 || (!p.whole_head && !chain_reads_rows(bwd, l2, N, Hv, V));
   p.q16_copy = l2;
   p.k16 = take(p.k16_copy ? nqk * (K == 128 ? KLayout<128>::BYTES : KLayout<64>::BYTES) : 0);
   p.q16 = take(p.q16_copy ? nqk * 64 * K * 2 : 0);
@@ -546,7 +617,20 @@ WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, 
     p.dd = take(nch * 64 * V * 2);
     p.qtfrag = take((size_t)p.ncmax * Hqk * (K / 16) * 2 * 64 * 16);
   }
+  if (p.seg) {
+    p.nseg = (int)(has_cu ? p.ncmax / p.seg + N
+                          : (long long)N * std::max(1LL, ((T + 63) / 64 + p.seg - 1) / (long long)p.seg));
+    p.soff = take((size_t)(N + 1) * 4);
+    p.segs = take((size_t)p.nseg * Hv * K * V * 4);
+    p.segm = take((size_t)p.nseg * Hv * K * K * 4);
+  }
   p.total = at;
+  // no segments where their buffers alone would take the problem over the
+  // scratch of gdn_chunk_fwd_noalloc
+  if (p.seg && !bwd && p.total > GDN_NOALLOC_SCRATCH_BYTES) {
+    const WsPlan q = plan_ws(B, T, Hqk, Hv, K, V, N, has_cu, l2, false, false);
+    if (q.total <= GDN_NOALLOC_SCRATCH_BYTES) return q;
+  }
   return p;
 }
 
@@ -561,6 +645,11 @@ ChunkWs ws_pointers(const WsPlan& p, unsigned char* wsb) {
   ws.q16 = p.q16_copy ? reinterpret_cast<u16x8*>(wsb + p.q16) : nullptr;
   ws.qn = reinterpret_cast<uint16_t*>(wsb + p.qn);
   ws.kn = reinterpret_cast<uint16_t*>(wsb + p.kn);
+  if (p.seg) {
+    ws.soff = reinterpret_cast<int32_t*>(wsb + p.soff);
+    ws.segs = reinterpret_cast<float*>(wsb + p.segs);
+    ws.segm = reinterpret_cast<u16x8*>(wsb + p.segm);
+  }
   if (p.hs) {
     ws.tmat = reinterpret_cast<float*>(wsb + p.tmat);
     ws.ttfrag = reinterpret_cast<u16x8*>(wsb + p.ttfrag);
@@ -582,7 +671,7 @@ static void launch_chunk(const uint16_t* q, const uint16_t* k, const uint16_t* v
   const int total = B * T;
   if (cu)
     hipLaunchKernelGGL(chunk_table_kernel, dim3(1), dim3(256), 0, st, cu, N, T, total,
-                       (int)p.ncmax, ws.off, ws.status);
+                       (int)p.ncmax, p.seg, ws.off, ws.soff, ws.status);
   if (p.ncmax > 0) {
     if (l2)
       hipLaunchKernelGGL((chunk_prep_kernel<K, BWD, OUT, true>), dim3((unsigned)p.ncmax, Hv), dim3(256),
@@ -593,7 +682,11 @@ static void launch_chunk(const uint16_t* q, const uint16_t* k, const uint16_t* v
   }
   // the chain reads K and Q as the prep kernel's fp16 copies where the plan
   // has them (normalised with use_qk_l2norm), else as the caller's bf16 rows
-  launch_chain_sw<K, BWD, OUT>(v, ws.q16 ? nullptr : q, ws.k16 ? nullptr : k, h0,
+  if (p.whole_head)
+    launch_chain_head<K, BWD, OUT>(q, k, v, h0, OUT ? ht : nullptr, OUT ? o : nullptr, cu, N, T,
+                                   total, Hqk, Hv, V, scale, l2, p, ws, st);
+  else
+    launch_chain_sw<K, BWD, OUT>(v, ws.q16 ? nullptr : q, ws.k16 ? nullptr : k, h0,
                                OUT ? ht : nullptr, OUT ? o : nullptr, cu, N, T, total, Hqk, Hv,
                                V, scale, ws, st);
   // a cu_seqlens violation left every sequence empty: o is zero-filled (and

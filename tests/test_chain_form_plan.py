@@ -1,0 +1,33 @@
+"""Workspace of the segmented chain form (CPU): segments never take a problem that fits the
+scratch of gdn_chunk_fwd_noalloc over it, and the backward's workspace covers them."""
+import pytest
+
+from avelang_amd import _native
+
+LIMIT = 32 << 20
+
+
+def _plain(T, Hqk, Hv, K, l2):
+    """Bytes without segments: per (chunk, v-head) G and the Tb, P fragments; with l2norm the
+    fp16 K, Q copies per (chunk, qk-head); each buffer rounded up to 256, the two tables too."""
+    n = -(-T // 64)
+    up = lambda x: -(-x // 256) * 256  # noqa: E731
+    return (512 + up(n * Hv * 256) + 2 * up(n * Hv * 6144) +
+            (2 * up(n * Hqk * 64 * K * 2) if l2 else 0))
+
+
+@pytest.mark.parametrize("K", [64, 128])
+@pytest.mark.parametrize("l2", [0, 1])
+@pytest.mark.parametrize("Hqk,Hv", [(1, 2), (2, 4), (4, 8), (16, 16), (16, 32)])
+def test_noalloc_limit_is_kept(Hqk, Hv, K, l2):
+    lib = _native.lib()
+    grown = 0
+    for chunks in list(range(1, 200, 7)) + [256, 300, 500, 700, 1000, 2000]:
+        T = 64 * chunks - 3
+        plain = _plain(T, Hqk, Hv, K, l2)
+        got = lib.gdn_chunk_workspace_bytes(1, T, Hqk, Hv, K, K, 1, 0, l2)
+        assert got >= plain
+        assert (got <= LIMIT) == (plain <= LIMIT), (T, plain, got)
+        grown += got > plain
+        assert lib.gdn_chunk_bwd_workspace_bytes(1, T, Hqk, Hv, K, K, 1, 0, l2) > got
+    assert grown > 0   # some of them do run in segments

@@ -1,0 +1,160 @@
+"""The forward chain's whole-head and segmented forms at the sizes where they
+can go wrong: against the CPU oracles, and against the state-wave form.
+
+Which form a call takes depends on its sizes (chain_form in gdn_chunk.hip):
+from half a workgroup per compute unit on (K = V = 128; a whole one
+otherwise) every (sequence, v-head) is one workgroup, and few long chains are
+cut into segments.  Tolerances: the operator's (o 2e-2 absolute + relative,
+final state 1e-3, gradients 1e-2 relative Frobenius).
+"""
+import numpy as np
+import pytest
+import torch
+
+from avelang_amd import workloads as W
+from oracle import cpu as oracle
+from oracle import gdn_bwd_ref as RB
+
+pytestmark = pytest.mark.gpu
+
+
+def _cus(dev):
+    return torch.cuda.get_device_properties(dev).multi_processor_count
+
+
+def _run(wl, dev, l2=False, fn=None, **kw):
+    from avelang_amd import chunk_gated_delta_rule
+    t = wl.torch(dev)
+    r = (fn or chunk_gated_delta_rule)(
+        t["q"], t["k"], t["v"], t["g"], t["beta"], initial_state=t["initial_state"],
+        output_final_state=True, cu_seqlens=t["cu_seqlens"], use_qk_l2norm_in_kernel=l2, **kw)
+    torch.cuda.synchronize()
+    return r
+
+
+def _check(wl, dev, l2=False, what=""):
+    o, s = _run(wl, dev, l2)
+    a = wl.numpy()
+    if l2:
+        nrm = lambda x: x / np.sqrt((x * x).sum(-1, keepdims=True) + 1e-6)  # noqa: E731
+        a["q"], a["k"] = W._bf16_round(nrm(a["q"])), W._bf16_round(nrm(a["k"]))
+    o_ref, s_ref = oracle.run("chunk", **a)
+    o, s = o.float().cpu().numpy(), s.cpu().numpy()
+    bad = np.abs(o - o_ref) > 2e-2 + 2e-2 * np.abs(o_ref)
+    assert not bad.any(), f"{what}: {bad.sum()} / {bad.size} outputs off"
+    fro = np.linalg.norm(s - s_ref) / max(np.linalg.norm(s_ref), 1e-30)
+    assert fro <= 1e-3, f"{what}: state {fro:.2e}"
+
+
+@pytest.mark.parametrize("K,V,l2", [(128, 128, False), (128, 128, True), (64, 64, False),
+                                    (64, 64, True), (128, 64, False), (64, 128, True)])
+@pytest.mark.parametrize("T", [1, 63, 64, 65, 129, 200])
+def test_whole_head(rocm_device, K, V, l2, T):
+    """Tails of one to 64 tokens, one to four chunks, every head size, GQA 1 / 2 / 4."""
+    Hqk, Hv = {1: (4, 4), 63: (1, 4), 64: (2, 4)}.get(T, (2, 4))
+    B = -(-_cus(rocm_device) // Hv)
+    wl = W.make(B, T, Hqk, Hv, K, V, seed=T, h0_scale=0.01 if T != 65 else 0.0, l2norm=not l2)
+    _check(wl, rocm_device, l2, f"K{K} V{V} T{T}")
+
+
+def _cu(lens):
+    return np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+
+
+def _packed(dev, long=0):
+    """Sequences of 0 to 150 tokens (and one of `long`) over enough heads for the form."""
+    Hv = 8
+    n = -(-_cus(dev) // Hv)
+    rng = np.random.Generator(np.random.PCG64(5))
+    lens = rng.integers(1, 151, size=n)
+    lens[3], lens[n // 2] = 0, long or lens[n // 2]
+    cu = _cu(lens)
+    return W.make(1, int(cu[-1]), 4, Hv, 128, 128, seed=6, cu_seqlens=cu)
+
+
+def test_whole_head_packed(rocm_device):
+    _check(_packed(rocm_device), rocm_device, what="packed")
+
+
+def test_whole_head_packed_with_one_long_sequence(rocm_device):
+    """A sequence far over the mean is cut into segments, the others stay whole."""
+    _check(_packed(rocm_device, long=6011), rocm_device, what="packed, one long")
+
+
+@pytest.mark.parametrize("B,T,Hqk,Hv,D,l2,decay", [
+    (1, 4096, 1, 2, 128, False, 0.1),      # segments divide the chunks or not,
+    (1, 4096 + 1, 2, 2, 128, True, 0.1),   # the last chunk of one token,
+    (2, 5000, 1, 2, 128, False, 0.002),    # and states that carry through many segments
+    (1, 6200, 2, 4, 64, False, 0.002),
+    (2, 4159, 1, 4, 64, True, 0.01)])
+def test_segments(rocm_device, B, T, Hqk, Hv, D, l2, decay):
+    wl = W.make(B, T, Hqk, Hv, D, D, seed=T, decay=decay, h0_scale=0.05, l2norm=not l2)
+    _check(wl, rocm_device, l2, f"segments T{T}")
+
+
+def test_segments_without_an_initial_state(rocm_device):
+    _check(W.make(1, 4500, 1, 2, 128, 128, seed=1, decay=0.01, h0_scale=0.0), rocm_device)
+
+
+@pytest.mark.parametrize("lens", [[9000, 0, 1, 7000], [130, 8200, 5000], [0, 0, 13000]])
+def test_segments_packed(rocm_device, lens):
+    """Sequences of many, one and no segments."""
+    cu = _cu(lens)
+    _check(W.make(1, int(cu[-1]), 1, 2, 128, 128, seed=2, cu_seqlens=cu, decay=0.01,
+                  h0_scale=0.05), rocm_device, what=str(lens))
+
+
+@pytest.mark.parametrize("T,Hv,n", [(9000, 2, 2), (400, 8, 64)])
+def test_violated_cu_seqlens(rocm_device, T, Hv, n):
+    """The device contract in both forms: o zero-filled, the final state the initial one."""
+    wl = W.make(1, T, 1, Hv, 128, 128, seed=3, cu_seqlens=_cu([T // n] * n))
+    t = wl.torch(rocm_device)
+    from avelang_amd import chunk_gated_delta_rule
+    cu = t["cu_seqlens"].clone()
+    cu[1] = T + 5
+    out = torch.full_like(t["v"], 7.0)
+    _, ht = chunk_gated_delta_rule(t["q"], t["k"], t["v"], t["g"], t["beta"],
+                                   initial_state=t["initial_state"], output_final_state=True,
+                                   cu_seqlens=cu, out=out)
+    torch.cuda.synchronize()
+    assert not out.any() and torch.equal(ht, t["initial_state"])
+
+
+def _training(dev, l2):
+    """(workload, what): one of each form."""
+    B = -(-_cus(dev) // 4)
+    yield W.make(B, 70, 2, 4, 128, 128, seed=8, h0_scale=0.01, l2norm=not l2), "whole"
+    yield W.make(1, 4200, 1, 2, 128, 128, seed=9, h0_scale=0.05, decay=0.01,
+                 l2norm=not l2), "segments"
+
+
+@pytest.mark.parametrize("l2", [False, True])
+def test_training_forward_equals_the_plain_one(rocm_device, l2):
+    from avelang_amd import chunk_gated_delta_rule_fwd_save
+    for wl, what in _training(rocm_device, l2):
+        o, s = _run(wl, rocm_device, l2)
+        o2, s2, _ = _run(wl, rocm_device, l2, fn=chunk_gated_delta_rule_fwd_save)
+        assert torch.equal(o, o2) and torch.equal(s, s2), what
+
+
+def test_gradients(rocm_device):
+    """The saved states and deltas of both forms, through the backward; recomputed == saved."""
+    from avelang_amd import chunk_gated_delta_rule_bwd, chunk_gated_delta_rule_fwd_save
+    for wl, what in _training(rocm_device, False):
+        a, t = wl.numpy(), wl.torch(rocm_device)
+        rng = np.random.Generator(np.random.PCG64(1))
+        do = W._bf16_round(rng.standard_normal(a["v"].shape, dtype=np.float32))
+        ref = RB.chunked_bwd(a["q"], a["k"], a["v"], a["g"], a["beta"], do, None,
+                             initial_state=a["initial_state"])
+        args = (t["q"], t["k"], t["v"], t["g"], t["beta"],
+                torch.from_numpy(do).to(device=rocm_device, dtype=torch.bfloat16))
+        _, _, ws = _run(wl, rocm_device, fn=chunk_gated_delta_rule_fwd_save)
+        got = chunk_gated_delta_rule_bwd(*args, initial_state=t["initial_state"], workspace=ws,
+                                         saved=True)
+        again = chunk_gated_delta_rule_bwd(*args, initial_state=t["initial_state"])
+        torch.cuda.synchronize()
+        for name, x, y in zip(("dq", "dk", "dv", "dg", "dbeta", "dh0"), got, again):
+            assert torch.equal(x, y), f"{what}: {name} saved != recomputed"
+            x = x.double().cpu().numpy()
+            rel = np.linalg.norm(x - ref[name]) / np.linalg.norm(ref[name])
+            assert rel <= (1e-3 if name == "dh0" else 1e-2), f"{what}: {name} {rel:.2e}"
