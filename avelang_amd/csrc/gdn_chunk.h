@@ -197,7 +197,9 @@ inline bool chain_reads_rows(bool bwd, bool l2, int N, int Hv, int V) {
 struct WsPlan {
   size_t off, status, gate, tfrag, pfrag, k16, q16, qn, kn, total;
   size_t soff, segs, segm;
-  int seg, nseg;   // chunks per segment (0: none), segments of all sequences at most
+  // chunks per segment (0: none), segments of all sequences at most, and those
+  // among them that another follows
+  int seg, nseg, nfull;
   bool whole_head;   // the forward chain takes the whole-head form (gdn_chunk_head.hip)
   bool k16_copy, q16_copy;   // k16 / q16 planned (else the chains read the caller's rows)
   // backward only (0 when not planned)

@@ -537,18 +537,23 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // in ~0.86 us while W x 8 workgroups leave compute units free, the whole-head
 // form in ~1.9 us with an eighth of the operand traffic.  So the latter pays
 //  - unsegmented once W fills half the GPU: W = 128 (4 x 32 heads of T = 4096)
-//    276 -> 237 us per prefill, W = 256 (8 x 32 of 2048) 282 -> 187, 64 packed
-//    sequences x 32 heads 2298 -> 1490; at W = 64 it loses (128 -> 159).  With
+//    276 -> 220 us per prefill, W = 256 (8 x 32 of 2048) 282 -> 187, 64 packed
+//    sequences x 32 heads 2346 -> 1500; at W = 64 it loses (128 -> 159).  With
 //    64-wide heads from W = 256 on (143 -> 107; at 128 64 -> 72);
 //  - in segments for few long chains, whose segments' two passes run in
-//    parallel: W = 4, T = 4096 62 -> 53, 16384 219 -> 88; W = 8, 8192
-//    120 -> 77; W = 16, 8192 127 -> 101; W = 32, 16384 390 -> 283; at
-//    W = 32, T = 8192 it loses (142 -> 150), at T = 2048 everywhere (W = 4
-//    36 -> 43).  64-wide heads: W = 16, 4096 58 -> 41; W = 32, 8192 101 -> 83.
-// The segment count balances the passes over a segment (~3.8 us per chunk)
-// against the serial combine (~1.1 us per segment) and fills the GPU at most
-// once.  With cu_seqlens nct is the mean; an unsegmented form still cuts a
-// sequence much longer than that, which would otherwise run on its own.
+//    parallel: W = 4, T = 4096 62 -> 54, 16384 219 -> 88; W = 8, 8192
+//    120 -> 72; W = 16, 8192 127 -> 94; W = 32, 8192 143 -> 138 (other inputs
+//    each call: 177 -> 150), 16384 390 -> 273, 65536 1593 -> 1061; W = 64,
+//    32768 1077 -> 963; at T = 2048 it loses everywhere (W = 4 36 -> 43), at
+//    W = 16, T = 4096 it is even.
+//    64-wide heads: W = 16, 4096 58 -> 44; W = 32, 8192 101 -> 86.
+// The segment count fills the GPU once with the first pass's workgroups (two
+// per segment but the last, one per compute unit, 64-wide heads' two; at
+// W = 32, T = 8192 5 segments 138 us, 4 155, 6 159, 8 152), and balances the
+// passes over a segment (~3.5 us per chunk) against the serial combine (~1.1
+// us per segment; W = 4, T = 20011 25 segments 97 us, 16 106, 12 120).
+// With cu_seqlens nct is the mean; an unsegmented form still cuts a sequence
+// much longer than that, which would otherwise run on its own.
 static void chain_form(long long ncmax, long long nctotal, int N, int Hv, int K, int V,
                        bool has_cu, bool segments, WsPlan& p) {
   p.seg = 0;
@@ -557,15 +562,16 @@ static void chain_form(long long ncmax, long long nctotal, int N, int Hv, int K,
   const long long W = (long long)N * Hv, cus = device_cus();
   const long long nct = std::max(1LL, ncmax / N);
   const bool square = K == V && segments;
-  if (square && 2 * W <= cus && nct >= std::max(64LL, (K == 128 ? 6 : 4) * W)) {
-    const double ns = std::min((double)cus / W, 1.9 * std::sqrt((double)nct));
+  if (square && 2 * W <= cus && nct >= (W <= 8 ? 64 : std::max(72LL, 4 * W))) {
+    const double fill = K == 128 ? (double)cus / (2 * W) + 1 : (double)cus / W;
+    const double ns = std::min(fill, 1.5 * std::sqrt((double)nct));
     p.seg = (int)std::ceil(nct / ns);
     p.whole_head = true;
     return;
   }
   p.whole_head = W >= (K == 128 && V == 128 ? cus / 2 : cus);
   if (p.whole_head && square && has_cu) {
-    const long long seg = std::max(32LL, 4 * nct);
+    const long long seg = std::max(64LL, 6 * nct);
     if (nctotal > 2 * seg) p.seg = (int)seg;
   }
 }
@@ -618,19 +624,14 @@ WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, 
     p.qtfrag = take((size_t)p.ncmax * Hqk * (K / 16) * 2 * 64 * 16);
   }
   if (p.seg) {
-    p.nseg = (int)(has_cu ? p.ncmax / p.seg + N
-                          : (long long)N * std::max(1LL, ((T + 63) / 64 + p.seg - 1) / (long long)p.seg));
+    const long long per = std::max(1LL, ((T + 63LL) / 64 + p.seg - 1) / p.seg);
+    p.nfull = (int)(has_cu ? p.ncmax / p.seg : N * (per - 1));
+    p.nseg = p.nfull + N;
     p.soff = take((size_t)(N + 1) * 4);
     p.segs = take((size_t)p.nseg * Hv * K * V * 4);
     p.segm = take((size_t)p.nseg * Hv * K * K * 4);
   }
   p.total = at;
-  // no segments where their buffers alone would take the problem over the
-  // scratch of gdn_chunk_fwd_noalloc
-  if (p.seg && !bwd && p.total > GDN_NOALLOC_SCRATCH_BYTES) {
-    const WsPlan q = plan_ws(B, T, Hqk, Hv, K, V, N, has_cu, l2, false, false);
-    if (q.total <= GDN_NOALLOC_SCRATCH_BYTES) return q;
-  }
   return p;
 }
 
@@ -855,8 +856,9 @@ extern "C" int gdn_chunk_fwd_noalloc(const void* q, const void* k, const void* v
   if (rc) return rc;
   if (N == 0 || ((long long)B * T == 0 && !ht)) return GDN_OK;  // nothing to compute
   gdn_host::launch_begin();
+  // (without segments, whose buffers would take problems over the scratch)
   const gdn::WsPlan p = gdn::plan_ws(B, T, Hqk, Hv, K, V, N, cu_seqlens != nullptr,
-                                     use_qk_l2norm != 0, false);
+                                     use_qk_l2norm != 0, false, false);
   if (p.total > kNoAllocScratchBytes)
     return gdn_host::fail(GDN_ERR_WORKSPACE,
                           "gdn_chunk_fwd_noalloc: the problem needs " + std::to_string(p.total) +

@@ -23,9 +23,8 @@
 // eight compute waves of 16 columns, staging themselves, took 2.5 us per
 // chunk, and a split into state and output waves 2.8.
 //
-// Staging: as many helper waves hold the next two chunks' K, Q and V units
-// and Tb / P fragments in registers (a load has a whole step to land) and
-// write them to the other of two LDS buffers, K (KLayout) and Q as fp16 --
+// Staging: as many helper waves hold the next three chunks' K, Q and V units
+// and Tb / P fragments in registers (a load has two steps to land) and write them to the other of two LDS buffers, K (KLayout) and Q as fp16 --
 // COPY (use_qk_l2norm): the prep kernel's normalised fp16 copies as they are
 // (normalising here instead made the helper the longer wave: 2.9 us per
 // chunk) -- V as fp16, and the chunk's gate factors.
@@ -35,6 +34,7 @@
 // and transfer matrices M (from I, with V = 0) are formed in parallel (XFER),
 // chunk_combine_kernel runs S_j = M_j S_(j-1) + B_j over them, and the
 // segments' outputs then start from those states, again in parallel.
+#include <algorithm>
 #include <type_traits>
 
 #include "gdn_chunk.h"
@@ -70,32 +70,38 @@ __device__ __forceinline__ void seg_range(int n, int seg, const int32_t* cu, int
 }
 struct SegPos {
   int n;            // sequence, -1 past the last segment
-  int first;        // its chunk the segment starts at
+  int sg;           // global index of the segment
+  int first;        // its sequence's chunk it starts at
   int c_begin, nc;  // global first chunk, chunks
   bool last;        // the sequence's last segment
 };
-// workgroup index -> segment (or, seg == 0, whole sequence)
-__device__ __forceinline__ SegPos seg_pos(int i, int seg, const int32_t* cu, int N, int T,
-                                          const ChunkWs& ws) {
-  SegPos r{i, 0, 0, 0, true};
+// i-th segment -- or (full) the i-th that is not its sequence's last, or
+// (seg == 0) the i-th sequence as a whole
+__device__ __forceinline__ SegPos seg_pos(int i, bool full, int seg, const int32_t* cu, int N,
+                                          int T, const ChunkWs& ws) {
+  SegPos r{i, i, 0, 0, 0, true};
+  const int nct = (T + kChunk - 1) / kChunk;
   int j = 0, cnt = 1;
   if (seg) {
+    // (a sequence has one segment that is not full: full ones are counted by
+    // soff[n] - n)
     if (cu) {
-      if (i >= ws.soff[N]) return SegPos{-1, 0, 0, 0, true};
-      int lo = 0, hi = N;   // the largest n with soff[n] <= i
+      if (i >= ws.soff[N] - (full ? N : 0)) return SegPos{-1, 0, 0, 0, 0, true};
+      int lo = 0, hi = N;   // the largest n whose first segment is i or before
       while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
-        if (ws.soff[mid] <= i) lo = mid; else hi = mid;
+        if (ws.soff[mid] - (full ? mid : 0) <= i) lo = mid; else hi = mid;
       }
       r.n = lo;
     } else {
-      r.n = i / max(1, ((T + kChunk - 1) / kChunk + seg - 1) / seg);
+      const int per = max(1, (nct + seg - 1) / seg) - (full ? 1 : 0);
+      r.n = i / per;
     }
     int first;
     seg_range(r.n, seg, cu, T, ws, first, cnt);
-    j = i - first;
+    r.sg = full ? i + r.n : i;
+    j = r.sg - first;
   }
-  const int nct = (T + kChunk - 1) / kChunk;
   const int c0 = cu ? ws.off[r.n] : r.n * nct;
   const int c1 = cu ? ws.off[r.n + 1] : c0 + nct;
   r.first = j * seg;
@@ -178,16 +184,16 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int r16 = lane % 16, grp = lane / 16;
 
-  // this workgroup's chunks: a sequence's, or one segment of them (sg counts
-  // the segments of all sequences, sj those of this one)
-  const SegPos sp = seg_pos(bid / a.Hv, a.seg, a.cu, a.N, a.T, ws);
+  // this workgroup's chunks: a sequence's, or one segment of them (XFER: one
+  // that another follows)
+  const SegPos sp = seg_pos(bid / a.Hv, XFER, a.seg, a.cu, a.N, a.T, ws);
   if (sp.n < 0) return;
-  const int n = sp.n, sg = bid / a.Hv;
+  const int n = sp.n, sg = sp.sg;
   int s, e;
   seq_bounds(a.cu, n, a.T, a.total, s, e);
   const int c_begin = sp.c_begin, nc = sp.nc;
   s += sp.first * kChunk;
-  if (XFER && (sp.last || (mpart && sp.first == 0))) return;
+  if (mpart && sp.first == 0) return;   // the first segment starts from h0: no M needed
 
   if (w >= NW) {
     // ---------------------------------------------------- helper waves ----
@@ -196,7 +202,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
       u32x4 k[KPT], q[OUT ? KPT : 1], v[VPT], f[SPW];
       float g;
     };
-    Regs ra, rb;
+    Regs r0, r1, r2;
     auto load = [&](Regs& r, int j) {
       const int ci = c_begin + j, t0 = s + j * kChunk, L = min(kChunk, e - t0);
       // K, Q: the prep kernel's fp16 copies (contiguous), or the caller's rows
@@ -279,25 +285,29 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
       }
     };
     if (nc > 0) {
-      load(ra, 0);
-      load(rb, min(1, nc - 1));
-      __builtin_amdgcn_sched_barrier(0);
-      stage(ra, 0, 0);
+      // during step j chunk j+1 is written from its set and chunk j+4
+      // requested into that set, so a load has two to three steps to land
+      // (past the last chunk repeated, into a buffer no step reads)
+      load(r0, 0);
+      load(r1, min(1, nc - 1));
+      load(r2, min(2, nc - 1));
+      stage(r0, 0, 0);
+      load(r0, min(3, nc - 1));
       lds_barrier();
-      // during step j: chunk j+2's loads go out, chunk j+1's are written (past
-      // the last chunk repeated, into a buffer no step reads)
+      auto turn = [&](Regs& r, int j) {
+        stage(r, min(j + 1, nc - 1), (j + 1) & 1);
+        __builtin_amdgcn_sched_barrier(0);
+        load(r, min(j + 4, nc - 1));
+        lds_barrier();
+      };
       int j = 0;
-      for (; j + 1 < nc; j += 2) {
-        load(ra, min(j + 2, nc - 1));
-        __builtin_amdgcn_sched_barrier(0);
-        stage(rb, j + 1, 1);
-        lds_barrier();
-        load(rb, min(j + 3, nc - 1));
-        __builtin_amdgcn_sched_barrier(0);
-        stage(ra, min(j + 2, nc - 1), 0);
-        lds_barrier();
+      for (; j + 2 < nc; j += 3) {
+        turn(r1, j);
+        turn(r2, j + 1);
+        turn(r0, j + 2);
       }
-      if (j < nc) lds_barrier();
+      if (j < nc) turn(r1, j);
+      if (j + 1 < nc) turn(r2, j + 1);
     }
     return;
   }
@@ -648,6 +658,8 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
                                                ((2 * ct + 1) * 64 + lane) * 16, 0, kStoreStream);
       }
     }
+  };
+  auto next = [&](int j) {
     lds_barrier();
     // the next step's buffer
     const int d = (j & 1) ? -kBufStep : kBufStep;
@@ -669,7 +681,10 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
 
   if (nc > 0) {
     lds_barrier();
-    for (int j = 0; j < nc; ++j) step(j);
+    for (int j = 0; j < nc; ++j) {
+      step(j);
+      next(j);
+    }
     if constexpr (OUT) {
       out_mfma(0, 4);
 #pragma unroll
@@ -726,74 +741,91 @@ template <int K>
 __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkWs ws) {
   constexpr int ST = K / 16, KB = K / 32;   // row tiles (waves), k-blocks
   __shared__ __attribute__((aligned(16))) u16x4 St[2][2][ST][64];   // [parity][hi, lo]
-  // (column tiles of one head a multiple of 8 workgroups apart where N Hv is
-  // one: on one XCD, whose L2 then serves the M they share)
-  const int heads = a.N * a.Hv, vt = blockIdx.x / heads;
-  const int h = blockIdx.x % heads % a.Hv, n = blockIdx.x % heads / a.Hv;
+  const int h = blockIdx.x % a.Hv, vt = blockIdx.x / a.Hv;
   const int lane = threadIdx.x % 64;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int r16 = lane % 16, grp = lane / 16;
-  int first, count;   // this sequence's segments
-  seg_range(n, a.seg, a.cu, a.T, ws, first, count);
-  if (count < 3) return;   // nothing after the first segment that another starts from
-  auto head = [&](int j) { return (size_t)(first + j) * a.Hv + h; };
-  auto load_m = [&](u16x8 (&m)[2][KB], int j) {
-    const u16x8* p = ws.segm + head(j) * (2 * ST * KB * 64) + w * KB * 64 + lane;
-#pragma unroll
-    for (int b = 0; b < KB; ++b) {
-      m[0][b] = p[b * 64];
-      m[1][b] = p[(ST * KB + b) * 64];
-    }
-  };
-  // this wave's state tile: lane (r16, grp), element r = row rho(16 w + 4 grp
-  // + r), column 16 vt + r16
-  auto tile_at = [&](int j) {
-    return ws.segs + head(j) * K * K + (size_t)rho_row(w, 4 * grp) * K + 16 * vt + r16;
-  };
-  auto load_b = [&](int j) {
-    const float* p = tile_at(j);
-    return f32x4{p[0], p[K], p[2 * K], p[3 * K]};
-  };
-  auto publish = [&](f32x4 x, int par) {
-    u16x4 hi, lo;
-    split_bf4(x, hi, lo);
-    St[par][0][w][lane] = hi;
-    St[par][1][w][lane] = lo;
+  // The sequences with three segments or more (with fewer nothing but the first
+  // segment is started from), every gridDim.y-th of them here: found NT at a
+  // time, a bit per thread.
+  constexpr int NT = 4 * K;
+  __shared__ unsigned long long many[NT / 64];
+  int seen = 0;
+  for (int base = 0; base < a.N; base += NT) {
+    int first = 0, count = 0;   // a sequence's segments
+    if (base + (int)threadIdx.x < a.N)
+      seg_range(base + threadIdx.x, a.seg, a.cu, a.T, ws, first, count);
+    const unsigned long long mine = __ballot(count >= 3);
+    if (lane == 0) many[w] = mine;
     lds_barrier();
-  };
-  // segment j's M fragments and B tile in set j % 3
-  u16x8 m[3][2][KB];
-  f32x4 bt[3];
-  load_m(m[1], 1);
-  bt[1] = load_b(1);
-  load_m(m[2], min(2, count - 2));
-  bt[2] = load_b(min(2, count - 2));
-  publish(load_b(0), 0);
-  auto step = [&](int j, auto jc) {
-    constexpr int c = decltype(jc)::value;   // j % 3
-    const int jn = min(j + 2, count - 2);
-    load_m(m[(c + 2) % 3], jn);
-    bt[(c + 2) % 3] = load_b(jn);
-    f32x4 acc = bt[c], acc1 = zero4(), acc2 = zero4();
+    for (int word = 0; word < NT / 64; ++word) {
+      for (unsigned long long left = many[word]; left; left &= left - 1) {
+        if (seen++ % (int)gridDim.y != (int)blockIdx.y) continue;
+        const int n = __builtin_amdgcn_readfirstlane(base + 64 * word + __builtin_ctzll(left));
+        seg_range(n, a.seg, a.cu, a.T, ws, first, count);
+        auto head = [&](int j) { return (size_t)(first + j) * a.Hv + h; };
+        auto load_m = [&](u16x8 (&m)[2][KB], int j) {
+          const u16x8* p = ws.segm + head(j) * (2 * ST * KB * 64) + w * KB * 64 + lane;
 #pragma unroll
-    for (int b = 0; b < KB; ++b) {
-      const auto& sp = St[(j + 1) & 1];
-      const u16x8 hi = cat8(sp[0][2 * b][lane], sp[0][2 * b + 1][lane]);
-      const u16x8 lo = cat8(sp[1][2 * b][lane], sp[1][2 * b + 1][lane]);
-      acc = mfma16(m[c][0][b], hi, acc);
-      acc1 = mfma16(m[c][0][b], lo, acc1);
-      acc2 = mfma16(m[c][1][b], hi, acc2);
+          for (int b = 0; b < KB; ++b) {
+            m[0][b] = p[b * 64];
+            m[1][b] = p[(ST * KB + b) * 64];
+          }
+        };
+        // this wave's state tile: lane (r16, grp), element r = row rho(16 w + 4 grp
+        // + r), column 16 vt + r16
+        auto tile_at = [&](int j) {
+          return ws.segs + head(j) * K * K + (size_t)rho_row(w, 4 * grp) * K + 16 * vt + r16;
+        };
+        auto load_b = [&](int j) {
+          const float* p = tile_at(j);
+          return f32x4{p[0], p[K], p[2 * K], p[3 * K]};
+        };
+        auto publish = [&](f32x4 x, int par) {
+          u16x4 hi, lo;
+          split_bf4(x, hi, lo);
+          St[par][0][w][lane] = hi;
+          St[par][1][w][lane] = lo;
+          lds_barrier();
+        };
+        // segment j's M fragments and B tile in set j % 3
+        u16x8 m[3][2][KB];
+        f32x4 bt[3];
+        load_m(m[1], 1);
+        bt[1] = load_b(1);
+        load_m(m[2], min(2, count - 2));
+        bt[2] = load_b(min(2, count - 2));
+        publish(load_b(0), 0);
+        auto step = [&](int j, auto jc) {
+          constexpr int c = decltype(jc)::value;   // j % 3
+          const int jn = min(j + 2, count - 2);
+          load_m(m[(c + 2) % 3], jn);
+          bt[(c + 2) % 3] = load_b(jn);
+          f32x4 acc = bt[c], acc1 = zero4(), acc2 = zero4();
+#pragma unroll
+          for (int b = 0; b < KB; ++b) {
+            const auto& sp = St[(j + 1) & 1];
+            const u16x8 hi = cat8(sp[0][2 * b][lane], sp[0][2 * b + 1][lane]);
+            const u16x8 lo = cat8(sp[1][2 * b][lane], sp[1][2 * b + 1][lane]);
+            acc = mfma16(m[c][0][b], hi, acc);
+            acc1 = mfma16(m[c][0][b], lo, acc1);
+            acc2 = mfma16(m[c][1][b], hi, acc2);
+          }
+          acc = acc + (acc1 + acc2);
+          float* o = tile_at(j);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[(size_t)r * K] = acc[r];
+          publish(acc, j & 1);
+        };
+        for (int j = 1; j < count - 1;) {
+          step(j++, std::integral_constant<int, 1>{});
+          if (j < count - 1) step(j++, std::integral_constant<int, 2>{});
+          if (j < count - 1) step(j++, std::integral_constant<int, 0>{});
+        }
+        lds_barrier();   // St is free for the next sequence
+      }
     }
-    acc = acc + (acc1 + acc2);
-    float* o = tile_at(j);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[(size_t)r * K] = acc[r];
-    publish(acc, j & 1);
-  };
-  for (int j = 1; j < count - 1;) {
-    step(j++, std::integral_constant<int, 1>{});
-    if (j < count - 1) step(j++, std::integral_constant<int, 2>{});
-    if (j < count - 1) step(j++, std::integral_constant<int, 0>{});
+    lds_barrier();   // as is `many`
   }
 }
 
@@ -807,13 +839,15 @@ void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, 
   auto go = [&](auto kern, unsigned g) {
     hipLaunchKernelGGL(kern, dim3(g), dim3(4 * V), 0, st, a, ws);
   };
-  if (p.seg) {
-    if (V == K) {   // (segments are planned for K == V only)
-      if (l2) go(chunk_head_kernel<K, K, true, false, false, true>, 2 * grid);
-      else go(chunk_head_kernel<K, K, false, false, false, true>, 2 * grid);
-      hipLaunchKernelGGL((chunk_combine_kernel<K>), dim3((unsigned)(N * Hv * (V / 16))),
-                         dim3(4 * K), 0, st, a, ws);
-    }
+  if (p.seg && p.nfull > 0 && V == K) {   // (segments are planned for K == V only)
+    const unsigned full = (unsigned)(p.nfull * Hv);
+    if (l2) go(chunk_head_kernel<K, K, true, false, false, true>, 2 * full);
+    else go(chunk_head_kernel<K, K, false, false, false, true>, 2 * full);
+    // a workgroup per (v-head, column tile) and, as far as the GPU holds them,
+    // sequence; with many sequences the rest in turn (most have no segments)
+    const unsigned tiles = (unsigned)(Hv * (V / 16));
+    const unsigned seqs = std::min<unsigned>(N, std::max(1u, 4u * device_cus() / tiles));
+    hipLaunchKernelGGL((chunk_combine_kernel<K>), dim3(tiles, seqs), dim3(4 * K), 0, st, a, ws);
   }
   if (V == 128) {
     if (l2) go(chunk_head_kernel<K, 128, true, SAVE, OUT, false>, grid);

@@ -73,9 +73,12 @@ extern "C" {
  * q / k (or use_qk_l2norm) and the v of a Qwen3-Next layer are orders of
  * magnitude inside it.  The final state is within ~4e-4 relative Frobenius
  * of the exact recurrence at any length.  Without use_qk_l2norm the output's
- * q.S term is a bf16 MFMA product (q as given, the state rounded to bf16);
- * with it an fp16 one (the normalised q as fp16); gdn_chunk_fwd_save gives
- * the same o as gdn_chunk_fwd either way.
+ * q.S term is, for few short chains, a bf16 MFMA product (q as given, the
+ * state rounded to bf16); with it, and for many or long chains, an fp16 one
+ * (q as fp16); gdn_chunk_fwd_save gives the same o as gdn_chunk_fwd either
+ * way.  Few long sequences (64 chunks and more) are run in segments, whose
+ * buffers (128 KiB per segment and v-head at K = V = 128) are part of the
+ * workspace.
  */
 int gdn_chunk_fwd(const void* q, const void* k, const void* v,
                   const float* g, const float* beta,
@@ -104,7 +107,9 @@ size_t gdn_chunk_workspace_bytes(int B, int T, int Hqk, int Hv, int K, int V,
  * The array is part of libgdn.so's device code object: every process that
  * loads the library holds those 32 MiB on every GPU it uses, until it ends,
  * whether or not it calls this entry point.
- * Problems whose gdn_chunk_workspace_bytes(...) exceeds 32 MiB (about 5,300
+ * It never runs in segments (whose buffers would not fit), so that where
+ * gdn_chunk_fwd does, the two agree to rounding, else bit for bit.
+ * Problems whose workspace without segments exceeds 32 MiB (about 5,300
  * tokens at 32 v-heads / 16 qk-heads, K = V = 128; about 2,300 with
  * use_qk_l2norm, whose chain reads fp16 copies of the normalised q, k rows
  * from the workspace) are rejected with

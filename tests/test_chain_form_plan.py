@@ -1,5 +1,5 @@
-"""Workspace of the segmented chain form (CPU): segments never take a problem that fits the
-scratch of gdn_chunk_fwd_noalloc over it, and the backward's workspace covers them."""
+"""Workspace of the segmented chain form (CPU): what gdn_chunk_fwd_noalloc refuses is still
+decided by the buffers without segments, and the backward's workspace covers the forward's."""
 import pytest
 
 from avelang_amd import _native
@@ -19,15 +19,18 @@ def _plain(T, Hqk, Hv, K, l2):
 @pytest.mark.parametrize("K", [64, 128])
 @pytest.mark.parametrize("l2", [0, 1])
 @pytest.mark.parametrize("Hqk,Hv", [(1, 2), (2, 4), (4, 8), (16, 16), (16, 32)])
-def test_noalloc_limit_is_kept(Hqk, Hv, K, l2):
+def test_workspace_with_segments(Hqk, Hv, K, l2):
     lib = _native.lib()
+    fake = [i << 40 for i in range(1, 6)] + [None, None, 6 << 40, None]
     grown = 0
-    for chunks in list(range(1, 200, 7)) + [256, 300, 500, 700, 1000, 2000]:
+    for chunks in list(range(1, 200, 7)) + [256, 300, 500, 700, 1000, 2000, 6000]:
         T = 64 * chunks - 3
         plain = _plain(T, Hqk, Hv, K, l2)
         got = lib.gdn_chunk_workspace_bytes(1, T, Hqk, Hv, K, K, 1, 0, l2)
         assert got >= plain
-        assert (got <= LIMIT) == (plain <= LIMIT), (T, plain, got)
         grown += got > plain
         assert lib.gdn_chunk_bwd_workspace_bytes(1, T, Hqk, Hv, K, K, 1, 0, l2) > got
+        if plain > LIMIT:   # (refused before any launch; what is accepted would launch)
+            assert lib.gdn_chunk_fwd_noalloc(*fake, 1, T, Hqk, Hv, K, K, 1, 0.1, l2, None) == -4
+            assert str(plain) in lib.gdn_last_error().decode()
     assert grown > 0   # some of them do run in segments

@@ -158,3 +158,23 @@ def test_gradients(rocm_device):
             x = x.double().cpu().numpy()
             rel = np.linalg.norm(x - ref[name]) / np.linalg.norm(ref[name])
             assert rel <= (1e-3 if name == "dh0" else 1e-2), f"{what}: {name} {rel:.2e}"
+
+
+def test_noalloc_takes_what_fits_without_segments(rocm_device):
+    """A problem that gdn_chunk_fwd runs in segments, its workspace with them over the library's
+    scratch, without them under it: still accepted, and the same up to rounding."""
+    from avelang_amd import _native
+    lib = _native.lib()
+    wl = W.make(1, 8192, 16, 16, 128, 128, seed=12, h0_scale=0.01)
+    assert lib.gdn_chunk_workspace_bytes(1, 8192, 16, 16, 128, 128, 1, 0, 0) > (32 << 20)
+    o, s = _run(wl, rocm_device)
+    t = wl.torch(rocm_device)
+    o2, s2 = torch.full_like(o, 5.0), torch.full_like(s, 5.0)
+    rc = lib.gdn_chunk_fwd_noalloc(
+        *(t[n].data_ptr() for n in ("q", "k", "v", "g", "beta", "initial_state")), s2.data_ptr(),
+        o2.data_ptr(), None, 1, 8192, 16, 16, 128, 128, 1, 128 ** -0.5, 0,
+        torch.cuda.current_stream(rocm_device).cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0, lib.gdn_last_error().decode()
+    assert (s2 - s).norm() <= 1e-3 * s.norm()
+    assert (o2.float() - o.float()).norm() <= 1e-2 * o.float().norm()
