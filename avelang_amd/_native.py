@@ -41,6 +41,9 @@ EXPORTS = (
     "gdn_recurrent_fwd_spec",
 )
 
+# Declared in include/gdn_rows.h.
+EXPORTS_ROWS = ("gdn_chunk_fwd_rows", "gdn_recurrent_fwd_rows")
+
 GDN_DTYPE_F32 = 0
 GDN_DTYPE_BF16 = 1
 GDN_DTYPE_F16 = 2
@@ -168,6 +171,13 @@ def lib():
             + [_i, _vp]                       # index_stride num_accepted_tokens
             + [_i] * 8                        # B T Hqk Hv K V N num_slots
             + [_f, _i, _vp])
+        # q k v, their token strides, g beta, then the gating's
+        _rows = [_vp] * 3 + [_ll] * 3 + [_vp] * 2 + _gate
+        h.gdn_chunk_fwd_rows.restype = _i
+        h.gdn_chunk_fwd_rows.argtypes = (_rows + [_vp] * 4 + [_i] * 7
+                                         + [_f, _i, _vp, _sz, _vp])
+        h.gdn_recurrent_fwd_rows.restype = _i
+        h.gdn_recurrent_fwd_rows.argtypes = _rows + [_vp] * 5 + [_i] * 8 + [_f, _i, _vp]
         _lib = h
         return _lib
 

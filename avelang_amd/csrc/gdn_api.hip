@@ -98,6 +98,30 @@ int validate_gate_size(const char* name, long long elements) {
   return GDN_OK;
 }
 
+// Token strides (elements) of q, k, v as column slices: rows of at least the
+// heads' width, 16-byte aligned (the kernels move 16 bytes per lane), within
+// the 32-bit offsets of a chunk's buffer loads; o apart from all of them.
+int validate_rows(const char* name, const void* q, const void* k, const void* v, long long q_row,
+                  long long k_row, long long v_row, const void* o, long long tokens, int Hqk,
+                  int Hv, int K, int V, gdn::TokenStride& ts) {
+  const void* p[3] = {q, k, v};
+  const long long row[3] = {q_row, k_row, v_row};
+  const long long width[3] = {(long long)Hqk * K, (long long)Hqk * K, (long long)Hv * V};
+  for (int i = 0; i < 3; ++i) {
+    if (row[i] < width[i] || row[i] % 8 || row[i] >= (1LL << 23) ||
+        reinterpret_cast<uintptr_t>(p[i]) % 16)
+      return fail(GDN_ERR_SHAPE, std::string(name) + ": q, k and v rows must be 16-byte aligned, at "
+                                                     "least as long as their heads and under 2^23 "
+                                                     "elements");
+    if (o && tokens > 0 &&
+        overlaps(o, (size_t)(tokens * Hv * V * 2), p[i],
+                 (size_t)(((tokens - 1) * row[i] + width[i]) * 2)))
+      return fail(GDN_ERR_ALIAS, std::string(name) + ": o must not overlap q, k or v");
+  }
+  ts = gdn::TokenStride{(int)q_row, (int)k_row, (int)v_row};
+  return GDN_OK;
+}
+
 }  // namespace gdn_host
 
 extern "C" const char* gdn_last_error(void) { return gdn_host::g_last_error.c_str(); }

@@ -220,7 +220,8 @@ void launch_chunk_fwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, c
                       const float* beta, const float* h0, float* ht, uint16_t* o,
                       const int32_t* cu, int B, int T, int Hqk, int Hv, int K, int V, int N,
                       float scale, bool l2, FwdMode mode, const WsPlan& p, unsigned char* wsb,
-                      hipStream_t st, const GateIn& gate = GateIn{});
+                      hipStream_t st, const GateIn& gate = GateIn{},
+                      const TokenStride* rows = nullptr);
 
 ChunkWs ws_pointers(const WsPlan& p, unsigned char* wsb);
 
@@ -231,8 +232,8 @@ ChunkWs ws_pointers(const WsPlan& p, unsigned char* wsb);
 template <int K, bool SAVE, bool OUT>
 void launch_chain_sw(const uint16_t* v, const uint16_t* qraw, const uint16_t* kraw,
                      const float* h0, float* ht, uint16_t* o, const int32_t* cu, int N, int T,
-                     int total, int Hqk, int Hv, int V, float scale, const ChunkWs& ws,
-                     hipStream_t st);
+                     int total, int Hqk, int Hv, int V, float scale, TokenStride ts,
+                     const ChunkWs& ws, hipStream_t st);
 
 // Forward chain, whole-head form (gdn_chunk_head.hip), in segments where the
 // plan has them: the same results and buffers, K and Q from the caller's rows
@@ -240,8 +241,8 @@ void launch_chain_sw(const uint16_t* v, const uint16_t* qraw, const uint16_t* kr
 template <int K, bool SAVE, bool OUT>
 void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, const float* h0,
                        float* ht, uint16_t* o, const int32_t* cu, int N, int T, int total, int Hqk,
-                       int Hv, int V, float scale, bool l2, const WsPlan& p, const ChunkWs& ws,
-                       hipStream_t st);
+                       int Hv, int V, float scale, bool l2, TokenStride ts, const WsPlan& p,
+                       const ChunkWs& ws, hipStream_t st);
 
 // Reverse chain of the backward (gdn_chunk_rev.hip): dS' of every chunk into
 // dse, dd into dd, dh0 (K rows from ws.k16).

@@ -42,6 +42,7 @@
 #include <type_traits>
 
 #include "gdn_chunk.h"
+#include "../../include/gdn_rows.h"
 
 namespace gdn {
 
@@ -183,7 +184,7 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const float* __restrict__ g, const float* __restrict__ beta,
     const int32_t* __restrict__ cu, int N, int T, int total, int Hqk, int Hv, float scale,
-    ChunkWs ws, GateIn gate) {
+    ChunkWs ws, GateIn gate, TokenStride ts) {
   constexpr int KB = K / 32;
   // strictly lower 16 x 16 blocks of A only (block (bi, m), m < bi, at
   // bi (bi - 1) / 2 + m; row stride 20 keeps float4 rows aligned and the 16
@@ -253,11 +254,12 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(
   // be finite, and the loads stay branch-free.
   u16x8 ka[KB], qa[KB];
   {
-    const size_t ro = ((size_t)(t0 + min(16 * w + r16, L - 1)) * Hqk + hq) * K + 8 * grp;
+    const size_t row = t0 + min(16 * w + r16, L - 1), col = hq * K + 8 * grp;
+    const uint16_t *kr = k + row * ts.k + col, *qr = q + row * ts.q + col;
 #pragma unroll
     for (int b = 0; b < KB; ++b) {
-      ka[b] = *reinterpret_cast<const u16x8*>(k + ro + 32 * b);
-      qa[b] = *reinterpret_cast<const u16x8*>(q + ro + 32 * b);
+      ka[b] = *reinterpret_cast<const u16x8*>(kr + 32 * b);
+      qa[b] = *reinterpret_cast<const u16x8*>(qr + 32 * b);
     }
     if constexpr (L2) {
       // use_qk_l2norm: a row's K values sit in the 4 lanes r16 + 16 grp; the
@@ -667,7 +669,7 @@ static void launch_chunk(const uint16_t* q, const uint16_t* k, const uint16_t* v
                          const float* g, const float* beta, const float* h0, float* ht,
                          uint16_t* o, const int32_t* cu, int B, int T, int Hqk, int Hv, int V,
                          int N, float scale, bool l2, const WsPlan& p, unsigned char* wsb,
-                         hipStream_t st, const GateIn& gate) {
+                         hipStream_t st, const GateIn& gate, TokenStride ts) {
   const ChunkWs ws = ws_pointers(p, wsb);
   const int total = B * T;
   if (cu)
@@ -676,20 +678,20 @@ static void launch_chunk(const uint16_t* q, const uint16_t* k, const uint16_t* v
   if (p.ncmax > 0) {
     if (l2)
       hipLaunchKernelGGL((chunk_prep_kernel<K, BWD, OUT, true>), dim3((unsigned)p.ncmax, Hv), dim3(256),
-                         0, st, q, k, g, beta, cu, N, T, total, Hqk, Hv, scale, ws, gate);
+                         0, st, q, k, g, beta, cu, N, T, total, Hqk, Hv, scale, ws, gate, ts);
     else
       hipLaunchKernelGGL((chunk_prep_kernel<K, BWD, OUT, false>), dim3((unsigned)p.ncmax, Hv), dim3(256),
-                         0, st, q, k, g, beta, cu, N, T, total, Hqk, Hv, scale, ws, gate);
+                         0, st, q, k, g, beta, cu, N, T, total, Hqk, Hv, scale, ws, gate, ts);
   }
   // the chain reads K and Q as the prep kernel's fp16 copies where the plan
   // has them (normalised with use_qk_l2norm), else as the caller's bf16 rows
   if (p.whole_head)
     launch_chain_head<K, BWD, OUT>(q, k, v, h0, OUT ? ht : nullptr, OUT ? o : nullptr, cu, N, T,
-                                   total, Hqk, Hv, V, scale, l2, p, ws, st);
+                                   total, Hqk, Hv, V, scale, l2, ts, p, ws, st);
   else
     launch_chain_sw<K, BWD, OUT>(v, ws.q16 ? nullptr : q, ws.k16 ? nullptr : k, h0,
                                OUT ? ht : nullptr, OUT ? o : nullptr, cu, N, T, total, Hqk, Hv,
-                               V, scale, ws, st);
+                               V, scale, ts, ws, st);
   // a cu_seqlens violation left every sequence empty: o is zero-filled (and
   // ht = h0, written by the chain for an empty sequence)
   if (cu && OUT) {
@@ -704,10 +706,11 @@ void launch_chunk_fwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, c
                       const float* beta, const float* h0, float* ht, uint16_t* o,
                       const int32_t* cu, int B, int T, int Hqk, int Hv, int K, int V, int N,
                       float scale, bool l2, FwdMode mode, const WsPlan& p, unsigned char* wsb,
-                      hipStream_t st, const GateIn& gate) {
+                      hipStream_t st, const GateIn& gate, const TokenStride* rows) {
+  const TokenStride ts = rows ? *rows : TokenStride{Hqk * K, Hqk * K, Hv * V};
 #define GDN_FWD(KK_, BWD_, OUT_)                                                             \
   launch_chunk<KK_, BWD_, OUT_>(q, k, v, g, beta, h0, ht, o, cu, B, T, Hqk, Hv, V, N, scale, l2, \
-                                p, wsb, st, gate)
+                                p, wsb, st, gate, ts)
   if (K == 128) {
     if (mode == FwdMode::kForward) GDN_FWD(128, false, true);
     else if (mode == FwdMode::kRecompute) GDN_FWD(128, true, false);
@@ -726,6 +729,9 @@ namespace gdn_host {
 int validate_gate(const char* name, const void* A_log, const void* dt_bias, int a_dtype,
                   int b_dtype, int p_dtype, float sp_beta, long long tokens);
 int validate_gate_size(const char* name, long long elements);
+int validate_rows(const char* name, const void* q, const void* k, const void* v, long long q_row,
+                  long long k_row, long long v_row, const void* o, long long tokens, int Hqk,
+                  int Hv, int K, int V, gdn::TokenStride& ts);
 int validate_common(const void* q, const void* k, const void* v, const float* g,
                     const float* beta, const float* h0, const float* ht, const void* o,
                     const int32_t* cu, int B, int T, int Hqk, int Hv, int K, int V, int N);
@@ -743,7 +749,8 @@ int chunk_fwd_impl(const void* q, const void* k, const void* v, const float* g,
                    const float* beta, const float* h0, float* ht, void* o,
                    const int32_t* cu_seqlens, int B, int T, int Hqk, int Hv, int K, int V, int N,
                    float scale, int use_qk_l2norm, void* workspace, size_t workspace_bytes,
-                   const gdn::GateIn& gate, void* stream, const char* name) {
+                   const gdn::GateIn& gate, void* stream, const char* name,
+                   const gdn::TokenStride* rows = nullptr) {
   if (N == 0 || ((long long)B * T == 0 && !ht)) return GDN_OK;  // nothing to compute
   gdn_host::launch_begin();
   const gdn::WsPlan p = gdn::plan_ws(B, T, Hqk, Hv, K, V, N, cu_seqlens != nullptr,
@@ -759,7 +766,7 @@ int chunk_fwd_impl(const void* q, const void* k, const void* v, const float* g,
                         static_cast<uint16_t*>(o), cu_seqlens, B, T, Hqk, Hv, K, V, N, scale,
                         use_qk_l2norm != 0, gdn::FwdMode::kForward, p,
                         static_cast<unsigned char*>(workspace), static_cast<hipStream_t>(stream),
-                        gate);
+                        gate, rows);
   return gdn_host::check_launch(name);
 }
 }  // namespace
@@ -801,6 +808,41 @@ extern "C" int gdn_chunk_fwd_gating(const void* q, const void* k, const void* v,
                          (long long)B * T * Hv, Hv};
   return chunk_fwd_impl(q, k, v, nullptr, nullptr, h0, ht, o, cu_seqlens, B, T, Hqk, Hv, K, V, N,
                         scale, use_qk_l2norm, workspace, workspace_bytes, gate, stream, name);
+}
+
+// Prefill on column slices of wider tensors (declared in gdn_rows.h).
+extern "C" int gdn_chunk_fwd_rows(const void* q, const void* k, const void* v, long long q_row,
+                                  long long k_row, long long v_row, const float* g,
+                                  const float* beta, const void* A_log, const void* a,
+                                  const void* b, const void* dt_bias, int a_dtype, int b_dtype,
+                                  int p_dtype, float sp_beta, float sp_threshold, const float* h0,
+                                  float* ht, void* o, const int32_t* cu_seqlens, int B, int T,
+                                  int Hqk, int Hv, int K, int V, int N, float scale,
+                                  int use_qk_l2norm, void* workspace, size_t workspace_bytes,
+                                  void* stream) {
+  const char* name = "gdn_chunk_fwd_rows";
+  const float* gg = A_log ? static_cast<const float*>(a) : g;
+  const float* bb = A_log ? static_cast<const float*>(b) : beta;
+  int rc = gdn_host::validate_common(q, k, v, gg, bb, h0, ht, o, cu_seqlens, B, T, Hqk, Hv, K, V,
+                                     N);
+  if (rc) return rc;
+  gdn::TokenStride ts;
+  rc = gdn_host::validate_rows(name, q, k, v, q_row, k_row, v_row, o, (long long)B * T, Hqk, Hv, K,
+                               V, ts);
+  if (rc) return rc;
+  gdn::GateIn gate{};
+  if (A_log) {
+    rc = gdn_host::validate_gate(name, A_log, dt_bias, a_dtype, b_dtype, p_dtype, sp_beta,
+                                 (long long)B * T);
+    if (rc) return rc;
+    rc = gdn_host::validate_gate_size(name, (long long)B * T * Hv);
+    if (rc) return rc;
+    gate = gdn::GateIn{A_log, a, b, dt_bias, a_dtype, b_dtype, p_dtype, sp_beta, sp_threshold,
+                       (long long)B * T * Hv, Hv};
+  }
+  return chunk_fwd_impl(q, k, v, A_log ? nullptr : g, A_log ? nullptr : beta, h0, ht, o,
+                        cu_seqlens, B, T, Hqk, Hv, K, V, N, scale, use_qk_l2norm, workspace,
+                        workspace_bytes, gate, stream, name, &ts);
 }
 
 // ----------------------------------------------- allocation-free form ----

@@ -83,7 +83,7 @@ __global__ __launch_bounds__((chain_waves<SAVE, OUT, NS, RAWK>() * 64)) void
 chunk_chain_sw_kernel(const uint16_t* __restrict__ v, const uint16_t* __restrict__ qraw,
                       const uint16_t* __restrict__ kraw, const float* h0, float* ht,
                       uint16_t* __restrict__ o, const int32_t* __restrict__ cu, int N, int T,
-                      int total, int Hqk, int Hv, int V, float scale, ChunkWs ws) {
+                      int total, int Hqk, int Hv, int V, float scale, TokenStride ts, ChunkWs ws) {
   static_assert(!RAWK || (OUT && !SAVE && NS == 1 && RAWQ), "RAWK is a plain forward");
   static_assert(!RAWQ || OUT, "RAWQ forms o");
   static_assert(!OUT || chain_split_out<SAVE, OUT, NS>(), "every form with o splits its output");
@@ -321,14 +321,14 @@ chunk_chain_sw_kernel(const uint16_t* __restrict__ v, const uint16_t* __restrict
       // 32 x + l / 2 (rows past the sequence end read as 0)
       const int t0 = s + j * kChunk, L = min(kChunk, e - t0);
       const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<uint16_t*>(v + (size_t)t0 * Hv * V), 0, L * Hv * V * 2, kBufferFlags);
+          const_cast<uint16_t*>(v + (size_t)t0 * ts.v), 0, L * ts.v * 2, kBufferFlags);
 #pragma unroll
       for (int sl = 0; sl < NS; ++sl) {
 #pragma unroll
         for (int x = 0; x < 2; ++x)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
               rv, (lds_ptr)&Vrw[buf][sl][32 * x][0], 16,
-              ((32 * x + (lane >> 1)) * Hv * V + h * V + 16 * (vt0 + sl)) * 2 + 16 * (lane & 1),
+              ((32 * x + (lane >> 1)) * ts.v + h * V + 16 * (vt0 + sl)) * 2 + 16 * (lane & 1),
               0, 0, 0);
       }
     };
@@ -362,12 +362,12 @@ chunk_chain_sw_kernel(const uint16_t* __restrict__ v, const uint16_t* __restrict
     auto load = [&](u32x4v (&x)[KL::LOADS], int c) {
       const int t0 = s + c * kChunk, L = min(kChunk, e - t0);
       const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<uint16_t*>(kraw + ((size_t)t0 * Hqk + hq) * K), 0, L * Hqk * K * 2,
+          const_cast<uint16_t*>(kraw + (size_t)t0 * ts.k + hq * K), 0, L * ts.k * 2,
           kBufferFlags);
 #pragma unroll
       for (int i = 0; i < KL::LOADS; ++i)
         x[i] = __builtin_amdgcn_raw_buffer_load_b128(
-            rk, (RPL * i + lane / UPR) * Hqk * K * 2 + 16 * (lane % UPR), 0, 0);
+            rk, (RPL * i + lane / UPR) * ts.k * 2 + 16 * (lane % UPR), 0, 0);
     };
     auto convert = [&](const u32x4v (&x)[KL::LOADS], int c) {
       const int t0 = s + c * kChunk, L = min(kChunk, e - t0);
@@ -506,7 +506,7 @@ chunk_chain_sw_kernel(const uint16_t* __restrict__ v, const uint16_t* __restrict
           if constexpr (RAWQ) {
             const int t0 = s + j * kChunk, L = min(kChunk, e - t0);
             const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<uint16_t*>(qraw + ((size_t)t0 * Hqk + hq) * K), 0, L * Hqk * K * 2,
+                const_cast<uint16_t*>(qraw + (size_t)t0 * ts.q + hq * K), 0, L * ts.q * 2,
                 kBufferFlags);
 #pragma unroll
             for (int x = 0; x < 2; ++x) {
@@ -515,7 +515,7 @@ chunk_chain_sw_kernel(const uint16_t* __restrict__ v, const uint16_t* __restrict
               for (int b = 0; b < KB; ++b)
                 r.qf[x][b] = __builtin_bit_cast(
                     u16x8, __builtin_amdgcn_raw_buffer_load_b128(
-                               rq, ((16 * ti + r16) * Hqk * K + 32 * b + 8 * grp) * 2, 0, 0));
+                               rq, ((16 * ti + r16) * ts.q + 32 * b + 8 * grp) * 2, 0, 0));
             }
           } else {
             const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
@@ -727,8 +727,8 @@ chunk_chain_sw_kernel(const uint16_t* __restrict__ v, const uint16_t* __restrict
 template <int K, bool SAVE, bool OUT>
 void launch_chain_sw(const uint16_t* v, const uint16_t* qraw, const uint16_t* kraw,
                      const float* h0, float* ht, uint16_t* o, const int32_t* cu, int N, int T,
-                     int total, int Hqk, int Hv, int V, float scale, const ChunkWs& ws,
-                     hipStream_t st) {
+                     int total, int Hqk, int Hv, int V, float scale, TokenStride ts,
+                     const ChunkWs& ws, hipStream_t st) {
   // two V tiles per workgroup once the chains fill the GPU twice over: the
   // tiles share the stage and output waves' operand traffic, and every chain
   // still has a state wave of its own (not with both outputs, where a save
@@ -740,7 +740,7 @@ void launch_chain_sw(const uint16_t* v, const uint16_t* qraw, const uint16_t* kr
   const dim3 grid((unsigned)(two ? chains / 2 : chains));
   auto go = [&](auto kern, int waves) {
     hipLaunchKernelGGL(kern, grid, dim3(waves * 64), 0, st, v, qraw, kraw, h0, ht, o, cu, N, T,
-                       total, Hqk, Hv, V, scale, ws);
+                       total, Hqk, Hv, V, scale, ts, ws);
   };
   if constexpr (OUT) {
     if constexpr (!SAVE) {
@@ -765,7 +765,8 @@ void launch_chain_sw(const uint16_t* v, const uint16_t* qraw, const uint16_t* kr
 #define GDN_CHAIN_INST(K_, SAVE_, OUT_)                                                     \
   template void launch_chain_sw<K_, SAVE_, OUT_>(                                           \
       const uint16_t*, const uint16_t*, const uint16_t*, const float*, float*, uint16_t*,   \
-      const int32_t*, int, int, int, int, int, int, float, const ChunkWs&, hipStream_t);
+      const int32_t*, int, int, int, int, int, int, float, TokenStride, const ChunkWs&,       \
+      hipStream_t);
 GDN_CHAIN_INST(64, false, true)
 GDN_CHAIN_INST(64, true, false)
 GDN_CHAIN_INST(64, true, true)

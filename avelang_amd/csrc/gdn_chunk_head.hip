@@ -52,6 +52,7 @@ struct HeadArgs {
   int N, T, total, Hqk, Hv;
   float scale;
   int seg;      // chunks per segment (0: whole sequences)
+  TokenStride ts;
 };
 
 // Segments.  Sequence n's chunks are cut into segments of `seg` chunks (one
@@ -207,33 +208,37 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
       const int ci = c_begin + j, t0 = s + j * kChunk, L = min(kChunk, e - t0);
       // K, Q: the prep kernel's fp16 copies (contiguous), or the caller's rows
       // (rows past the sequence end read as 0)
-      const size_t qo = ((size_t)t0 * a.Hqk + hq) * K, co = (size_t)ci * a.Hqk + hq;
-      const int rows = L * a.Hqk * K * 2;
+      const size_t co = (size_t)ci * a.Hqk + hq;
+      const uint16_t* kp = a.k + (size_t)t0 * a.ts.k + hq * K;
+      const uint16_t* qp = a.q + (size_t)t0 * a.ts.q + hq * K;
       const __amdgpu_buffer_rsrc_t rk =
           COPY ? __builtin_amdgcn_make_buffer_rsrc(ws.k16 + co * KL::BYTES, 0, KL::BYTES,
                                                    kBufferFlags)
-               : __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.k + qo), 0, rows,
+               : __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kp), 0, L * a.ts.k * 2,
                                                    kBufferFlags);
       const __amdgpu_buffer_rsrc_t rq =
           COPY ? __builtin_amdgcn_make_buffer_rsrc(ws.q16 + co * 4 * KB * 64, 0, 128 * K,
                                                    kBufferFlags)
-               : __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.q + qo), 0, rows,
+               : __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(qp), 0, L * a.ts.q * 2,
                                                    kBufferFlags);
 #pragma unroll
       for (int i = 0; i < KPT; ++i) {
         const int x = tid + HT * i;
-        const int at = COPY ? 16 * x : (x / UPR) * a.Hqk * K * 2 + 16 * (x % UPR);
-        r.k[i] = __builtin_amdgcn_raw_buffer_load_b128(rk, at, 0, 0);
-        if constexpr (OUT) r.q[i] = __builtin_amdgcn_raw_buffer_load_b128(rq, at, 0, 0);
+        const int row = x / UPR, unit = 16 * (x % UPR);
+        r.k[i] = __builtin_amdgcn_raw_buffer_load_b128(
+            rk, COPY ? 16 * x : row * a.ts.k * 2 + unit, 0, 0);
+        if constexpr (OUT)
+          r.q[i] = __builtin_amdgcn_raw_buffer_load_b128(
+              rq, COPY ? 16 * x : row * a.ts.q * 2 + unit, 0, 0);
       }
       const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<uint16_t*>(a.v + ((size_t)t0 * a.Hv + h) * V), 0,
-          mpart ? 0 : L * a.Hv * V * 2, kBufferFlags);   // (a transfer matrix has V = 0)
+          const_cast<uint16_t*>(a.v + (size_t)t0 * a.ts.v + h * V), 0,
+          mpart ? 0 : L * a.ts.v * 2, kBufferFlags);   // (a transfer matrix has V = 0)
 #pragma unroll
       for (int i = 0; i < VPT; ++i) {
         const int x = tid + HT * i;
         r.v[i] = __builtin_amdgcn_raw_buffer_load_b128(
-            rv, (x / (V / 8)) * a.Hv * V * 2 + 16 * (x % (V / 8)), 0, 0);
+            rv, (x / (V / 8)) * a.ts.v * 2 + 16 * (x % (V / 8)), 0, 0);
       }
       const size_t fo = ((size_t)ci * a.Hv + h) * 6 * 64;
 #pragma unroll
@@ -832,9 +837,9 @@ __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkW
 template <int K, bool SAVE, bool OUT>
 void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, const float* h0,
                        float* ht, uint16_t* o, const int32_t* cu, int N, int T, int total, int Hqk,
-                       int Hv, int V, float scale, bool l2, const WsPlan& p, const ChunkWs& ws,
-                       hipStream_t st) {
-  const HeadArgs a{q, k, v, h0, ht, o, cu, N, T, total, Hqk, Hv, scale, p.seg};
+                       int Hv, int V, float scale, bool l2, TokenStride ts, const WsPlan& p,
+                       const ChunkWs& ws, hipStream_t st) {
+  const HeadArgs a{q, k, v, h0, ht, o, cu, N, T, total, Hqk, Hv, scale, p.seg, ts};
   const unsigned grid = (unsigned)((p.seg ? p.nseg : N) * Hv);
   auto go = [&](auto kern, unsigned g) {
     hipLaunchKernelGGL(kern, dim3(g), dim3(4 * V), 0, st, a, ws);
@@ -861,7 +866,7 @@ void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, 
 #define GDN_HEAD_INST(K_, SAVE_, OUT_)                                                       \
   template void launch_chain_head<K_, SAVE_, OUT_>(                                          \
       const uint16_t*, const uint16_t*, const uint16_t*, const float*, float*, uint16_t*,    \
-      const int32_t*, int, int, int, int, int, int, float, bool, const WsPlan&,              \
+      const int32_t*, int, int, int, int, int, int, float, bool, TokenStride, const WsPlan&, \
       const ChunkWs&, hipStream_t);
 GDN_HEAD_INST(64, false, true)
 GDN_HEAD_INST(64, true, false)

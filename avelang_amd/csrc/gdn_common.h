@@ -18,6 +18,13 @@ typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kChunk = 64;  // tokens per chunk of the prefill path
+
+// Elements from one token's rows to the next's in q, k and v (heads and their
+// elements contiguous): Hqk K, Hqk K and Hv V, or more for the column slices of
+// a wider tensor.
+struct TokenStride {
+  int q, k, v;
+};
 // Word 3 of a raw (stride 0) buffer resource on gfx950: out-of-range loads
 // return 0 and out-of-range stores are dropped.
 constexpr int kBufferFlags = 0x00020000;

@@ -26,6 +26,7 @@
 //     o  = scale (e^g S^T q + d (k.q))
 // so the updated tile never has to be re-read.
 #include "gdn_common.h"
+#include "../../include/gdn_rows.h"
 
 namespace gdn {
 
@@ -57,7 +58,7 @@ __global__ __launch_bounds__(NT) void recurrent_kernel(
     uint16_t* __restrict__ o, const int32_t* __restrict__ cu, int T,
     int total_tokens, int Hqk, int Hv, float scale, int l2norm,
     const int32_t* __restrict__ slots, int num_slots, int ntiles, int slot_stride,
-    const int32_t* __restrict__ accepted, GateIn gate) {
+    const int32_t* __restrict__ accepted, GateIn gate, TokenStride ts) {
   constexpr int COLG = V / 4;          // float4 column groups per row
   constexpr int ROWG = NT / COLG;      // row groups
   constexpr int RPT = K / ROWG;        // rows per lane
@@ -225,7 +226,6 @@ __global__ __launch_bounds__(NT) void recurrent_kernel(
           gsh[1] = b0;
         }
       }
-      const size_t qk_row = ((size_t)t * Hqk + hq) * K;
       // speculative decoding: slot receiving the state after this token
       int tslot = -1;
       if (slot_stride > 0 && t - s < slot_stride) {
@@ -233,11 +233,11 @@ __global__ __launch_bounds__(NT) void recurrent_kernel(
         if (tslot >= num_slots) tslot = -1;
       }
       if (tid < K) {
-        kq_s[0][tid] = bf2f(k[qk_row + tid]);
-        kq_s[1][tid] = bf2f(q[qk_row + tid]);
+        kq_s[0][tid] = bf2f(k[(size_t)t * ts.k + hq * K + tid]);
+        kq_s[1][tid] = bf2f(q[(size_t)t * ts.q + hq * K + tid]);
       }
       const size_t vh = (size_t)t * Hv + h;
-      const u16x4 vb = *reinterpret_cast<const u16x4*>(v + vh * V + 4 * cg);
+      const u16x4 vb = *reinterpret_cast<const u16x4*>(v + (size_t)t * ts.v + h * V + 4 * cg);
       float gt = 0.f, bt = 0.f;
       if constexpr (GATE) {
         // later tokens (multi-token steps): formed here
@@ -353,7 +353,8 @@ static void launch_recurrent(const uint16_t* q, const uint16_t* k, const uint16_
                              int Hqk, int Hv, int N, float scale, int l2norm,
                              const int32_t* slots, int num_slots, hipStream_t stream,
                              int slot_stride = 0, const int32_t* accepted = nullptr,
-                             const GateIn& gate = GateIn{}) {
+                             const GateIn& gate = GateIn{}, const TokenStride* rows = nullptr) {
+  const TokenStride ts = rows ? *rows : TokenStride{Hqk * K, Hqk * K, Hv * V};
   const int total_tokens = B * T;
   constexpr int NT = (K * V >= 128 * 128) ? 512 : 256;
   const int ntiles = N * Hv;
@@ -363,11 +364,11 @@ static void launch_recurrent(const uint16_t* q, const uint16_t* k, const uint16_
   if (gate.a)
     hipLaunchKernelGGL((recurrent_kernel<K, V, NT, true>), dim3(grid), dim3(NT), 0, stream, q,
                        k, v, g, beta, h0, ht, o, cu, T, total_tokens, Hqk, Hv, scale, l2norm,
-                       slots, num_slots, ntiles, slot_stride, accepted, gate);
+                       slots, num_slots, ntiles, slot_stride, accepted, gate, ts);
   else
     hipLaunchKernelGGL((recurrent_kernel<K, V, NT, false>), dim3(grid), dim3(NT), 0, stream, q,
                        k, v, g, beta, h0, ht, o, cu, T, total_tokens, Hqk, Hv, scale, l2norm,
-                       slots, num_slots, ntiles, slot_stride, accepted, gate);
+                       slots, num_slots, ntiles, slot_stride, accepted, gate, ts);
 }
 
 }  // namespace gdn
@@ -376,6 +377,9 @@ namespace gdn_host {
 int validate_gate(const char* name, const void* A_log, const void* dt_bias, int a_dtype,
                   int b_dtype, int p_dtype, float sp_beta, long long tokens);
 int validate_gate_size(const char* name, long long elements);
+int validate_rows(const char* name, const void* q, const void* k, const void* v, long long q_row,
+                  long long k_row, long long v_row, const void* o, long long tokens, int Hqk,
+                  int Hv, int K, int V, gdn::TokenStride& ts);
 int validate_common(const void* q, const void* k, const void* v, const float* g,
                     const float* beta, const float* h0, const float* ht, const void* o,
                     const int32_t* cu, int B, int T, int Hqk, int Hv, int K, int V, int N);
@@ -387,7 +391,7 @@ int recurrent_plain(const void* q, const void* k, const void* v, const float* g,
                     const float* beta, const float* h0, float* ht, void* o,
                     const int32_t* cu_seqlens, int B, int T, int Hqk, int Hv, int K, int V, int N,
                     float scale, int use_qk_l2norm, const gdn::GateIn& gate, void* stream,
-                    const char* name) {
+                    const char* name, const gdn::TokenStride* rows = nullptr) {
   if (N == 0 || ((long long)B * T == 0 && !ht)) return GDN_OK;  // nothing to compute
   gdn_host::launch_begin();
   auto* qq = static_cast<const uint16_t*>(q);
@@ -399,7 +403,7 @@ int recurrent_plain(const void* q, const void* k, const void* v, const float* g,
   if (K == KK && V == VV) {                                                               \
     gdn::launch_recurrent<KK, VV>(qq, kk, vv, g, beta, h0, ht, oo, cu_seqlens, B, T, Hqk, \
                                   Hv, N, scale, use_qk_l2norm, nullptr, N, st, 0, nullptr, \
-                                  gate);                                                  \
+                                  gate, rows);                                                  \
     return gdn_host::check_launch(name);                                                  \
   }
   GDN_REC(128, 128)
@@ -416,7 +420,7 @@ int recurrent_indexed(const void* q, const void* k, const void* v, const float* 
                       const int32_t* cu_seqlens, const int32_t* state_indices, int B, int T,
                       int Hqk, int Hv, int K, int V, int N, int num_slots, float scale,
                       int use_qk_l2norm, const gdn::GateIn& gate, void* stream,
-                      const char* name) {
+                      const char* name, const gdn::TokenStride* rows = nullptr) {
   if (num_slots < 0)
     return gdn_host::fail(GDN_ERR_SHAPE, std::string(name) + ": num_slots must be >= 0");
   if (N > 0 && !state_indices)
@@ -438,7 +442,7 @@ int recurrent_indexed(const void* q, const void* k, const void* v, const float* 
   if (K == KK && V == VV) {                                                               \
     gdn::launch_recurrent<KK, VV>(qq, kk, vv, g, beta, h0, ht, oo, cu_seqlens, B, T, Hqk, \
                                   Hv, N, scale, use_qk_l2norm, state_indices, num_slots,  \
-                                  st, 0, nullptr, gate);                                  \
+                                  st, 0, nullptr, gate, rows);                                  \
     return gdn_host::check_launch(name);                                                  \
   }
   GDN_RECI(128, 128)
@@ -553,4 +557,44 @@ extern "C" int gdn_recurrent_fwd_spec(const void* q, const void* k, const void* 
   GDN_RECS(64, 128)
 #undef GDN_RECS
   return gdn_host::fail(GDN_ERR_SHAPE, "gdn_recurrent_fwd_spec: unsupported K/V");
+}
+
+// Decode on column slices of wider tensors (declared in gdn_rows.h).
+extern "C" int gdn_recurrent_fwd_rows(const void* q, const void* k, const void* v, long long q_row,
+                                      long long k_row, long long v_row, const float* g,
+                                      const float* beta, const void* A_log, const void* a,
+                                      const void* b, const void* dt_bias, int a_dtype,
+                                      int b_dtype, int p_dtype, float sp_beta, float sp_threshold,
+                                      const float* h0, float* ht, void* o,
+                                      const int32_t* cu_seqlens, const int32_t* state_indices,
+                                      int B, int T, int Hqk, int Hv, int K, int V, int N,
+                                      int num_slots, float scale, int use_qk_l2norm,
+                                      void* stream) {
+  const char* name = "gdn_recurrent_fwd_rows";
+  const float* gg = A_log ? static_cast<const float*>(a) : g;
+  const float* bb = A_log ? static_cast<const float*>(b) : beta;
+  int rc = gdn_host::validate_common(q, k, v, gg, bb, state_indices ? nullptr : h0,
+                                     state_indices ? nullptr : ht, o, cu_seqlens, B, T, Hqk, Hv, K,
+                                     V, N);
+  if (rc) return rc;
+  gdn::TokenStride ts;
+  rc = gdn_host::validate_rows(name, q, k, v, q_row, k_row, v_row, o, (long long)B * T, Hqk, Hv, K,
+                               V, ts);
+  if (rc) return rc;
+  gdn::GateIn gate{};
+  if (A_log) {
+    rc = gdn_host::validate_gate(name, A_log, dt_bias, a_dtype, b_dtype, p_dtype, sp_beta,
+                                 (long long)B * T);
+    if (rc) return rc;
+    rc = gdn_host::validate_gate_size(name, (long long)B * T * Hv);
+    if (rc) return rc;
+    gate = gdn::GateIn{A_log, a, b, dt_bias, a_dtype, b_dtype, p_dtype, sp_beta, sp_threshold,
+                       (long long)B * T * Hv, Hv};
+    g = beta = nullptr;
+  }
+  if (state_indices)
+    return recurrent_indexed(q, k, v, g, beta, h0, ht, o, cu_seqlens, state_indices, B, T, Hqk, Hv,
+                             K, V, N, num_slots, scale, use_qk_l2norm, gate, stream, name, &ts);
+  return recurrent_plain(q, k, v, g, beta, h0, ht, o, cu_seqlens, B, T, Hqk, Hv, K, V, N, scale,
+                         use_qk_l2norm, gate, stream, name, &ts);
 }

@@ -42,14 +42,47 @@ _HEAD_SIZES = (64, 128)
 
 
 def _stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the raw handle, without a Stream object around it (~1 us of a decode call)
+    return torch._C._cuda_getCurrentRawStream(
+        device.index if device.index is not None else torch.cuda.current_device())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
-def _check_inputs(q, k, v, g, beta, initial_state, cu_seqlens, name, convert_gates=True):
+def _row(t: torch.Tensor) -> Optional[int]:
+    """Elements from one token of ``t`` [B, T, H, D] to the next, if the kernels
+    can read it in place: a token's heads contiguous, 16-byte aligned, tokens
+    evenly spaced and apart (a column slice of a wider tensor); else None."""
+    B, T, H, D = t.shape
+    s0, s1, s2, s3 = t.stride()
+    row = s1 if T > 1 else (s0 if B > 1 else H * D)
+    if (s3 != 1 or (H > 1 and s2 != D) or (B > 1 and T > 1 and s0 != T * s1) or row < H * D
+            or row % 8 or row >= 1 << 23 or t.data_ptr() % 16):
+        return None
+    return row
+
+
+def _rows(q, k, v) -> Optional[Tuple[int, int, int]]:
+    """Token strides of q, k, v for the ``*_rows`` entry points, or None where all
+    three are contiguous or one cannot be read in place."""
+    if q.is_contiguous() and k.is_contiguous() and v.is_contiguous():
+        return None
+    rows = (_row(q), _row(k), _row(v))
+    return None if None in rows else rows
+
+
+def _in_place(q, k, v):
+    """q, k, v as the kernels take them, and their token strides (None: contiguous)."""
+    rows = _rows(q, k, v)
+    if rows is None:
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    return q, k, v, rows
+
+
+def _check_inputs(q, k, v, g, beta, initial_state, cu_seqlens, name, convert_gates=True,
+                  contiguous=True):
     for nm, t in (("q", q), ("k", k), ("v", v)):
         if not isinstance(t, torch.Tensor):
             raise ValueError(f"{name}: {nm} must be a torch.Tensor")
@@ -58,11 +91,11 @@ def _check_inputs(q, k, v, g, beta, initial_state, cu_seqlens, name, convert_gat
         if t.dim() != 4:
             raise ValueError(f"{name}: {nm} must be 4-D [B, T, H, D], got {tuple(t.shape)}.")
     B, T, Hqk, K = q.shape
-    if tuple(k.shape) != (B, T, Hqk, K):
+    if k.shape != q.shape:
         raise ValueError(f"{name}: k must have shape {tuple(q.shape)}, got {tuple(k.shape)}.")
-    if tuple(v.shape[:2]) != (B, T):
+    Bv, Tv, Hv, V = v.shape
+    if Bv != B or Tv != T:
         raise ValueError(f"{name}: v must have shape [B, T, Hv, V] with B, T = {B}, {T}.")
-    Hv, V = v.shape[2], v.shape[3]
     if Hqk == 0 or Hv % Hqk != 0:
         raise ValueError(f"{name}: v-heads ({Hv}) must be a multiple of qk-heads ({Hqk}).")
     if K not in _HEAD_SIZES or V not in _HEAD_SIZES:
@@ -70,7 +103,7 @@ def _check_inputs(q, k, v, g, beta, initial_state, cu_seqlens, name, convert_gat
     for nm, t in (("g", g), ("beta", beta)):
         if not isinstance(t, torch.Tensor):
             raise ValueError(f"{name}: {nm} must be a torch.Tensor")
-        if tuple(t.shape) != (B, T, Hv):
+        if t.shape != (B, T, Hv):
             raise ValueError(f"{name}: {nm} must have shape {(B, T, Hv)}, got {tuple(t.shape)}.")
         if not t.is_floating_point():
             raise ValueError(f"{name}: {nm} must be floating point, got {t.dtype}.")
@@ -106,7 +139,7 @@ def _check_inputs(q, k, v, g, beta, initial_state, cu_seqlens, name, convert_gat
         cu = None
 
     if initial_state is not None:
-        if tuple(initial_state.shape) != (N, Hv, K, V):
+        if initial_state.shape != (N, Hv, K, V):
             raise ValueError(f"{name}: initial_state must have shape {(N, Hv, K, V)}, "
                              f"got {tuple(initial_state.shape)}.")
         if initial_state.dtype != torch.float32:
@@ -118,8 +151,19 @@ def _check_inputs(q, k, v, g, beta, initial_state, cu_seqlens, name, convert_gat
         beta = beta.to(torch.float32).contiguous()
     else:   # the gating inputs a, b of the fused entry points, in their own dtype
         g, beta = g.contiguous(), beta.contiguous()
-    return (q.contiguous(), k.contiguous(), v.contiguous(), g, beta, cu,
-            (B, T, Hqk, Hv, K, V, N))
+    if contiguous:   # else the caller takes slices as they are (_in_place)
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    return q, k, v, g, beta, cu, (B, T, Hqk, Hv, K, V, N)
+
+
+def _out(v, out, name):
+    """The caller's ``out``, checked, or a new contiguous tensor of v's shape."""
+    if out is None:
+        return torch.empty_like(v, memory_format=torch.contiguous_format)
+    if (out.shape != v.shape or out.dtype != torch.bfloat16 or out.device != v.device
+            or not out.is_contiguous()):
+        raise ValueError(f"{name}: out must be a contiguous bf16 tensor of shape {tuple(v.shape)}.")
+    return out
 
 
 def chunk_workspace_bytes(B: int, T: int, Hqk: int, Hv: int, K: int, V: int, N: int,
@@ -352,13 +396,15 @@ def _chunk_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, cu_se
     backward-sized workspace the backward then reuses), or with ``gate``
     gdn_chunk_fwd_gating (g, beta are then the gating inputs a, b)."""
     q, k, v, g, beta, cu, (B, T, Hqk, Hv, K, V, N) = _check_inputs(
-        q, k, v, g, beta, initial_state, cu_seqlens, name, convert_gates=gate is None)
+        q, k, v, g, beta, initial_state, cu_seqlens, name, convert_gates=gate is None,
+        contiguous=save_workspace is not None)
+    rows = None
+    if save_workspace is None:
+        q, k, v, rows = _in_place(q, k, v)
     if scale is None:
         scale = K ** -0.5
     dev = q.device
-    o = torch.empty_like(v) if out is None else out
-    if o.shape != v.shape or o.dtype != torch.bfloat16 or o.device != dev or not o.is_contiguous():
-        raise ValueError(f"{name}: out must be a contiguous bf16 tensor of shape {tuple(v.shape)}.")
+    o = _out(v, out, name)
     h0 = initial_state.contiguous() if initial_state is not None else None
     ht = None
     if output_final_state:
@@ -381,6 +427,15 @@ def _chunk_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, cu_se
         workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
     elif workspace.numel() * workspace.element_size() < nbytes or workspace.device != dev:
         raise ValueError(f"{name}: workspace must be >= {nbytes} bytes on {dev}.")
+    if rows is not None:
+        rc = _native.lib().gdn_chunk_fwd_rows(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), *rows,
+            *_rows_gates(gate, g, beta, Hv, dev, name), _ptr(h0), _ptr(ht), o.data_ptr(), _ptr(cu),
+            B, T, Hqk, Hv, K, V, N, float(scale), int(bool(use_qk_l2norm_in_kernel)),
+            workspace.data_ptr(), workspace.numel() * workspace.element_size(),
+            _stream_ptr(dev))
+        _native.check(rc, name)
+        return o, ht
     if gate is not None:
         rc = _native.lib().gdn_chunk_fwd_gating(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), *_gate_ptrs(gate, g, beta, Hv, dev, name),
@@ -460,13 +515,13 @@ def fused_recurrent_gated_delta_rule(
 def _recurrent_plain(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens,
                      use_qk_l2norm_in_kernel, inplace_final_state, out, name, gate=None):
     q, k, v, g, beta, cu, (B, T, Hqk, Hv, K, V, N) = _check_inputs(
-        q, k, v, g, beta, initial_state, cu_seqlens, name, convert_gates=gate is None)
+        q, k, v, g, beta, initial_state, cu_seqlens, name, convert_gates=gate is None,
+        contiguous=False)
+    q, k, v, rows = _in_place(q, k, v)
     if scale is None:
         scale = K ** -0.5
     dev = q.device
-    o = torch.empty_like(v) if out is None else out
-    if o.shape != v.shape or o.dtype != torch.bfloat16 or o.device != dev or not o.is_contiguous():
-        raise ValueError(f"{name}: out must be a contiguous bf16 tensor of shape {tuple(v.shape)}.")
+    o = _out(v, out, name)
     h0 = initial_state
     if h0 is not None and not h0.is_contiguous():
         if output_final_state and inplace_final_state:
@@ -478,7 +533,13 @@ def _recurrent_plain(q, k, v, g, beta, scale, initial_state, output_final_state,
             ht = h0
         else:
             ht = torch.empty((N, Hv, K, V), dtype=torch.float32, device=dev)
-    if gate is not None:
+    if rows is not None:
+        rc = _native.lib().gdn_recurrent_fwd_rows(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), *rows,
+            *_rows_gates(gate, g, beta, Hv, dev, name), _ptr(h0), _ptr(ht), o.data_ptr(), _ptr(cu),
+            None, B, T, Hqk, Hv, K, V, N, N, float(scale), int(bool(use_qk_l2norm_in_kernel)),
+            _stream_ptr(dev))
+    elif gate is not None:
         rc = _native.lib().gdn_recurrent_fwd_gating(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), *_gate_ptrs(gate, g, beta, Hv, dev, name),
             _ptr(h0), _ptr(ht), o.data_ptr(), _ptr(cu), None,
@@ -502,7 +563,8 @@ def _recurrent_indexed(q, k, v, g, beta, scale, pool, output_final_state, cu_seq
     if output_final_state and not inplace_final_state:
         raise ValueError(f"{name}: with ssm_state_indices the final state is written in place.")
     q, k, v, g, beta, cu, (B, T, Hqk, Hv, K, V, N) = _check_inputs(
-        q, k, v, g, beta, None, cu_seqlens, name, convert_gates=gate is None)
+        q, k, v, g, beta, None, cu_seqlens, name, convert_gates=gate is None, contiguous=False)
+    q, k, v, rows = _in_place(q, k, v)
     dev = q.device
     if (tuple(pool.shape[1:]) != (Hv, K, V) or pool.dtype != torch.float32
             or pool.device != dev or not pool.is_contiguous()):
@@ -516,11 +578,15 @@ def _recurrent_indexed(q, k, v, g, beta, scale, pool, output_final_state, cu_seq
     idx = idx.to(dev)
     if scale is None:
         scale = K ** -0.5
-    o = torch.empty_like(v) if out is None else out
-    if o.shape != v.shape or o.dtype != torch.bfloat16 or o.device != dev or not o.is_contiguous():
-        raise ValueError(f"{name}: out must be a contiguous bf16 tensor of shape {tuple(v.shape)}.")
+    o = _out(v, out, name)
     ht = pool if output_final_state else None
-    if gate is not None:
+    if rows is not None:
+        rc = _native.lib().gdn_recurrent_fwd_rows(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), *rows,
+            *_rows_gates(gate, g, beta, Hv, dev, name), pool.data_ptr(), _ptr(ht), o.data_ptr(),
+            _ptr(cu), idx.contiguous().data_ptr(), B, T, Hqk, Hv, K, V, N, pool.shape[0],
+            float(scale), int(bool(use_qk_l2norm_in_kernel)), _stream_ptr(dev))
+    elif gate is not None:
         rc = _native.lib().gdn_recurrent_fwd_gating(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), *_gate_ptrs(gate, g, beta, Hv, dev, name),
             pool.data_ptr(), _ptr(ht), o.data_ptr(), _ptr(cu), idx.contiguous().data_ptr(),
@@ -608,6 +674,14 @@ def _gate_ptrs(gate, a, b, Hv, dev, name):
     adt, bdt, pdt = _dt(a, name, "a"), _dt(b, name, "b"), _dt(A_log, name, "A_log")
     return (A_log.contiguous().data_ptr(), a.data_ptr(), b.data_ptr(),
             dt_bias.contiguous().data_ptr(), adt, bdt, pdt, float(spb), float(spt))
+
+
+def _rows_gates(gate, g, beta, Hv, dev, name):
+    """The gate arguments of the *_rows entry points: g, beta, or (``gate``) the
+    gating parameters and inputs a, b in their place."""
+    if gate is None:
+        return g.data_ptr(), beta.data_ptr(), None, None, None, None, 0, 0, 0, 1.0, 20.0
+    return None, None, *_gate_ptrs(gate, g, beta, Hv, dev, name)
 
 
 def chunk_gated_delta_rule_gated(
