@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const float* __restrict__ g, const float* __restrict__ beta,
     const int32_t* __restrict__ cu, int N, int T, int total, int Hqk, int Hv, float scale,
-    ChunkWs ws, GateIn gate, TokenStride ts) {
+    ChunkWs ws, GateIn gate, TokenStride ts, int ncmax, int apart) {
   constexpr int KB = K / 32;
   // strictly lower 16 x 16 blocks of A only (block (bi, m), m < bi, at
   // bi (bi - 1) / 2 + m; row stride 20 keeps float4 rows aligned and the 16
@@ -202,8 +202,18 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(
   // P (bf16, row-major) for the P^T fragments (backward only)
   __shared__ __attribute__((aligned(16))) uint16_t Ps[BWD ? 64 : 1][72];
 
-  const int ci = blockIdx.x;
-  const int h = blockIdx.y;
+  // The G v-heads of a (chunk, qk-head) read the same K, Q rows: their
+  // workgroups are `apart` (a multiple of 8, 128 at most) from each other, so
+  // on one XCD (workgroups are dealt to the 8 XCDs in turn) and close enough
+  // that the later ones find the rows in its L2 -- a head-major order has them
+  // a whole sequence apart.  32 v-heads: T = 65536 291 -> 270 us, 64 sequences
+  // of 513-4096 685 -> 658, T = 8192 the same 32.6.  8 apart, both miss at
+  // once: 260 at T = 65536 but 33.2 at 8192 and 26.5 for 25.6 at 4096.
+  const int slot = blockIdx.x % (apart * (Hv / Hqk));
+  const int pair = blockIdx.x / (apart * (Hv / Hqk)) * apart + slot % apart;   // (chunk, qk-head)
+  const int ci = pair % ncmax;
+  const int h = pair / ncmax * (Hv / Hqk) + slot / apart;
+  if (pair >= ncmax * Hqk) return;
   int n, cfirst;
   if (cu) {
     const int32_t* off = ws.off;
@@ -676,12 +686,17 @@ static void launch_chunk(const uint16_t* q, const uint16_t* k, const uint16_t* v
     hipLaunchKernelGGL(chunk_table_kernel, dim3(1), dim3(256), 0, st, cu, N, T, total,
                        (int)p.ncmax, p.seg, ws.off, ws.soff, ws.status);
   if (p.ncmax > 0) {
+    const long long pairs = p.ncmax * (long long)Hqk;
+    const int apart = (int)std::min(128LL, (pairs + 7) / 8 * 8);
+    const unsigned grid = (unsigned)((pairs + apart - 1) / apart * apart * (Hv / Hqk));
     if (l2)
-      hipLaunchKernelGGL((chunk_prep_kernel<K, BWD, OUT, true>), dim3((unsigned)p.ncmax, Hv), dim3(256),
-                         0, st, q, k, g, beta, cu, N, T, total, Hqk, Hv, scale, ws, gate, ts);
+      hipLaunchKernelGGL((chunk_prep_kernel<K, BWD, OUT, true>), dim3(grid), dim3(256),
+                         0, st, q, k, g, beta, cu, N, T, total, Hqk, Hv, scale, ws, gate, ts,
+                         (int)p.ncmax, apart);
     else
-      hipLaunchKernelGGL((chunk_prep_kernel<K, BWD, OUT, false>), dim3((unsigned)p.ncmax, Hv), dim3(256),
-                         0, st, q, k, g, beta, cu, N, T, total, Hqk, Hv, scale, ws, gate, ts);
+      hipLaunchKernelGGL((chunk_prep_kernel<K, BWD, OUT, false>), dim3(grid), dim3(256),
+                         0, st, q, k, g, beta, cu, N, T, total, Hqk, Hv, scale, ws, gate, ts,
+                         (int)p.ncmax, apart);
   }
   // the chain reads K and Q as the prep kernel's fp16 copies where the plan
   // has them (normalised with use_qk_l2norm), else as the caller's bf16 rows

@@ -57,6 +57,14 @@ def test_whole_head(rocm_device, K, V, l2, T):
     _check(wl, rocm_device, l2, f"K{K} V{V} T{T}")
 
 
+@pytest.mark.parametrize("chunks,Hqk,Hv", [(1, 1, 1), (1, 1, 3), (3, 3, 6), (127, 1, 3),
+                                           (64, 2, 2), (43, 3, 9), (129, 1, 2), (51, 5, 10)])
+def test_prep_workgroup_order(rocm_device, chunks, Hqk, Hv):
+    """Every (chunk, v-head) once, with (chunk, qk-head) pairs under, at and over multiples of
+    the 128 that the prep kernel takes between two v-heads of a pair."""
+    _check(W.make(1, 64 * chunks - 5, Hqk, Hv, 128, 128, seed=chunks, h0_scale=0.01), rocm_device)
+
+
 def _cu(lens):
     return np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
 
