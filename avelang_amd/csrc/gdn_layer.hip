@@ -13,7 +13,7 @@
 // All of these are HBM-bound elementwise / stencil operators: the kernels
 // move 16 bytes per lane per access on their contiguous axis (a wavefront
 // covers 1 KiB), keep sliding windows in registers, and compute in fp32.
-#include "gdn_common.h"
+#include "gdn_chunk.h"
 #include "../../include/gdn_layer.h"
 
 namespace gdn {
@@ -272,11 +272,19 @@ struct ConvArgs {
 // bf16), each lane walks TT time steps with the last W-1 inputs in
 // registers.  Workgroups of one time tile are adjacent in dispatch order, so
 // a time step's row is read as a few wide pieces at once (measured: 4.2 TB/s
-// against 3.9 with 1 KiB pieces from 4 time tiles per workgroup).
-template <int DT, int W>
+// against 3.9 with 1 KiB pieces from 4 time tiles per workgroup).  The next U
+// steps' loads are in flight while U are computed, and the sequence ids'
+// compares are compiled in only where they are given.  Short calls are bound
+// by a tile's serial steps (conv1d_cl_tile), long ones by HBM; D = 8192 bf16,
+// loads of 8 steps then their arithmetic in tiles of 64 -> this: T = 256 31.1
+// -> 7.2 us, 1024 35.6 -> 13.6, 4096 39.2 -> 32.9 (4.1 TB/s), 8192 60 -> 56
+// (4.8 TB/s).  U = 8 is 5 to 9 % slower (registers: fewer waves), U = 2 the
+// same within a few percent.
+template <int DT, int W, bool SEQ>
 __global__ __launch_bounds__(256) void conv1d_cl_kernel(ConvArgs a, int TT) {
+  using E = typename Elt<DT>::T;
   constexpr int N = Elt<DT>::VEC;
-  constexpr int U = 8;   // time steps whose loads are issued together
+  constexpr int U = 4;   // time steps whose loads are issued together
   const int d0 = (blockIdx.x * 256 + threadIdx.x) * N;
   const int b = blockIdx.z;
   const int t0 = blockIdx.y * TT;
@@ -293,7 +301,7 @@ __global__ __launch_bounds__(256) void conv1d_cl_kernel(ConvArgs a, int TT) {
   }
   const long long xb = (long long)b * a.x_sb + d0;
   const long long ob = (long long)b * a.o_sb + d0;
-  const int32_t* sq = a.seq_idx ? a.seq_idx + (long long)b * a.T : nullptr;
+  const int32_t* sq = SEQ ? a.seq_idx + (long long)b * a.T : nullptr;
 
   // window slot j holds the input at t - (W-1) + j (oldest first) and its
   // sequence id (padding before the row start never matches a token)
@@ -304,33 +312,48 @@ __global__ __launch_bounds__(256) void conv1d_cl_kernel(ConvArgs a, int TT) {
     const int p = t0 - (W - 1) + j;
     if (p >= 0) {
       ldv<DT>(a.x, xb + p * a.x_st, win[j]);
-      sw[j] = sq ? sq[p] : 0;
+      if constexpr (SEQ) sw[j] = sq[p];
     } else {
 #pragma unroll
       for (int c = 0; c < N; ++c)
         win[j][c] = a.init ? lde<DT>(a.init, ((long long)b * a.D + d0 + c) * (W - 1) + (W - 1) + p)
                            : 0.f;
-      sw[j] = sq ? -2147483647 - 1 : 0;
+      if constexpr (SEQ) sw[j] = -2147483647 - 1;
     }
   }
-  for (int tb = t0; tb < t1; tb += U) {
-    float cur[U][N];
-    int sc[U];
+  uint4 nxt[U];
+  int sn[U];
+  const auto fetch = [&](int tb) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int t = min(tb + u, t1 - 1);   // clamped: steps past t1 are not used
-      ldv<DT>(a.x, xb + t * a.x_st, cur[u]);
-      sc[u] = sq ? sq[t] : 0;
+      nxt[u] = *reinterpret_cast<const uint4*>(static_cast<const E*>(a.x) + xb + t * a.x_st);
+      if constexpr (SEQ) sn[u] = sq[t];
     }
+  };
+  fetch(t0);
+  for (int tb = t0; tb < t1; tb += U) {
+    uint4 raw[U];
+    int sc[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      raw[u] = nxt[u];
+      if constexpr (SEQ) sc[u] = sn[u];
+    }
+    if (tb + U < t1) fetch(tb + U);   // in flight while this batch is computed
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (tb + u >= t1) break;
-      float acc[N];
+      float cur[N], acc[N];
+      const E* e = reinterpret_cast<const E*>(&raw[u]);
 #pragma unroll
-      for (int c = 0; c < N; ++c) acc[c] = bs[c] + wf[c * W + W - 1] * cur[u][c];
+      for (int c = 0; c < N; ++c) {
+        cur[c] = Elt<DT>::to_f(e[c]);
+        acc[c] = bs[c] + wf[c * W + W - 1] * cur[c];
+      }
 #pragma unroll
       for (int j = 0; j < W - 1; ++j) {
-        if (sw[j] == sc[u]) {
+        if (!SEQ || sw[j] == sc[u]) {
 #pragma unroll
           for (int c = 0; c < N; ++c) acc[c] += wf[c * W + j] * win[j][c];
         }
@@ -344,11 +367,11 @@ __global__ __launch_bounds__(256) void conv1d_cl_kernel(ConvArgs a, int TT) {
       for (int j = 0; j + 1 < W - 1; ++j) {
 #pragma unroll
         for (int c = 0; c < N; ++c) win[j][c] = win[j + 1][c];
-        sw[j] = sw[j + 1];
+        if constexpr (SEQ) sw[j] = sw[j + 1];
       }
 #pragma unroll
-      for (int c = 0; c < N; ++c) win[W - 2][c] = cur[u][c];
-      sw[W - 2] = sc[u];
+      for (int c = 0; c < N; ++c) win[W - 2][c] = cur[c];
+      if constexpr (SEQ) sw[W - 2] = sc[u];
     }
   }
   // the tile that ends the row leaves the last W-1 inputs in its window
@@ -739,6 +762,21 @@ extern "C" int gdn_rmsnorm_gated_fwd(const void* x, const void* z, const void* w
 
 namespace {
 
+// Time steps per workgroup of conv1d_cl_kernel, `rows` workgroups per time
+// tile.  A tile is a serial chain of about 0.45 us per step and re-reads W-1
+// rows before it (from beyond L2), so tiles are as long as the grid still
+// fills the chip: 32 from two workgroups per CU on (D = 8192, bf16: T = 4096
+// 32.9 us against 34.6 in tiles of 16 and 36.2 of 64), 16 over one
+// (T = 2048 20.8, 22.3 of 32, 21.3 of 8), else 8 (T = 256 7.2, 10.0 of 16;
+// T = 1024, 256 workgroups of 16, 13.6 against 14.4).  A row over 2^21 steps
+// takes 64: the grid's y stays under 2^16 as far as it can.
+int conv1d_cl_tile(long long rows, long long T) {
+  const long long cus = gdn::device_cus();
+  if ((T + 31) / 32 > 65535) return 64;
+  if (rows * ((T + 31) / 32) >= 2 * cus) return 32;
+  return rows * ((T + 15) / 16) > cus ? 16 : 8;
+}
+
 template <int DT, int W>
 int launch_conv(const gdn::ConvArgs& a, hipStream_t st) {
   const int N = vec_of(DT);
@@ -756,10 +794,13 @@ int launch_conv(const gdn::ConvArgs& a, hipStream_t st) {
   }
   if (a.x_sd == 1 && a.o_sd == 1 && a.D % N == 0 && a.x_sb % N == 0 && a.x_st % N == 0 &&
       a.o_sb % N == 0 && a.o_st % N == 0 && vec_aligned_x && vec_aligned_o && vec_aligned_w) {
-    const int TT = 64;   // halo re-reads (W-1 rows per tile) miss L2: keep tiles long
+    const int TT = conv1d_cl_tile((a.D / N + 255) / 256 * (long long)a.B, a.T);
     const dim3 grid((unsigned)((a.D / N + 255) / 256), (unsigned)((a.T + TT - 1) / TT),
                     (unsigned)a.B);
-    hipLaunchKernelGGL((gdn::conv1d_cl_kernel<DT, W>), grid, dim3(256), 0, st, a, TT);
+    if (a.seq_idx)
+      hipLaunchKernelGGL((gdn::conv1d_cl_kernel<DT, W, true>), grid, dim3(256), 0, st, a, TT);
+    else
+      hipLaunchKernelGGL((gdn::conv1d_cl_kernel<DT, W, false>), grid, dim3(256), 0, st, a, TT);
   } else if (a.x_st == 1 && a.o_st == 1 && !a.seq_idx && !a.init && !a.final_states &&
              a.x_sb % N == 0 && a.x_sd % N == 0 && a.o_sb % N == 0 && a.o_sd % N == 0 &&
              vec_aligned_x && vec_aligned_o) {

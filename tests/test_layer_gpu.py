@@ -163,6 +163,31 @@ def test_conv_fn_seq_idx_and_states(rocm_device):
         np.testing.assert_array_equal(_np(fin), fref)
 
 
+@pytest.mark.parametrize("B,T", [(1, 1), (1, 7), (3, 8), (3, 9), (2, 21), (140, 16), (140, 17),
+                                 (140, 33), (520, 31), (520, 32), (520, 33), (520, 71)])
+@pytest.mark.parametrize("given", ["none", "seq_idx", "states"])
+def test_conv_fn_time_tiles(rocm_device, B, T, given):
+    """Time tiles of 8, 16 and 32 steps (few, some and many rows): a step under, at and over
+    their edges and those of the 4 steps loaded together."""
+    dev, D = rocm_device, 16
+    x, w, bias = _conv_case(dev, B, D, T, 4, torch.bfloat16, "channel_last", seed=T)
+    kw, ref_kw = {}, {}
+    if given == "seq_idx":
+        sq = (torch.arange(T, dtype=torch.int32, device=dev) // 5).repeat(B, 1)
+        kw, ref_kw = dict(seq_idx=sq), dict(seq_idx=_np(sq))
+    elif given == "states":
+        init = _rand((B, D, 3), dev, seed=B)
+        kw, ref_kw = (dict(initial_states=init, return_final_states=True),
+                      dict(initial_states=_np(init)))
+    got = L.causal_conv1d_fn(x, w, bias, activation="silu", **kw)
+    torch.cuda.synchronize()
+    ref, fref = LR.causal_conv1d(_np(x), _np(w), _np(bias), silu=True, **ref_kw)
+    if given == "states":
+        np.testing.assert_array_equal(_np(got[1]), fref)
+        got = got[0]
+    _close_lowp(got, ref, f"conv B{B} T{T} {given}")
+
+
 def test_conv_fn_qwen3_next_shape(rocm_device):
     """Layer shape (conv_dim 8192, T 8192, channel-last bf16): oracle on 96 channels."""
     dev = rocm_device
