@@ -73,9 +73,21 @@ def _rows(q, k, v) -> Optional[Tuple[int, int, int]]:
     return None if None in rows else rows
 
 
-def _in_place(q, k, v):
-    """q, k, v as the kernels take them, and their token strides (None: contiguous)."""
+def _span(t: torch.Tensor) -> Tuple[int, int]:
+    """First and past-the-last byte address of a non-empty strided tensor."""
+    last = sum((n - 1) * s for n, s in zip(t.shape, t.stride()))
+    return t.data_ptr(), t.data_ptr() + (last + 1) * t.element_size()
+
+
+def _in_place(q, k, v, out=None):
+    """q, k, v as the kernels take them, and their token strides (None: contiguous).
+    Slices that ``out`` lies on or between are copied: o is written while q, k, v
+    are still read."""
     rows = _rows(q, k, v)
+    if rows is not None and out is not None and out.numel() > 0:
+        a, b = _span(out)
+        if any(a < e and s < b for s, e in map(_span, (q, k, v))):
+            rows = None
     if rows is None:
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     return q, k, v, rows
@@ -400,7 +412,7 @@ def _chunk_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, cu_se
         contiguous=save_workspace is not None)
     rows = None
     if save_workspace is None:
-        q, k, v, rows = _in_place(q, k, v)
+        q, k, v, rows = _in_place(q, k, v, out)
     if scale is None:
         scale = K ** -0.5
     dev = q.device
@@ -517,7 +529,7 @@ def _recurrent_plain(q, k, v, g, beta, scale, initial_state, output_final_state,
     q, k, v, g, beta, cu, (B, T, Hqk, Hv, K, V, N) = _check_inputs(
         q, k, v, g, beta, initial_state, cu_seqlens, name, convert_gates=gate is None,
         contiguous=False)
-    q, k, v, rows = _in_place(q, k, v)
+    q, k, v, rows = _in_place(q, k, v, out)
     if scale is None:
         scale = K ** -0.5
     dev = q.device
@@ -564,7 +576,7 @@ def _recurrent_indexed(q, k, v, g, beta, scale, pool, output_final_state, cu_seq
         raise ValueError(f"{name}: with ssm_state_indices the final state is written in place.")
     q, k, v, g, beta, cu, (B, T, Hqk, Hv, K, V, N) = _check_inputs(
         q, k, v, g, beta, None, cu_seqlens, name, convert_gates=gate is None, contiguous=False)
-    q, k, v, rows = _in_place(q, k, v)
+    q, k, v, rows = _in_place(q, k, v, out)
     dev = q.device
     if (tuple(pool.shape[1:]) != (Hv, K, V) or pool.dtype != torch.float32
             or pool.device != dev or not pool.is_contiguous()):

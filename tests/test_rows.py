@@ -35,6 +35,36 @@ def test_layouts_taken_in_place():
         assert G._row(bad) is None or bad.is_contiguous()
 
 
+def test_out_on_the_slices_tensor():
+    """An out inside the tensor the slices are cut from is not written beside them: copies."""
+    q, k, v = _slices(1, 6, 2, 4, 64, 64)
+    flat = q._base.view(-1) if q._base is not None else q.reshape(-1)
+    n = 6 * 4 * 64
+    for out, taken in ((flat[:n].view(1, 6, 4, 64), False), (flat[-n:].view(1, 6, 4, 64), False),
+                       (torch.empty(1, 6, 4, 64, dtype=torch.bfloat16), True), (None, True)):
+        q2, k2, v2, rows = G._in_place(q, k, v, out)
+        assert (rows is not None) == taken
+        assert taken or all(x.is_contiguous() for x in (q2, k2, v2))
+        assert all(torch.equal(x, y) for x, y in ((q, q2), (k, k2), (v, v2)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("decode", [False, True])
+def test_out_over_the_slices_gpu(rocm_device, decode):
+    from avelang_amd import chunk_gated_delta_rule, fused_recurrent_gated_delta_rule
+    op = fused_recurrent_gated_delta_rule if decode else chunk_gated_delta_rule
+    B, T = (7, 1) if decode else (1, 130)
+    gates = _gates(B, T, 4, rocm_device, False)
+    kw = dict(output_final_state=True, use_qk_l2norm_in_kernel=True)
+    want, _ = op(*_slices(B, T, 2, 4, 128, 128, device=rocm_device), *gates, **kw)
+    q, k, v = _slices(B, T, 2, 4, 128, 128, device=rocm_device)
+    n = B * T * 4 * 128
+    out = q._base.view(-1)[-n:].view(B, T, 4, 128)
+    o, _ = op(q, k, v, *gates, out=out, **kw)
+    torch.cuda.synchronize()
+    assert o is out and torch.equal(o, want)
+
+
 def test_refused_rows():
     lib = _native.lib()
     for name in _native.EXPORTS_ROWS:
