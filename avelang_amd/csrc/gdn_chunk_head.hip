@@ -24,8 +24,9 @@
 // chunk, and a split into state and output waves 2.8.
 //
 // Staging: as many helper waves hold the next three chunks' K, Q and V units
-// and Tb / P fragments in registers (a load has two steps to land) and write them to the other of two LDS buffers, K (KLayout) and Q as fp16 --
-// COPY (use_qk_l2norm): the prep kernel's normalised fp16 copies as they are
+// and Tb / P fragments in registers (a load has two steps to land) and write
+// them to the other of two LDS buffers, K (KLayout) and Q as fp16 -- COPY
+// (use_qk_l2norm): the prep kernel's normalised fp16 copies as they are
 // (normalising here instead made the helper the longer wave: 2.9 us per
 // chunk) -- V as fp16, and the chunk's gate factors.
 //
