@@ -636,7 +636,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
     }
     if constexpr (SAVE) {
       // the chunk's deltas: lane t stores token row t (16 columns per tile),
-      // through this wave's own LDS rows
+      // through this wave's own LDS rows and four transposing reads per tile
       const int L = min(kChunk, e - (s + j * kChunk));
       const __amdgpu_buffer_rsrc_t dr = __builtin_amdgcn_make_buffer_rsrc(
           ws.dl + ((size_t)(c_begin + j) * a.Hv + h) * 64 * V, 0, 64 * V * 2, kBufferFlags);
@@ -647,14 +647,10 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
         for (int b = 0; b < 2; ++b) Vx[ct][b][lane] = vx[x][b];
         __builtin_amdgcn_wave_barrier();
         const uint16_t* src =
-            reinterpret_cast<const uint16_t*>(&Vx[ct][lane >> 5][16 * ((lane >> 3) & 3)]) +
-            (lane & 7);
-        u16x8 d0, d1;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          d0[c] = src[8 * c];
-          d1[c] = src[8 * (c + 8)];
-        }
+            reinterpret_cast<const uint16_t*>(
+                &Vx[ct][grp >> 1][16 * (2 * (grp & 1) + (q4 >> 1)) + m4]) + 4 * (q4 & 1);
+        u16x8 d0 = cat8(lds_tr16(src), lds_tr16(src + 32));
+        u16x8 d1 = cat8(lds_tr16(src + 64), lds_tr16(src + 96));
         const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
         d0 = lane < L ? h2bf8(d0) : zero;
         d1 = lane < L ? h2bf8(d1) : zero;
