@@ -851,6 +851,20 @@ void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, 
     const unsigned seqs = std::min<unsigned>(N, std::max(1u, 4u * device_cus() / tiles));
     hipLaunchKernelGGL((chunk_combine_kernel<K>), dim3(tiles, seqs), dim3(4 * K), 0, st, a, ws);
   }
+  // A training forward in segments forms saves and o in two launches: with both
+  // the kernel is 32 registers over its 256, and each reload waits until the
+  // step's stores are in memory.  T = 8192, 32 heads (160 workgroups): 177 us in
+  // one launch, 98 + 70 in two.  Whole sequences (many workgroups, HBM-bound)
+  // keep one launch and read the operands once.
+  if constexpr (SAVE && OUT && K == 128) {
+    if (p.seg && V == 128) {
+      if (l2) go(chunk_head_kernel<K, 128, true, true, false, false>, grid);
+      else go(chunk_head_kernel<K, 128, false, true, false, false>, grid);
+      if (l2) go(chunk_head_kernel<K, 128, true, false, true, false>, grid);
+      else go(chunk_head_kernel<K, 128, false, false, true, false>, grid);
+      return;
+    }
+  }
   if (V == 128) {
     if (l2) go(chunk_head_kernel<K, 128, true, SAVE, OUT, false>, grid);
     else go(chunk_head_kernel<K, 128, false, SAVE, OUT, false>, grid);
