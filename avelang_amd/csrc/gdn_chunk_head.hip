@@ -10,7 +10,10 @@
 // every product's result tile is the next product's B operand where it
 // stands; so the compute waves exchange nothing and one barrier per chunk
 // hands the operand buffers over.  Every product takes fp16 operands rounded
-// from fp32 (Q, K and V rows as fp16, exact in fp16's normal range).
+// from fp32 (K and V rows as fp16, exact in fp16's normal range; the caller's
+// Q rows times a power of two that brings the largest of 16 or 32 rows to
+// 2^14 .. 2^15, taken back from the output's factor: Q S is then as exact for
+// a q outside fp16's range as the state-wave form's bf16 product).
 //
 // What bounds it: with a workgroup on every compute unit HBM (64 packed
 // sequences x 32 heads: 4.4 GB in 880 us, 5.0 TB/s; the state-wave form, whose
@@ -138,6 +141,42 @@ __device__ __forceinline__ u16x4 fma_h4(f32x4 a, f32x4 b, u16x4 c) {
   return __builtin_bit_cast(u16x4, r);
 }
 
+// Eight bf16 values times s (a power of two), as fp16 in one rounding.
+__device__ __forceinline__ u16x8 scale_h8(u16x8 x, float s) {
+  constexpr u16x4 kNegZero4 = {0x8000, 0x8000, 0x8000, 0x8000};
+  const f32x8 f = __builtin_convertvector(__builtin_bit_cast(bf16x8, x), f32x8);
+  const f32x4 s4 = {s, s, s, s};
+  return cat8(fma_h4(f32x4{f[0], f[1], f[2], f[3]}, s4, kNegZero4),
+              fma_h4(f32x4{f[4], f[5], f[6], f[7]}, s4, kNegZero4));
+}
+// Biased exponent of the largest |x| of a wave's bf16 values, 15 at least (so
+// that 2^(141 - e) and its inverse are normal floats; 255: an inf or NaN).
+template <int N>
+__device__ __forceinline__ int q_exponent(const u32x4 (&x)[N]) {
+  float m = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+#pragma unroll
+    for (int y = 0; y < 4; ++y)   // (both values of the word, sign bits ignored)
+      asm("v_max3_f32 %0, |%1|, |%2|, %0"
+          : "+v"(m) : "v"(x[i][y] << 16), "v"(x[i][y] & 0xffff0000u));
+  }
+  unsigned u = __float_as_uint(m);
+  auto ror = [&](auto n) {
+    u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x120 + decltype(n)::value, 0xf, 0xf,
+                                                     false));
+  };
+  ror(std::integral_constant<int, 8>{});
+  ror(std::integral_constant<int, 4>{});
+  ror(std::integral_constant<int, 2>{});
+  ror(std::integral_constant<int, 1>{});
+  unsigned top = 0;
+#pragma unroll
+  for (int row = 0; row < 4; ++row)
+    top = max(top, (unsigned)__builtin_amdgcn_readlane((int)u, 16 * row));
+  return max((int)(top >> 23), 15);
+}
+
 // Workgroup bid of nb with a qk-head group's workgroups on one XCD (they read the
 // same K, Q rows; workgroups are dealt to the 8 XCDs in turn).
 __device__ __forceinline__ int group_block(int bid, int nb, int G) {
@@ -166,11 +205,13 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
   constexpr int VPT = 64 * (V / 8) / HT;     // V units per helper thread
   constexpr int NSL = OUT ? 12 : 6;          // fragment slots: Tb, then P
   constexpr int SPW = (NSL + NW - 1) / NW;   // fragment slots per helper wave
+  constexpr bool kRowsQ = OUT && !COPY;      // Q from the caller's rows
   // Operand buffer b of the two sits at byte kBufStep b of one block: every
   // fragment address is then a per-lane offset of the step's buffer plus an
   // immediate (under 64 KiB), with no address registers per buffer.
   constexpr int kQ = KL::BYTES, kV = kQ + (OUT ? 128 * K : 0), kF = kV + 128 * V;
-  constexpr int kG = kF + NSL * 1024, kE = kG + 512, kBufStep = (kE + 16 + 255) / 256 * 256;
+  constexpr int kG = kF + NSL * 1024, kO = kG + 512, kE = kO + (OUT ? 256 : 0);
+  constexpr int kBufStep = (kE + 16 + 255) / 256 * 256;
   static_assert(kBufStep <= 65536, "a buffer's offsets fit the LDS immediates");
   __shared__ __attribute__((aligned(256))) unsigned char buf[2 * kBufStep];
   __shared__ __attribute__((aligned(16))) u16x8 Vx[SAVE ? 2 * NW : 1][2][64];
@@ -256,6 +297,9 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
     };
     auto stage = [&](const Regs& r, int j, int b) {
       unsigned char* bp = buf + b * kBufStep;
+      int qe = 141;   // biased exponent of this wave's Q rows, its scale 2^(141 - qe)
+      if constexpr (kRowsQ) qe = q_exponent(r.q);
+      const float qs = __int_as_float((268 - qe) << 23);
 #pragma unroll
       for (int i = 0; i < KPT; ++i) {
         const int x = tid + HT * i;
@@ -267,7 +311,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
               bf2h8(__builtin_bit_cast(u16x8, r.k[i]));
           if constexpr (OUT)
             *reinterpret_cast<u16x8*>(bp + kQ + qrow_off<K>(x / UPR, x % UPR)) =
-                bf2h8(__builtin_bit_cast(u16x8, r.q[i]));
+                scale_h8(__builtin_bit_cast(u16x8, r.q[i]), qs);
         }
       }
 #pragma unroll
@@ -280,6 +324,12 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
       for (int i = 0; i < SPW; ++i)
         if (hw + NW * i < NSL)
           *reinterpret_cast<u32x4*>(bp + kF + 1024 * (hw + NW * i) + 16 * lane) = r.f[i];
+      // the output's factor scale e^G of this wave's rows, the Q scale taken back
+      if constexpr (OUT) {
+        if (lane / (64 / UPR) % NW == hw)
+          *reinterpret_cast<float*>(bp + kO + 4 * lane) =
+              a.scale * __expf(r.g) * __int_as_float((qe - 14) << 23);
+      }
       if (hw == NW - 1) {
         const int L = min(kChunk, e - (s + j * kChunk));
         const float GL = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.g), L - 1));
@@ -287,7 +337,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
         float* gp = reinterpret_cast<float*>(bp + kG);
         gp[lane] = eg;
         gp[64 + lane] = __expf(GL - r.g);
-        if (lane == L - 1) gp[128] = eg;
+        if (lane == L - 1) *reinterpret_cast<float*>(bp + kE) = eg;
       }
     };
     if (nc > 0) {
@@ -343,7 +393,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
   // KLayout; the rest of every address is an immediate)
   const int m4 = r16 >> 2, q4 = r16 & 3;
   int ka_off[KB], tr_off[ST / 2], q_off[KB], v_off[2], f_off = kF + 16 * lane,
-      g_off = kG + 32 * grp, e_off = kG + 4 * r16;
+      g_off = kG + 32 * grp, e_off = kO + 4 * r16;
 #pragma unroll
   for (int b = 0; b < KB; ++b) {
     ka_off[b] = KL::off(rho_row(0, r16), 4 * b + grp);
@@ -441,7 +491,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
         }
       }
     };
-    const float egl = *reinterpret_cast<const float*>(buf + (g_off - 32 * grp) + 512);
+    const float egl = *reinterpret_cast<const float*>(buf + (g_off - 32 * grp) + (kE - kG));
     read_blk(0);
     if constexpr (SAVE) {
       // the chunk's start state: hs[chunk][v-head] = S^T (bf16), row 32 w +
@@ -627,7 +677,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
 #pragma unroll
         for (int ti = 2 * (y - (NK - 2)); ti < 2 * (y - (NK - 2)) + 2; ++ti) {
 #pragma unroll
-          for (int x = 0; x < 2; ++x) O[x][ti] = (a.scale * ego[ti]) * O[x][ti];
+          for (int x = 0; x < 2; ++x) O[x][ti] = ego[ti] * O[x][ti];
         }
         kReads(14)
         kMix(8, 2)

@@ -74,9 +74,11 @@ extern "C" {
  * magnitude inside it.  The final state is within ~4e-4 relative Frobenius
  * of the exact recurrence at any length.  Without use_qk_l2norm the output's
  * q.S term is, for few short chains, a bf16 MFMA product (q as given, the
- * state rounded to bf16); with it, and for many or long chains, an fp16 one
- * (q as fp16); gdn_chunk_fwd_save gives the same o as gdn_chunk_fwd either
- * way.  Few long sequences (64 chunks and more) are run in segments, whose
+ * state rounded to bf16), and for many or long chains an fp16 one (the state
+ * as fp16, q times a power of two per group of rows, so that its own size does
+ * not matter); with use_qk_l2norm it is an fp16 one (the normalised q as
+ * fp16); gdn_chunk_fwd_save gives the same o as gdn_chunk_fwd either way.
+ * P = scale q.k e^(G_i - G_j) is rounded to fp16 in every form.  Few long sequences (64 chunks and more) are run in segments, whose
  * buffers (128 KiB per segment and v-head at K = V = 128) are part of the
  * workspace.
  */

@@ -186,3 +186,20 @@ def test_noalloc_takes_what_fits_without_segments(rocm_device):
     assert rc == 0, lib.gdn_last_error().decode()
     assert (s2 - s).norm() <= 1e-3 * s.norm()
     assert (o2.float() - o.float()).norm() <= 1e-2 * o.float().norm()
+
+
+@pytest.mark.parametrize("what", ["state waves", "whole heads", "segments"])
+@pytest.mark.parametrize("shift", [-30, 20])
+def test_q_of_any_magnitude(rocm_device, what, shift):
+    """Without l2norm q counts as the caller's bf16, also far outside fp16's range (2^-14 to
+    65504): q 2^shift with scale 2^-shift, both exact, gives the same bits in every form."""
+    from avelang_amd import chunk_gated_delta_rule
+    B = -(-_cus(rocm_device) // 4)
+    shape = {"state waves": (1, 200, 2, 4), "whole heads": (B, 130, 2, 4),
+             "segments": (1, 4200, 1, 2)}[what]
+    t = W.make(*shape, 128, 128, seed=13, h0_scale=0.05, decay=0.01).torch(rocm_device)
+    o, o2 = (chunk_gated_delta_rule(t["q"] * 2.0 ** n, t["k"], t["v"], t["g"], t["beta"],
+                                    scale=128 ** -0.5 * 2.0 ** -n,
+                                    initial_state=t["initial_state"])[0] for n in (0, shift))
+    torch.cuda.synchronize()
+    assert bool(o.any()) and torch.equal(o, o2)
