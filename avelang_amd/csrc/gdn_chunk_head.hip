@@ -33,6 +33,12 @@
 // (normalising here instead made the helper the longer wave: 2.9 us per
 // chunk) -- V as fp16, and the chunk's gate factors.
 //
+// Registers: K = V = 128 takes 256 VGPRs, unspilled but for saves and o in one
+// launch.  K = 128 with V = 64 (four waves, 106 KB of LDS: alone on its compute
+// unit) takes up to 422 with the AGPRs.  K = V = 64 (74 KB) takes 244 with COPY
+// and 275 without, where a compute unit then holds one workgroup instead of
+// two (held to 256 it would spill 32).
+//
 // Segments (few long chains): a chunk maps the state by S -> M_c S + B_c, so a
 // sequence is cut into segments whose own contributions B (from a zero state)
 // and transfer matrices M (from I, with V = 0) are formed in parallel (XFER),
@@ -390,17 +396,14 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
     }
   }
   // per-lane byte offsets of the fragment reads in the step's buffer (see
-  // KLayout; the rest of every address is an immediate)
+  // KLayout; the rest of every address is an immediate, but for the k-block,
+  // which a row's unit permutation takes as an XOR of byte address bits 6 and
+  // up: one instruction per read block where an offset per k-block held nine
+  // registers more, and 16 were spilled)
   const int m4 = r16 >> 2, q4 = r16 & 3;
-  int ka_off[KB], tr_off[ST / 2], q_off[KB], v_off[2], f_off = kF + 16 * lane,
+  int ka_off = KL::off(rho_row(0, r16), grp), tr_off = KL::off(8 * grp + m4, q4),
+      q_off = kQ + (COPY ? 16 * lane : qrow_off<K>(r16, grp)), v_off[2], f_off = kF + 16 * lane,
       g_off = kG + 32 * grp, e_off = kO + 4 * r16;
-#pragma unroll
-  for (int b = 0; b < KB; ++b) {
-    ka_off[b] = KL::off(rho_row(0, r16), 4 * b + grp);
-    q_off[b] = COPY ? kQ + 1024 * b + 16 * lane : kQ + qrow_off<K>(r16, 4 * b + grp);
-  }
-#pragma unroll
-  for (int u = 0; u < ST / 2; ++u) tr_off[u] = KL::off(8 * grp + m4, 4 * u + q4);
 #pragma unroll
   for (int x = 0; x < 2; ++x)
     v_off[x] = kV + (8 * grp + m4) * 2 * V + 32 * ((2 * w + x) ^ vrow_swz<V>(8 * grp + m4)) + 8 * q4;
@@ -480,13 +483,13 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
 #pragma unroll
       for (int y = 0; y < 4; ++y) {
         if (i < KB) {
-          f[y] = lds8(ka_off[i] + KL::RS * (32 * (y >> 1) + 4 * (y & 1)));
+          f[y] = lds8((ka_off ^ 64 * i) + KL::RS * (32 * (y >> 1) + 4 * (y & 1)));
         } else if (i < NB) {
-          f[y] = lds8(q_off[i - KB] + y * (COPY ? KB * 1024 : 32 * K));
+          f[y] = lds8(COPY ? q_off + 1024 * (i - KB) + y * KB * 1024 : (q_off ^ 64 * (i - KB)) + y * 32 * K);
         } else if (i < NB + NK) {
           // element i of lane (m, grp): K[32 b + 8 grp + i][rho(16 t + m)]
           const int b = (i - NB) / (ST / 4), t = 4 * ((i - NB) % (ST / 4)) + y;
-          const int p = tr_off[t >> 1] + KL::RS * 32 * b + 8 * (t & 1);
+          const int p = (tr_off ^ 64 * (t >> 1)) + KL::RS * 32 * b + 8 * (t & 1);
           f[y] = cat8(ldst(p), ldst(p + KL::RS * 4));
         }
       }
@@ -715,13 +718,9 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
     lds_barrier();
     // the next step's buffer
     const int d = (j & 1) ? -kBufStep : kBufStep;
-#pragma unroll
-    for (int b = 0; b < KB; ++b) {
-      ka_off[b] += d;
-      q_off[b] += d;
-    }
-#pragma unroll
-    for (int u = 0; u < ST / 2; ++u) tr_off[u] += d;
+    ka_off += d;
+    q_off += d;
+    tr_off += d;
     v_off[0] += d;
     v_off[1] += d;
     f_off += d;
@@ -902,8 +901,8 @@ void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, 
     hipLaunchKernelGGL((chunk_combine_kernel<K>), dim3(tiles, seqs), dim3(4 * K), 0, st, a, ws);
   }
   // A training forward in segments forms saves and o in two launches: with both
-  // the kernel is 32 registers over its 256, and each reload waits until the
-  // step's stores are in memory.  T = 8192, 32 heads (160 workgroups): 177 us in
+  // the kernel is 15 to 17 registers over its 256 (32 when this was measured),
+  // and each reload waits until the step's stores are in memory.  T = 8192, 32 heads (160 workgroups): 177 us in
   // one launch, 98 + 70 in two.  Whole sequences (many workgroups, HBM-bound)
   // keep one launch and read the operands once.
   if constexpr (SAVE && OUT && K == 128) {

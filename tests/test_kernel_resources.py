@@ -115,3 +115,13 @@ def test_the_check_catches_scratch_and_spills():
     assert _violations({"_ZN3gdn16recurrent_kernelI": dict(ok, vgpr_spill_count=4)}) == []
     assert len(_violations({"_ZN3gdn19chunk_rev_sw_kernelI": dict(ok, private_segment_fixed_size=16)})) == 1
     assert len(_violations({"_ZN3gdn17chunk_grad_kernelI": dict(ok, vgpr_spill_count=2)})) == 1
+
+
+def test_whole_head_forms_spill_nothing(kernels):
+    """chunk_head_kernel<K, V, COPY, SAVE, OUT, XFER> keeps its state in registers in every form
+    but saves and o in one launch (K = V = 128 then spills a few; its waits are the compiler's)."""
+    forms = {n: m for n, m in kernels.items() if "chunk_head_kernel" in n}
+    assert forms
+    bad = [n for n, m in forms.items()
+           if "Lb1ELb1ELb0EEE" not in n and (m["private_segment_fixed_size"] or m["vgpr_spill_count"])]
+    assert not bad, bad
