@@ -62,6 +62,7 @@ struct HeadArgs {
   int N, T, total, Hqk, Hv;
   float scale;
   int seg;      // chunks per segment (0: whole sequences)
+  bool ht_in_segs;   // (segments, ht == h0) a cut sequence's final state goes to ws.segs
   TokenStride ts;
 };
 
@@ -765,6 +766,9 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
     return;
   }
   float* out = sp.last && a.ht ? a.ht + ((size_t)n * a.Hv + h) * kv : nullptr;
+  // in place the first segment's workgroup may yet read the state here: it
+  // goes over the one that this workgroup, and no other, started from
+  if (out && a.ht_in_segs && sp.first > 0) out = ws.segs + ((size_t)(sg - 1) * a.Hv + h) * kv;
   if constexpr (XFER) out = ws.segs + ((size_t)sg * a.Hv + h) * kv;
   if (out) {
 #pragma unroll
@@ -880,12 +884,27 @@ __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkW
   }
 }
 
+// ht_in_segs: the cut sequences' final states from where chunk_head_kernel left
+// them.  One workgroup per v-head and, as far as the grid goes, sequence.
+__global__ __launch_bounds__(256) void chunk_final_state_kernel(HeadArgs a, ChunkWs ws, int kv) {
+  const int h = blockIdx.x;
+  for (int n = blockIdx.y; n < a.N; n += gridDim.y) {
+    int first, count;
+    seg_range(n, a.seg, a.cu, a.T, ws, first, count);
+    if (count < 2) continue;
+    const float* src = ws.segs + ((size_t)(first + count - 2) * a.Hv + h) * kv;
+    float* dst = a.ht + ((size_t)n * a.Hv + h) * kv;
+    for (int i = threadIdx.x; i < kv; i += 256) dst[i] = src[i];
+  }
+}
+
 template <int K, bool SAVE, bool OUT>
 void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, const float* h0,
                        float* ht, uint16_t* o, const int32_t* cu, int N, int T, int total, int Hqk,
                        int Hv, int V, float scale, bool l2, TokenStride ts, const WsPlan& p,
                        const ChunkWs& ws, hipStream_t st) {
-  const HeadArgs a{q, k, v, h0, ht, o, cu, N, T, total, Hqk, Hv, scale, p.seg, ts};
+  const bool ht_in_segs = p.seg && p.nfull > 0 && ht && ht == h0;
+  const HeadArgs a{q, k, v, h0, ht, o, cu, N, T, total, Hqk, Hv, scale, p.seg, ht_in_segs, ts};
   const unsigned grid = (unsigned)((p.seg ? p.nseg : N) * Hv);
   auto go = [&](auto kern, unsigned g) {
     hipLaunchKernelGGL(kern, dim3(g), dim3(4 * V), 0, st, a, ws);
@@ -905,22 +924,28 @@ void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, 
   // and each reload waits until the step's stores are in memory.  T = 8192, 32 heads (160 workgroups): 177 us in
   // one launch, 98 + 70 in two.  Whole sequences (many workgroups, HBM-bound)
   // keep one launch and read the operands once.
+  bool apart = false;
   if constexpr (SAVE && OUT && K == 128) {
-    if (p.seg && V == 128) {
+    apart = p.seg && V == 128;
+    if (apart) {
       if (l2) go(chunk_head_kernel<K, 128, true, true, false, false>, grid);
       else go(chunk_head_kernel<K, 128, false, true, false, false>, grid);
       if (l2) go(chunk_head_kernel<K, 128, true, false, true, false>, grid);
       else go(chunk_head_kernel<K, 128, false, false, true, false>, grid);
-      return;
     }
   }
-  if (V == 128) {
-    if (l2) go(chunk_head_kernel<K, 128, true, SAVE, OUT, false>, grid);
-    else go(chunk_head_kernel<K, 128, false, SAVE, OUT, false>, grid);
-  } else {
-    if (l2) go(chunk_head_kernel<K, 64, true, SAVE, OUT, false>, grid);
-    else go(chunk_head_kernel<K, 64, false, SAVE, OUT, false>, grid);
+  if (!apart) {
+    if (V == 128) {
+      if (l2) go(chunk_head_kernel<K, 128, true, SAVE, OUT, false>, grid);
+      else go(chunk_head_kernel<K, 128, false, SAVE, OUT, false>, grid);
+    } else {
+      if (l2) go(chunk_head_kernel<K, 64, true, SAVE, OUT, false>, grid);
+      else go(chunk_head_kernel<K, 64, false, SAVE, OUT, false>, grid);
+    }
   }
+  if (ht_in_segs)
+    hipLaunchKernelGGL(chunk_final_state_kernel, dim3(Hv, std::min(N, 1024)), dim3(256), 0, st, a,
+                       ws, K * V);
 }
 
 #define GDN_HEAD_INST(K_, SAVE_, OUT_)                                                       \

@@ -203,3 +203,40 @@ def test_q_of_any_magnitude(rocm_device, what, shift):
                                     initial_state=t["initial_state"])[0] for n in (0, shift))
     torch.cuda.synchronize()
     assert bool(o.any()) and torch.equal(o, o2)
+
+
+def _in_place_cases(dev):
+    """(workload, l2) at segmented sizes: batched, and packed with cut and uncut sequences, the
+    last segments of one chunk and of more."""
+    yield W.make(2, 4096 + 1, 1, 2, 128, 128, seed=21, decay=0.01, h0_scale=0.05), False
+    yield W.make(1, 6200, 2, 4, 64, 64, seed=22, decay=0.002, h0_scale=0.05, l2norm=False), True
+    for lens in ([9000, 0, 1, 7000], [130, 8200, 5000]):
+        cu = _cu(lens)
+        yield W.make(1, int(cu[-1]), 1, 2, 128, 128, seed=23, cu_seqlens=cu, decay=0.01,
+                     h0_scale=0.05, l2norm=False), True
+
+
+@pytest.mark.parametrize("op", ["plain", "gated", "rows"])
+def test_final_state_in_place_of_the_initial_one(rocm_device, op):
+    from avelang_amd.gated_delta_rule import _chunk_fwd   # (with the gating, which the public form
+    for wl, l2 in _in_place_cases(rocm_device):   # gives no final_state, too)
+        t = wl.torch(rocm_device)
+        q, k, v = t["q"], t["k"], t["v"]
+        if op == "rows":   # column slices of one tensor, read in place
+            wide = torch.cat([x.flatten(2) for x in (q, k, v)], -1)
+            q, k, v = (x.reshape(y.shape) for x, y in zip(
+                wide.split([y[0, 0].numel() for y in (q, k, v)], -1), (q, k, v)))
+        g, beta, gate = t["g"], t["beta"], None
+        if op == "gated":
+            g, beta = g.to(torch.bfloat16), beta.to(torch.bfloat16)
+            zero = torch.zeros(v.shape[2], device=rocm_device)
+            gate = (zero - 4.0, zero, 1.0, 20.0)
+        res = []
+        for same in (False, True):
+            h0 = t["initial_state"].clone()
+            res.append(_chunk_fwd(q, k, v, g, beta, None, h0, True, t["cu_seqlens"], l2, gate=gate,
+                                  final_state=h0 if same else None))
+            assert not same or res[-1][1] is h0
+        torch.cuda.synchronize()
+        for x, y in zip(*res):
+            assert torch.equal(x, y), (op, wl.dims)
