@@ -928,8 +928,12 @@ void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, 
   if constexpr (SAVE && OUT && K == 128) {
     apart = p.seg && V == 128;
     if (apart) {
-      if (l2) go(chunk_head_kernel<K, 128, true, true, false, false>, grid);
-      else go(chunk_head_kernel<K, 128, false, true, false, false>, grid);
+      // (the saves leave ht alone: it may be h0, from which the outputs start)
+      HeadArgs saves = a;
+      saves.ht = nullptr;
+      const auto kern = l2 ? chunk_head_kernel<K, 128, true, true, false, false>
+                           : chunk_head_kernel<K, 128, false, true, false, false>;
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(4 * V), 0, st, saves, ws);
       if (l2) go(chunk_head_kernel<K, 128, true, false, true, false>, grid);
       else go(chunk_head_kernel<K, 128, false, false, true, false>, grid);
     }

@@ -216,7 +216,14 @@ def _in_place_cases(dev):
                      h0_scale=0.05, l2norm=False), True
 
 
-@pytest.mark.parametrize("op", ["plain", "gated", "rows"])
+def _save_workspace(wl, l2, dev):
+    from avelang_amd.gated_delta_rule import chunk_bwd_workspace_bytes
+    n = chunk_bwd_workspace_bytes(*(wl.dims[x] for x in ("B", "T", "Hqk", "Hv", "K", "V", "N")),
+                                  wl.cu_seqlens is not None, l2)
+    return torch.empty(n, dtype=torch.uint8, device=dev)
+
+
+@pytest.mark.parametrize("op", ["plain", "gated", "rows", "save"])
 def test_final_state_in_place_of_the_initial_one(rocm_device, op):
     from avelang_amd.gated_delta_rule import _chunk_fwd   # (with the gating, which the public form
     for wl, l2 in _in_place_cases(rocm_device):   # gives no final_state, too)
@@ -235,7 +242,9 @@ def test_final_state_in_place_of_the_initial_one(rocm_device, op):
         for same in (False, True):
             h0 = t["initial_state"].clone()
             res.append(_chunk_fwd(q, k, v, g, beta, None, h0, True, t["cu_seqlens"], l2, gate=gate,
-                                  final_state=h0 if same else None))
+                                  final_state=h0 if same else None,
+                                  save_workspace=_save_workspace(wl, l2, rocm_device)
+                                  if op == "save" else None))
             assert not same or res[-1][1] is h0
         torch.cuda.synchronize()
         for x, y in zip(*res):
