@@ -15,9 +15,9 @@ namespace gdn {
 struct ChunkWs {
   int32_t* off;     // [N+1] first global chunk of each sequence
   int32_t* soff;    // [N+1] first segment of each sequence (cu_seqlens and segments)
-  float* segs;      // [segments][Hv][K][V] a segment's own contribution to the state, then
+  float* segs;      // [full segments][Hv][K][V] a segment's own contribution to the state, then
                     // the state after it
-  u16x8* segm;      // [segments][Hv][hi, lo][K/16][K/32][64] a segment's transfer matrix M
+  u16x8* segm;      // [full segments][Hv][hi, lo][K/16][K/32][64] a segment's transfer matrix M
                     // as bf16 A-operand fragments, M = hi + lo (rows in rho order)
   int32_t* status;  // [1] 0, or the cu_seqlens violation the chunk table found
   float* gate;      // [NC][Hv][64]: G_i, the chunk-local cumulative log-decay
@@ -197,8 +197,8 @@ inline bool chain_reads_rows(bool bwd, bool l2, int N, int Hv, int V) {
 struct WsPlan {
   size_t off, status, gate, tfrag, pfrag, k16, q16, qn, kn, total;
   size_t soff, segs, segm;
-  // chunks per segment (0: none), segments of all sequences at most, and those
-  // among them that another follows
+  // chunks per segment (0: none), segments of all sequences at most, and the full
+  // ones among them, which another follows: these alone have buffers
   int seg, nseg, nfull;
   bool whole_head;   // the forward chain takes the whole-head form (gdn_chunk_head.hip)
   bool k16_copy, q16_copy;   // k16 / q16 planned (else the chains read the caller's rows)

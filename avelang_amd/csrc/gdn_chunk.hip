@@ -640,8 +640,8 @@ WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, 
     p.nfull = (int)(has_cu ? p.ncmax / p.seg : N * (per - 1));
     p.nseg = p.nfull + N;
     p.soff = take((size_t)(N + 1) * 4);
-    p.segs = take((size_t)p.nseg * Hv * K * V * 4);
-    p.segm = take((size_t)p.nseg * Hv * K * K * 4);
+    p.segs = take((size_t)p.nfull * Hv * K * V * 4);
+    p.segm = take((size_t)p.nfull * Hv * K * K * 4);
   }
   p.total = at;
   return p;

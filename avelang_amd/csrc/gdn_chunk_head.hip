@@ -69,7 +69,9 @@ struct HeadArgs {
 // Segments.  Sequence n's chunks are cut into segments of `seg` chunks (one
 // at least, also for an empty sequence); ws.soff[n] is its first segment's
 // global index with cu_seqlens (chunk_table_kernel), n times a constant
-// without.
+// without.  Every segment but a sequence's last is full; ws.segs and ws.segm
+// hold the full ones alone, which the n last segments before are left out of:
+// segment j of sequence n is full segment first + j - n.
 __device__ __forceinline__ void seg_range(int n, int seg, const int32_t* cu, int T,
                                           const ChunkWs& ws, int& first, int& count) {
   if (cu) {
@@ -82,7 +84,8 @@ __device__ __forceinline__ void seg_range(int n, int seg, const int32_t* cu, int
 }
 struct SegPos {
   int n;            // sequence, -1 past the last segment
-  int sg;           // global index of the segment
+  int full;         // index among the full segments (a last segment: one past the
+                    // full segment that it follows)
   int first;        // its sequence's chunk it starts at
   int c_begin, nc;  // global first chunk, chunks
   bool last;        // the sequence's last segment
@@ -95,8 +98,6 @@ __device__ __forceinline__ SegPos seg_pos(int i, bool full, int seg, const int32
   const int nct = (T + kChunk - 1) / kChunk;
   int j = 0, cnt = 1;
   if (seg) {
-    // (a sequence has one segment that is not full: full ones are counted by
-    // soff[n] - n)
     if (cu) {
       if (i >= ws.soff[N] - (full ? N : 0)) return SegPos{-1, 0, 0, 0, 0, true};
       int lo = 0, hi = N;   // the largest n whose first segment is i or before
@@ -111,8 +112,8 @@ __device__ __forceinline__ SegPos seg_pos(int i, bool full, int seg, const int32
     }
     int first;
     seg_range(r.n, seg, cu, T, ws, first, cnt);
-    r.sg = full ? i + r.n : i;
-    j = r.sg - first;
+    r.full = full ? i : i - r.n;
+    j = r.full - (first - r.n);
   }
   const int c0 = cu ? ws.off[r.n] : r.n * nct;
   const int c1 = cu ? ws.off[r.n + 1] : c0 + nct;
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
   // that another follows)
   const SegPos sp = seg_pos(bid / a.Hv, XFER, a.seg, a.cu, a.N, a.T, ws);
   if (sp.n < 0) return;
-  const int n = sp.n, sg = sp.sg;
+  const int n = sp.n, full = sp.full;
   int s, e;
   seq_bounds(a.cu, n, a.T, a.total, s, e);
   const int c_begin = sp.c_begin, nc = sp.nc;
@@ -382,7 +383,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
   // the state to start from: the caller's, or the state after the segment
   // before (chunk_combine_kernel)
   const float* init = a.h0 ? a.h0 + ((size_t)n * a.Hv + h) * kv : nullptr;
-  if (sp.first > 0) init = XFER ? nullptr : ws.segs + ((size_t)(sg - 1) * a.Hv + h) * kv;
+  if (sp.first > 0) init = XFER ? nullptr : ws.segs + ((size_t)(full - 1) * a.Hv + h) * kv;
   f32x4 S[2][ST];
 #pragma unroll
   for (int x = 0; x < 2; ++x) {
@@ -748,7 +749,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
     // transposed through this wave's share of the operand buffers
     constexpr int LD = 20;
     uint16_t* X = reinterpret_cast<uint16_t*>(buf + 4096 * w);
-    u16x8* dst = ws.segm + ((size_t)sg * a.Hv + h) * (2 * ST * KB * 64) + w * 64 + lane;
+    u16x8* dst = ws.segm + ((size_t)full * a.Hv + h) * (2 * ST * KB * 64) + w * 64 + lane;
 #pragma unroll
     for (int t = 0; t < ST; ++t) {
 #pragma unroll
@@ -768,8 +769,8 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
   float* out = sp.last && a.ht ? a.ht + ((size_t)n * a.Hv + h) * kv : nullptr;
   // in place the first segment's workgroup may yet read the state here: it
   // goes over the one that this workgroup, and no other, started from
-  if (out && a.ht_in_segs && sp.first > 0) out = ws.segs + ((size_t)(sg - 1) * a.Hv + h) * kv;
-  if constexpr (XFER) out = ws.segs + ((size_t)sg * a.Hv + h) * kv;
+  if (out && a.ht_in_segs && sp.first > 0) out = ws.segs + ((size_t)(full - 1) * a.Hv + h) * kv;
+  if constexpr (XFER) out = ws.segs + ((size_t)full * a.Hv + h) * kv;
   if (out) {
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
@@ -818,7 +819,7 @@ __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkW
         if (seen++ % (int)gridDim.y != (int)blockIdx.y) continue;
         const int n = __builtin_amdgcn_readfirstlane(base + 64 * word + __builtin_ctzll(left));
         seg_range(n, a.seg, a.cu, a.T, ws, first, count);
-        auto head = [&](int j) { return (size_t)(first + j) * a.Hv + h; };
+        auto head = [&](int j) { return (size_t)(first - n + j) * a.Hv + h; };
         auto load_m = [&](u16x8 (&m)[2][KB], int j) {
           const u16x8* p = ws.segm + head(j) * (2 * ST * KB * 64) + w * KB * 64 + lane;
 #pragma unroll
@@ -892,7 +893,7 @@ __global__ __launch_bounds__(256) void chunk_final_state_kernel(HeadArgs a, Chun
     int first, count;
     seg_range(n, a.seg, a.cu, a.T, ws, first, count);
     if (count < 2) continue;
-    const float* src = ws.segs + ((size_t)(first + count - 2) * a.Hv + h) * kv;
+    const float* src = ws.segs + ((size_t)(first - n + count - 2) * a.Hv + h) * kv;
     float* dst = a.ht + ((size_t)n * a.Hv + h) * kv;
     for (int i = threadIdx.x; i < kv; i += 256) dst[i] = src[i];
   }

@@ -78,8 +78,10 @@ extern "C" {
  * as fp16, q times a power of two per group of rows, so that its own size does
  * not matter); with use_qk_l2norm it is an fp16 one (the normalised q as
  * fp16); gdn_chunk_fwd_save gives the same o as gdn_chunk_fwd either way.
- * P = scale q.k e^(G_i - G_j) is rounded to fp16 in every form.  Few long sequences (64 chunks and more) are run in segments, whose
- * buffers (128 KiB per segment and v-head at K = V = 128) are part of the
+ * P = scale q.k e^(G_i - G_j) is rounded to fp16 in every form.  Few long
+ * sequences (64 chunks and more) are run in segments, and so are those of a
+ * packed batch that are far longer than its mean; their buffers (128 KiB per
+ * v-head at K = V = 128 and segment that another follows) are part of the
  * workspace.
  */
 int gdn_chunk_fwd(const void* q, const void* k, const void* v,

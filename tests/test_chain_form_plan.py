@@ -7,12 +7,12 @@ from avelang_amd import _native
 LIMIT = 32 << 20
 
 
-def _plain(T, Hqk, Hv, K, l2):
+def _plain(T, Hqk, Hv, K, l2, N=0):
     """Bytes without segments: per (chunk, v-head) G and the Tb, P fragments; with l2norm the
     fp16 K, Q copies per (chunk, qk-head); each buffer rounded up to 256, the two tables too."""
-    n = -(-T // 64)
+    n = (T + 63 * N) // 64 if N else -(-T // 64)   # (N packed sequences)
     up = lambda x: -(-x // 256) * 256  # noqa: E731
-    return (512 + up(n * Hv * 256) + 2 * up(n * Hv * 6144) +
+    return (up(4 * N + 4) + 256 + up(n * Hv * 256) + 2 * up(n * Hv * 6144) +
             (2 * up(n * Hqk * 64 * K * 2) if l2 else 0))
 
 
@@ -34,3 +34,16 @@ def test_workspace_with_segments(Hqk, Hv, K, l2):
             assert lib.gdn_chunk_fwd_noalloc(*fake, 1, T, Hqk, Hv, K, K, 1, 0.1, l2, None) == -4
             assert str(plain) in lib.gdn_last_error().decode()
     assert grown > 0   # some of them do run in segments
+
+
+@pytest.mark.parametrize("K", [64, 128])
+@pytest.mark.parametrize("N", [16, 64, 256, 1024, 4096])
+def test_packed_workspace_has_no_room_for_uncut_sequences(N, K):
+    """Buffers for the segments that another follows (64 chunks and more each), not for every
+    sequence's last one: many short prompts do not pay for a few long ones they might hold."""
+    lib = _native.lib()
+    for T in (16384, 262144):
+        plain = _plain(T, 16, 32, K, 0, N)
+        cut = (T + 63 * N) // 64 // 64
+        got = lib.gdn_chunk_workspace_bytes(1, T, 16, 32, K, K, N, 1, 0)
+        assert plain <= got <= plain + cut * 32 * 2 * K * K * 4 + 4 * (N + 1) + 3 * 256
