@@ -17,8 +17,8 @@ struct ChunkWs {
   int32_t* soff;    // [N+1] first segment of each sequence (cu_seqlens and segments)
   float* segs;      // [full segments][Hv][K][V] a segment's own contribution to the state, then
                     // the state after it
-  u16x8* segm;      // [full segments][Hv][hi, lo][K/16][K/32][64] a segment's transfer matrix M
-                    // as bf16 A-operand fragments, M = hi + lo (rows in rho order)
+  u16x8* segm;      // [full segments][Hv][part][K/16][K/32][64] a segment's transfer matrix M
+                    // as bf16 A-operand fragments of its three parts (rows in rho order)
   int32_t* status;  // [1] 0, or the cu_seqlens violation the chunk table found
   float* gate;      // [NC][Hv][64]: G_i, the chunk-local cumulative log-decay
   u16x8* tfrag;     // [NC][Hv][6 slots][64 lanes] fp16 A-operand fragments of Tb,

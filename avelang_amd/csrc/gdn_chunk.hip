@@ -562,8 +562,9 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // The segment count fills the GPU once with the first pass's workgroups (two
 // per segment but the last, one per compute unit, 64-wide heads' two; at
 // W = 32, T = 8192 5 segments 138 us, 4 155, 6 159, 8 152), and balances the
-// passes over a segment (~3.5 us per chunk) against the serial combine (~1.1
-// us per segment; W = 4, T = 20011 25 segments 97 us, 16 106, 12 120).
+// passes over a segment (~3.5 us per chunk) against the serial combine (~1.4
+// us per segment; W = 4, T = 20011 25 segments 105 us, at 1.1 us 97, and 16
+// 106, 12 120).
 // With cu_seqlens nct is the mean; an unsegmented form still cuts a sequence
 // much longer than that, which would otherwise run on its own.
 static void chain_form(long long ncmax, long long nctotal, int N, int Hv, int K, int V,
@@ -641,7 +642,7 @@ WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, 
     p.nseg = p.nfull + N;
     p.soff = take((size_t)(N + 1) * 4);
     p.segs = take((size_t)p.nfull * Hv * K * V * 4);
-    p.segm = take((size_t)p.nfull * Hv * K * K * 4);
+    p.segm = take((size_t)p.nfull * Hv * K * K * 6);
   }
   p.total = at;
   return p;

@@ -745,23 +745,27 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
     }
   }
   if (mpart) {
-    // M = hi + lo (bf16) as the combine's A fragments (row tile t, k-block w),
-    // transposed through this wave's share of the operand buffers
+    // M as three bf16 parts (split3_bf4), each as the combine's A fragments
+    // (row tile t, k-block w), transposed through this wave's share of the
+    // operand buffers
     constexpr int LD = 20;
+    static_assert(3 * 32 * LD * 2 <= 4096 && 4096 * NW <= 2 * kBufStep, "a wave's share");
     uint16_t* X = reinterpret_cast<uint16_t*>(buf + 4096 * w);
-    u16x8* dst = ws.segm + ((size_t)full * a.Hv + h) * (2 * ST * KB * 64) + w * 64 + lane;
+    u16x8* dst = ws.segm + ((size_t)full * a.Hv + h) * (3 * ST * KB * 64) + w * 64 + lane;
 #pragma unroll
     for (int t = 0; t < ST; ++t) {
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
-        u16x4 hi, lo;
-        split_bf4(S[x][t], hi, lo);
-        *reinterpret_cast<u16x4*>(X + (16 * x + r16) * LD + 4 * grp) = hi;
-        *reinterpret_cast<u16x4*>(X + (32 + 16 * x + r16) * LD + 4 * grp) = lo;
+        u16x4 part[3];
+        split3_bf4(S[x][t], part);
+#pragma unroll
+        for (int y = 0; y < 3; ++y)
+          *reinterpret_cast<u16x4*>(X + (32 * y + 16 * x + r16) * LD + 4 * grp) = part[y];
       }
       __builtin_amdgcn_wave_barrier();
-      dst[t * KB * 64] = lds_colfrag(X, LD, 0, 0, lane);
-      dst[(ST + t) * KB * 64] = lds_colfrag(X, LD, 32, 0, lane);
+#pragma unroll
+      for (int y = 0; y < 3; ++y)
+        dst[(y * ST + t) * KB * 64] = lds_colfrag(X, LD, 32 * y, 0, lane);
       __builtin_amdgcn_wave_barrier();
     }
     return;
@@ -788,15 +792,18 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
 // contributions B (ws.segs; the first segment's is already the state after
 // it) and transfer matrices M (ws.segm), in place of B.  One workgroup per
 // (sequence, v-head, 16 value columns), wave w the state rows rho(16 w + m).
-// The product takes bf16 hi + lo halves of both operands (three MFMA passes,
-// ~2^-17 relative, far inside the ~4e-4 of the chains): 21.7 us for 20 segments
-// of 4 heads, ~1.1 us each, where fp32 MFMA took 42 and waited on the matrix
-// pipe; the state passes between the waves through LDS, and a
-// segment's M fragments are requested two segments ahead.
+// The state keeps its fp32: both operands of the product are split into three
+// bf16 parts, which hold all 24 bits (split3_bf4), and the six products of
+// 2^-17 and up are taken (M = I, a stretch of g = beta = 0, leaves every bit
+// of the state).  ~1.4 us per segment (T = 20011 of 4 heads, 25 segments:
+// 104.8 us per prefill; 97.0 with two parts and three products, which moved
+// the state by up to 2^-17 per segment).
+// The state passes between the waves through LDS, and a segment's M fragments
+// are requested two segments ahead.
 template <int K>
 __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkWs ws) {
   constexpr int ST = K / 16, KB = K / 32;   // row tiles (waves), k-blocks
-  __shared__ __attribute__((aligned(16))) u16x4 St[2][2][ST][64];   // [parity][hi, lo]
+  __shared__ __attribute__((aligned(16))) u16x8 St[2][3][KB][64];   // [parity][part]
   const int h = blockIdx.x % a.Hv, vt = blockIdx.x / a.Hv;
   const int lane = threadIdx.x % 64;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -820,12 +827,12 @@ __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkW
         const int n = __builtin_amdgcn_readfirstlane(base + 64 * word + __builtin_ctzll(left));
         seg_range(n, a.seg, a.cu, a.T, ws, first, count);
         auto head = [&](int j) { return (size_t)(first - n + j) * a.Hv + h; };
-        auto load_m = [&](u16x8 (&m)[2][KB], int j) {
-          const u16x8* p = ws.segm + head(j) * (2 * ST * KB * 64) + w * KB * 64 + lane;
+        auto load_m = [&](u16x8 (&m)[3][KB], int j) {
+          const u16x8* p = ws.segm + head(j) * (3 * ST * KB * 64) + w * KB * 64 + lane;
 #pragma unroll
-          for (int b = 0; b < KB; ++b) {
-            m[0][b] = p[b * 64];
-            m[1][b] = p[(ST * KB + b) * 64];
+          for (int y = 0; y < 3; ++y) {
+#pragma unroll
+            for (int b = 0; b < KB; ++b) m[y][b] = p[(y * ST * KB + b) * 64];
           }
         };
         // this wave's state tile: lane (r16, grp), element r = row rho(16 w + 4 grp
@@ -838,14 +845,15 @@ __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkW
           return f32x4{p[0], p[K], p[2 * K], p[3 * K]};
         };
         auto publish = [&](f32x4 x, int par) {
-          u16x4 hi, lo;
-          split_bf4(x, hi, lo);
-          St[par][0][w][lane] = hi;
-          St[par][1][w][lane] = lo;
+          u16x4 part[3];
+          split3_bf4(x, part);
+#pragma unroll
+          for (int y = 0; y < 3; ++y)   // (a B fragment: tile w's half of k-block w / 2)
+            reinterpret_cast<u16x4*>(&St[par][y][w >> 1][lane])[w & 1] = part[y];
           lds_barrier();
         };
         // segment j's M fragments and B tile in set j % 3
-        u16x8 m[3][2][KB];
+        u16x8 m[3][3][KB];
         f32x4 bt[3];
         load_m(m[1], 1);
         bt[1] = load_b(1);
@@ -857,21 +865,25 @@ __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkW
           const int jn = min(j + 2, count - 2);
           load_m(m[(c + 2) % 3], jn);
           bt[(c + 2) % 3] = load_b(jn);
-          f32x4 acc = bt[c], acc1 = zero4(), acc2 = zero4();
+          f32x4 acc[3][3];   // [M part][state part], the largest six
 #pragma unroll
           for (int b = 0; b < KB; ++b) {
             const auto& sp = St[(j + 1) & 1];
-            const u16x8 hi = cat8(sp[0][2 * b][lane], sp[0][2 * b + 1][lane]);
-            const u16x8 lo = cat8(sp[1][2 * b][lane], sp[1][2 * b + 1][lane]);
-            acc = mfma16(m[c][0][b], hi, acc);
-            acc1 = mfma16(m[c][0][b], lo, acc1);
-            acc2 = mfma16(m[c][1][b], hi, acc2);
+#pragma unroll
+            for (int z = 0; z < 3; ++z) {
+              const u16x8 part = sp[z][b][lane];
+#pragma unroll
+              for (int y = 0; y < 3 - z; ++y)
+                acc[y][z] = mfma16(m[c][y][b], part,
+                                   b ? acc[y][z] : (y || z ? zero4() : bt[c]));
+            }
           }
-          acc = acc + (acc1 + acc2);
+          const f32x4 sum = acc[0][0] + ((acc[0][1] + acc[1][0]) +
+                                         ((acc[0][2] + acc[2][0]) + acc[1][1]));
           float* o = tile_at(j);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) o[(size_t)r * K] = acc[r];
-          publish(acc, j & 1);
+          for (int r = 0; r < 4; ++r) o[(size_t)r * K] = sum[r];
+          publish(sum, j & 1);
         };
         for (int j = 1; j < count - 1;) {
           step(j++, std::integral_constant<int, 1>{});

@@ -249,3 +249,18 @@ def test_final_state_in_place_of_the_initial_one(rocm_device, op):
         torch.cuda.synchronize()
         for x, y in zip(*res):
             assert torch.equal(x, y), (op, wl.dims)
+
+
+@pytest.mark.parametrize("what", ["state waves", "whole heads", "segments", "segments, 64"])
+def test_padding_leaves_the_state(rocm_device, what):
+    """Tokens of g = beta = 0 leave every bit of the fp32 state, in every form."""
+    from avelang_amd import chunk_gated_delta_rule
+    B = -(-_cus(rocm_device) // 4)
+    B, T, Hv, D = {"state waves": (1, 200, 4, 128), "whole heads": (B, 130, 4, 128),
+                   "segments": (1, 4200, 2, 128), "segments, 64": (2, 5000, 2, 64)}[what]
+    t = W.make(B, T, 1, Hv, D, D, seed=14, h0_scale=1.0).torch(rocm_device)
+    zero = torch.zeros_like(t["g"])
+    _, ht = chunk_gated_delta_rule(t["q"], t["k"], t["v"], zero, zero, output_final_state=True,
+                                   initial_state=t["initial_state"])
+    torch.cuda.synchronize()
+    assert torch.equal(ht, t["initial_state"])
