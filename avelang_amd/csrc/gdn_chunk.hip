@@ -553,12 +553,21 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 //    sequences x 32 heads 2346 -> 1500; at W = 64 it loses (128 -> 159).  With
 //    64-wide heads from W = 256 on (143 -> 107; at 128 64 -> 72);
 //  - in segments for few long chains, whose segments' two passes run in
-//    parallel: W = 4, T = 4096 62 -> 54, 16384 219 -> 88; W = 8, 8192
-//    120 -> 72; W = 16, 8192 127 -> 94; W = 32, 8192 143 -> 138 (other inputs
-//    each call: 177 -> 150), 16384 390 -> 273, 65536 1593 -> 1061; W = 64,
-//    32768 1077 -> 963; at T = 2048 it loses everywhere (W = 4 36 -> 43), at
-//    W = 16, T = 4096 it is even.
-//    64-wide heads: W = 16, 4096 58 -> 44; W = 32, 8192 101 -> 86.
+//    parallel (other inputs each call): W = 4, T = 8192 119 -> 77, 20000
+//    268 -> 112; W = 8, 8192 124 -> 86; W = 16, 8192 131 -> 105; W = 32, 8192
+//    179 -> 160, 16384 400 -> 296, 65536 1593 -> 1030; W = 64, 16384 537 -> 492;
+//    with l2norm 5 to 15 % less of a gain.  At T = 4096 it wins without l2norm
+//    and loses with it (W = 8 69.4 -> 66.1, 64.1 -> 66.1; even at 68 chunks), at
+//    W = 16 it is even, at T = 2048 it loses everywhere.
+//    64-wide heads: W = 4, 4096 49 -> 42; W = 32, 8192 106 -> 93.
+//  - with the backward's saves, in segments a launch of their own, later:
+//    training forward W = 4, 4096 72 -> 81, 8192 128 -> 101; W = 16, 8192 165
+//    either way; W = 32, 8192 284 either way, its recomputing backward 600 ->
+//    627 and with l2norm 654 -> 669, 16384 571 -> 521 and 1179 either way.
+//    (W = 64, 16384 1093 -> 909, W = 128, 4096 unsegmented 577 -> 468: the
+//    forward that saves is taken at its best, recomputing there is 3 to 4 %
+//    slower, 2118 -> 2211 and 1110 -> 1146.)  64-wide heads win from the plain
+//    forward's line on.
 // The segment count fills the GPU once with the first pass's workgroups (two
 // per segment but the last, one per compute unit, 64-wide heads' two; at
 // W = 32, T = 8192 5 segments 138 us, 4 155, 6 159, 8 152), and balances the
@@ -568,14 +577,16 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // With cu_seqlens nct is the mean; an unsegmented form still cuts a sequence
 // much longer than that, which would otherwise run on its own.
 static void chain_form(long long ncmax, long long nctotal, int N, int Hv, int K, int V,
-                       bool has_cu, bool segments, WsPlan& p) {
+                       bool has_cu, bool segments, bool saving, WsPlan& p) {
   p.seg = 0;
   p.whole_head = false;
   if (N <= 0 || ncmax <= 0) return;
   const long long W = (long long)N * Hv, cus = device_cus();
   const long long nct = std::max(1LL, ncmax / N);
   const bool square = K == V && segments;
-  if (square && 2 * W <= cus && nct >= (W <= 8 ? 64 : std::max(72LL, 4 * W))) {
+  const long long least = W > 8 ? std::max(72LL, 4 * W) : K == 128 ? 68 : 64;
+  const long long least_saving = K == 128 ? std::max(96LL, std::min(8 * W, 256LL)) : 0;
+  if (square && 2 * W <= cus && nct >= (saving ? std::max(least, least_saving) : least)) {
     const double fill = K == 128 ? (double)cus / (2 * W) + 1 : (double)cus / W;
     const double ns = std::min(fill, 1.5 * std::sqrt((double)nct));
     p.seg = (int)std::ceil(nct / ns);
@@ -595,13 +606,7 @@ WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, 
   const long long total = (long long)B * T;
   p.ncmax = has_cu ? (total + 63LL * N) / 64 : (long long)B * ((T + 63) / 64);
   const size_t nch = (size_t)p.ncmax * Hv;   // (chunk, v-head) pairs
-  if (bwd) {   // a training forward takes the plain forward's form, so that o is the same
-    const WsPlan f = plan_ws(B, T, Hqk, Hv, K, V, N, has_cu, l2, false);
-    p.whole_head = f.whole_head;
-    p.seg = f.seg;
-  } else {
-    chain_form(p.ncmax, (total + 63) / 64, N, Hv, K, V, has_cu, segments, p);
-  }
+  chain_form(p.ncmax, (total + 63) / 64, N, Hv, K, V, has_cu, segments, bwd, p);
   size_t at = 0;
   auto take = [&](size_t bytes) {
     const size_t here = at;

@@ -277,7 +277,8 @@ def chunk_gated_delta_rule_fwd_save(
 ):
     """Training forward (gdn_chunk_fwd_save): ``(o, final_state, workspace)``.
 
-    ``o`` and ``final_state`` equal ``chunk_gated_delta_rule``'s; the
+    ``o`` and ``final_state`` equal ``chunk_gated_delta_rule``'s (to rounding
+    where only that one, of a long sequence, runs in segments); the
     returned workspace (``chunk_bwd_workspace_bytes`` bytes) holds what
     ``chunk_gated_delta_rule_bwd(..., workspace=ws, saved=True)`` needs for
     these same inputs.

@@ -77,7 +77,8 @@ extern "C" {
  * state rounded to bf16), and for many or long chains an fp16 one (the state
  * as fp16, q times a power of two per group of rows, so that its own size does
  * not matter); with use_qk_l2norm it is an fp16 one (the normalised q as
- * fp16); gdn_chunk_fwd_save gives the same o as gdn_chunk_fwd either way.
+ * fp16); gdn_chunk_fwd_save gives the same o as gdn_chunk_fwd but where only
+ * the latter runs in segments (see there).
  * P = scale q.k e^(G_i - G_j) is rounded to fp16 in every form.  Few long
  * sequences (64 chunks and more) are run in segments, and so are those of a
  * packed batch that are far longer than its mean; their buffers (160 KiB per
@@ -133,7 +134,9 @@ int gdn_chunk_fwd_noalloc(const void* q, const void* k, const void* v,
                           void* stream);
 
 /*
- * Training forward: gdn_chunk_fwd's results (o, ht) plus, in `workspace`
+ * Training forward: gdn_chunk_fwd's results (o, ht; bit for bit, but to
+ * rounding for long sequences that only the plain forward, which has no saves
+ * to make, cuts into segments) plus, in `workspace`
  * (at least gdn_chunk_bwd_workspace_bytes(...)), everything gdn_chunk_bwd
  * needs, so that a later gdn_chunk_bwd(..., saved = 1, same workspace) on
  * the same inputs skips its forward recomputation.  The forward half of an

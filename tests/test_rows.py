@@ -101,7 +101,7 @@ def _gates(B, T, Hv, dev, gated):
     (1, 130, 2, 4, 128, 128), (2, 65, 1, 2, 64, 64), (1, 77, 2, 2, 128, 64),   # state-wave form
     (16, 70, 2, 8, 128, 128),                    # two tiles per workgroup
     (64, 70, 2, 4, 128, 128), (64, 3, 4, 4, 64, 128),                          # whole heads
-    (1, 4170, 1, 2, 128, 128)])                  # segments
+    (1, 4170, 1, 2, 128, 128), (1, 4353, 1, 2, 128, 128)])                     # segments
 def test_prefill(rocm_device, B, T, Hqk, Hv, K, V, l2):
     from avelang_amd import chunk_gated_delta_rule, chunk_gated_delta_rule_gated
     qkv = _slices(B, T, Hqk, Hv, K, V, pad=16, device=rocm_device)
