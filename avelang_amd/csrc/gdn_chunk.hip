@@ -568,9 +568,11 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 //    forward that saves is taken at its best, recomputing there is 3 to 4 %
 //    slower, 2118 -> 2211 and 1110 -> 1146.)  64-wide heads win from the plain
 //    forward's line on.
-// The segment count fills the GPU once with the first pass's workgroups (two
-// per segment but the last, one per compute unit, 64-wide heads' two; at
-// W = 32, T = 8192 5 segments 138 us, 4 155, 6 159, 8 152), and balances the
+// The segment count fills the GPU once, and no more, with the first pass's
+// workgroups (two per segment, the first and last 1 and 0: W (2 ns - 3), one
+// per compute unit, 64-wide heads' two; at W = 32, T = 8192 5 segments 138 us,
+// 4 155, 6 159, 8 152; a few workgroups over cost a second round: W = 24,
+// T = 32768 in 7 segments 519, in 6 440, W = 112 in 3 1837, in 2 1464), and balances the
 // passes over a segment (~3.5 us per chunk) against the serial combine (~1.4
 // us per segment; W = 4, T = 20011 25 segments 105 us, at 1.1 us 97, and 16
 // 106, 12 120).
@@ -587,8 +589,8 @@ static void chain_form(long long ncmax, long long nctotal, int N, int Hv, int K,
   const long long least = W > 8 ? std::max(72LL, 4 * W) : K == 128 ? 68 : 64;
   const long long least_saving = K == 128 ? std::max(96LL, std::min(8 * W, 256LL)) : 0;
   if (square && 2 * W <= cus && nct >= (saving ? std::max(least, least_saving) : least)) {
-    const double fill = K == 128 ? (double)cus / (2 * W) + 1 : (double)cus / W;
-    const double ns = std::min(fill, 1.5 * std::sqrt((double)nct));
+    const long long fill = K == 128 ? (cus + 3 * W) / (2 * W) : cus / W;
+    const double ns = std::min((double)fill, 1.5 * std::sqrt((double)nct));
     p.seg = (int)std::ceil(nct / ns);
     p.whole_head = true;
     return;

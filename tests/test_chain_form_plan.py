@@ -47,3 +47,15 @@ def test_packed_workspace_has_no_room_for_uncut_sequences(N, K):
         cut = (T + 63 * N) // 64 // 64
         got = lib.gdn_chunk_workspace_bytes(1, T, 16, 32, K, K, N, 1, 0)
         assert plain <= got <= plain + cut * 32 * 10 * K * K + 4 * (N + 1) + 3 * 256
+
+
+@pytest.mark.parametrize("Hv", list(range(2, 129, 2)))
+def test_segments_fill_the_gpu_once(Hv):
+    """The first pass over the segments has a workgroup for each one's own contribution and, but
+    for a chain's first, its transfer matrix, the last segment apart: no more of them than compute
+    units (256 where no GPU is seen), beside which a few more would run alone."""
+    T = 64 * 1024
+    buffers = (_native.lib().gdn_chunk_workspace_bytes(1, T, Hv, Hv, 128, 128, 1, 0, 0) -
+               _plain(T, Hv, Hv, 128, 0)) // (Hv * 10 * 128 * 128)   # segments that another follows
+    assert buffers >= 1
+    assert Hv * (2 * buffers - 1) <= 256
