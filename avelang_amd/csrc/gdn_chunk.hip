@@ -560,14 +560,13 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 //    and loses with it (W = 8 69.4 -> 66.1, 64.1 -> 66.1; even at 68 chunks), at
 //    W = 16 it is even, at T = 2048 it loses everywhere.
 //    64-wide heads: W = 4, 4096 49 -> 42; W = 32, 8192 106 -> 93.
-//  - with the backward's saves, in segments a launch of their own, later:
-//    training forward W = 4, 4096 72 -> 81, 8192 128 -> 101; W = 16, 8192 165
-//    either way; W = 32, 8192 284 either way, its recomputing backward 600 ->
-//    627 and with l2norm 654 -> 669, 16384 571 -> 521 and 1179 either way.
-//    (W = 64, 16384 1093 -> 909, W = 128, 4096 unsegmented 577 -> 468: the
-//    forward that saves is taken at its best, recomputing there is 3 to 4 %
-//    slower, 2118 -> 2211 and 1110 -> 1146.)  64-wide heads win from the plain
-//    forward's line on.
+//  - with the backward's saves, from 9 chains on, later: training forward W =
+//    16, T = 8192 165 -> 160, W = 32, 8192 284 -> 280, but its recomputing
+//    backward 600 -> 627 and with l2norm 654 -> 669, 16384 571 -> 476 and 1179
+//    either way.  (W = 64, 16384 1093 -> 811, W = 128, 4096 unsegmented 577 ->
+//    468: the forward that saves is taken at its best, recomputing there is 3 to
+//    4 % slower, 2118 -> 2211 and 1110 -> 1146.)  64-wide heads win from the
+//    plain forward's line on.
 // The segment count fills the GPU once, and no more, with the first pass's
 // workgroups (two per segment, the first and last 1 and 0: W (2 ns - 3), one
 // per compute unit, 64-wide heads' two; at W = 32, T = 8192 5 segments 138 us,
@@ -587,7 +586,7 @@ static void chain_form(long long ncmax, long long nctotal, int N, int Hv, int K,
   const long long nct = std::max(1LL, ncmax / N);
   const bool square = K == V && segments;
   const long long least = W > 8 ? std::max(72LL, 4 * W) : K == 128 ? 68 : 64;
-  const long long least_saving = K == 128 ? std::max(96LL, std::min(8 * W, 256LL)) : 0;
+  const long long least_saving = K == 128 && W > 8 ? std::min(8 * W, 256LL) : 0;
   if (square && 2 * W <= cus && nct >= (saving ? std::max(least, least_saving) : least)) {
     const long long fill = K == 128 ? (cus + 3 * W) / (2 * W) : cus / W;
     const double ns = std::min((double)fill, 1.5 * std::sqrt((double)nct));

@@ -34,7 +34,10 @@
 // chunk) -- V as fp16, and the chunk's gate factors.
 //
 // Registers: K = V = 128 takes 256 VGPRs, unspilled but for saves and o in one
-// launch.  K = 128 with V = 64 (four waves, 106 KB of LDS: alone on its compute
+// launch, which spills 15 to 17 and is 2 to 15 % faster than a launch for each,
+// in segments too (W = 4, T = 20000 148 -> 129 us, W = 32, T = 16384 526 -> 476,
+// W = 64 897 -> 811; at 32 spilled registers it was slower there).
+// K = 128 with V = 64 (four waves, 106 KB of LDS: alone on its compute
 // unit) takes up to 422 with the AGPRs.  K = V = 64 (74 KB) takes 244 with COPY
 // and 275 without, where a compute unit then holds one workgroup instead of
 // two (held to 256 it would spill 32).
@@ -932,33 +935,12 @@ void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, 
     const unsigned seqs = std::min<unsigned>(N, std::max(1u, 4u * device_cus() / tiles));
     hipLaunchKernelGGL((chunk_combine_kernel<K>), dim3(tiles, seqs), dim3(4 * K), 0, st, a, ws);
   }
-  // A training forward in segments forms saves and o in two launches: with both
-  // the kernel is 15 to 17 registers over its 256 (32 when this was measured),
-  // and each reload waits until the step's stores are in memory.  T = 8192, 32 heads (160 workgroups): 177 us in
-  // one launch, 98 + 70 in two.  Whole sequences (many workgroups, HBM-bound)
-  // keep one launch and read the operands once.
-  bool apart = false;
-  if constexpr (SAVE && OUT && K == 128) {
-    apart = p.seg && V == 128;
-    if (apart) {
-      // (the saves leave ht alone: it may be h0, from which the outputs start)
-      HeadArgs saves = a;
-      saves.ht = nullptr;
-      const auto kern = l2 ? chunk_head_kernel<K, 128, true, true, false, false>
-                           : chunk_head_kernel<K, 128, false, true, false, false>;
-      hipLaunchKernelGGL(kern, dim3(grid), dim3(4 * V), 0, st, saves, ws);
-      if (l2) go(chunk_head_kernel<K, 128, true, false, true, false>, grid);
-      else go(chunk_head_kernel<K, 128, false, false, true, false>, grid);
-    }
-  }
-  if (!apart) {
-    if (V == 128) {
-      if (l2) go(chunk_head_kernel<K, 128, true, SAVE, OUT, false>, grid);
-      else go(chunk_head_kernel<K, 128, false, SAVE, OUT, false>, grid);
-    } else {
-      if (l2) go(chunk_head_kernel<K, 64, true, SAVE, OUT, false>, grid);
-      else go(chunk_head_kernel<K, 64, false, SAVE, OUT, false>, grid);
-    }
+  if (V == 128) {
+    if (l2) go(chunk_head_kernel<K, 128, true, SAVE, OUT, false>, grid);
+    else go(chunk_head_kernel<K, 128, false, SAVE, OUT, false>, grid);
+  } else {
+    if (l2) go(chunk_head_kernel<K, 64, true, SAVE, OUT, false>, grid);
+    else go(chunk_head_kernel<K, 64, false, SAVE, OUT, false>, grid);
   }
   if (ht_in_segs)
     hipLaunchKernelGGL(chunk_final_state_kernel, dim3(Hv, std::min(N, 1024)), dim3(256), 0, st, a,

@@ -136,8 +136,10 @@ def _training(dev, l2):
     yield W.make(B, 70, 2, 4, 128, 128, seed=8, h0_scale=0.01, l2norm=not l2), "whole"
     yield W.make(1, 4200, 1, 2, 128, 128, seed=9, h0_scale=0.05, decay=0.01,
                  l2norm=not l2), "segments"
-    yield W.make(1, 6200, 1, 2, 128, 128, seed=9, h0_scale=0.05, decay=0.01,
-                 l2norm=not l2), "segments, with the saves too"
+    yield W.make(1, 4400, 1, 2, 128, 128, seed=9, h0_scale=0.05, decay=0.01,
+                 l2norm=not l2), "segments, of 68 chunks and more"
+    yield W.make(1, 6200, 5, 10, 128, 128, seed=9, h0_scale=0.05, decay=0.01,
+                 l2norm=not l2), "segments, nine chains and more"
 
 
 @pytest.mark.parametrize("l2", [False, True])
@@ -154,7 +156,7 @@ def test_training_forward_beside_a_plain_one_in_segments(rocm_device, l2):
     """Sizes whose plain forward alone is cut: o and the final state agree to rounding (o within
     two bf16 steps of its size, the state as the forms' own 4e-4 from 64 bits allow)."""
     from avelang_amd import chunk_gated_delta_rule_fwd_save
-    wl = W.make(1, 5500, 1, 2, 128, 128, seed=9, h0_scale=0.05, decay=0.01, l2norm=not l2)
+    wl = W.make(1, 5500, 6, 12, 128, 128, seed=9, h0_scale=0.05, decay=0.01, l2norm=not l2)
     o, s = _run(wl, rocm_device, l2)
     o2, s2, _ = _run(wl, rocm_device, l2, fn=chunk_gated_delta_rule_fwd_save)
     assert not torch.equal(s, s2)
