@@ -122,6 +122,19 @@ int validate_rows(const char* name, const void* q, const void* k, const void* v,
   return GDN_OK;
 }
 
+int plan_for(const char* name, int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu,
+             bool l2, bool bwd, const void* workspace, size_t bytes, gdn::WsPlan& p) {
+  size_t best = 0;
+  for (const gdn::Room room : {gdn::Room::kBest, gdn::Room::kLeast}) {
+    p = gdn::plan_ws(B, T, Hqk, Hv, K, V, N, has_cu, l2, bwd, room);
+    if (workspace && bytes >= p.total) return GDN_OK;
+    if (room == gdn::Room::kBest) best = p.total;
+  }
+  return fail(GDN_ERR_WORKSPACE, std::string(name) + ": workspace needs " +
+                                     std::to_string(p.total) + " bytes (" + std::to_string(best) +
+                                     " to run at its best), got " + std::to_string(bytes));
+}
+
 }  // namespace gdn_host
 
 extern "C" const char* gdn_last_error(void) { return gdn_host::g_last_error.c_str(); }

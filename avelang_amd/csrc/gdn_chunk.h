@@ -207,8 +207,12 @@ struct WsPlan {
   long long ncmax;
 };
 
+// What a plan may ask for: all that makes the call faster, no segments, or
+// nothing that the call can run without (one V tile per workgroup reads K from
+// the caller's rows), which grows with B, T and N.
+enum class Room { kBest, kNoSegments, kLeast };
 WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, bool l2,
-               bool bwd, bool segments = true);
+               bool bwd, Room room = Room::kBest);
 
 // What a forward launch sequence writes: kForward = o / ht only; kRecompute =
 // the backward's inputs only (prep adds tmat / ttfrag / ptfrag, the chain
@@ -224,6 +228,16 @@ void launch_chunk_fwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, c
                       const TokenStride* rows = nullptr);
 
 ChunkWs ws_pointers(const WsPlan& p, unsigned char* wsb);
+
+}  // namespace gdn
+namespace gdn_host {
+// The plan of the entry point `name` for a workspace of `bytes`: the best one,
+// or where it does not fit the least (a caller's buffer for its largest problem
+// holds any smaller one), or GDN_ERR_WORKSPACE.
+int plan_for(const char* name, int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu,
+             bool l2, bool bwd, const void* workspace, size_t bytes, gdn::WsPlan& p);
+}  // namespace gdn_host
+namespace gdn {
 
 // Forward chain, state-wave form (gdn_chunk_chain.hip).  SAVE: the state at
 // every chunk start and the per-token deltas for the backward; OUT: o, ht.

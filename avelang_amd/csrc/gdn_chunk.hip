@@ -602,12 +602,12 @@ static void chain_form(long long ncmax, long long nctotal, int N, int Hv, int K,
 }
 
 WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, bool l2,
-               bool bwd, bool segments) {
+               bool bwd, Room room) {
   WsPlan p{};
   const long long total = (long long)B * T;
   p.ncmax = has_cu ? (total + 63LL * N) / 64 : (long long)B * ((T + 63) / 64);
   const size_t nch = (size_t)p.ncmax * Hv;   // (chunk, v-head) pairs
-  chain_form(p.ncmax, (total + 63) / 64, N, Hv, K, V, has_cu, segments, bwd, p);
+  chain_form(p.ncmax, (total + 63) / 64, N, Hv, K, V, has_cu, room == Room::kBest, bwd, p);
   size_t at = 0;
   auto take = [&](size_t bytes) {
     const size_t here = at;
@@ -623,7 +623,8 @@ WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, 
   // Q only with use_qk_l2norm (normalised), K also for the backward's reverse
   // chain and for two V tiles per workgroup of the state-wave form
   const size_t nqk = (size_t)p.ncmax * Hqk;   // (chunk, qk-head) pairs
-  p.k16_copy = bwd || l2 || (!p.whole_head && !chain_reads_rows(bwd, l2, N, Hv, V));
+  p.k16_copy = bwd || l2 || (!p.whole_head && room != Room::kLeast &&
+                             !chain_reads_rows(bwd, l2, N, Hv, V));
   p.q16_copy = l2;
   p.k16 = take(p.k16_copy ? nqk * (K == 128 ? KLayout<128>::BYTES : KLayout<64>::BYTES) : 0);
   p.q16 = take(p.q16_copy ? nqk * 64 * K * 2 : 0);
@@ -775,12 +776,10 @@ int chunk_fwd_impl(const void* q, const void* k, const void* v, const float* g,
                    const gdn::TokenStride* rows = nullptr) {
   if (N == 0 || ((long long)B * T == 0 && !ht)) return GDN_OK;  // nothing to compute
   gdn_host::launch_begin();
-  const gdn::WsPlan p = gdn::plan_ws(B, T, Hqk, Hv, K, V, N, cu_seqlens != nullptr,
-                                     use_qk_l2norm != 0, false);
-  if (!workspace || workspace_bytes < p.total)
-    return gdn_host::fail(GDN_ERR_WORKSPACE, std::string(name) + ": workspace needs " +
-                                                 std::to_string(p.total) + " bytes, got " +
-                                                 std::to_string(workspace_bytes));
+  gdn::WsPlan p;
+  const int rc = gdn_host::plan_for(name, B, T, Hqk, Hv, K, V, N, cu_seqlens != nullptr,
+                                    use_qk_l2norm != 0, false, workspace, workspace_bytes, p);
+  if (rc) return rc;
   if (p.ncmax > (1LL << 30) || (long long)N * Hv * (V / 16) >= (1LL << 31))
     return gdn_host::fail(GDN_ERR_SHAPE, std::string(name) + ": problem too large");
   gdn::launch_chunk_fwd(static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),
@@ -921,8 +920,12 @@ extern "C" int gdn_chunk_fwd_noalloc(const void* q, const void* k, const void* v
   if (N == 0 || ((long long)B * T == 0 && !ht)) return GDN_OK;  // nothing to compute
   gdn_host::launch_begin();
   // (without segments, whose buffers would take problems over the scratch)
-  const gdn::WsPlan p = gdn::plan_ws(B, T, Hqk, Hv, K, V, N, cu_seqlens != nullptr,
-                                     use_qk_l2norm != 0, false, false);
+  gdn::WsPlan p;
+  for (const gdn::Room room : {gdn::Room::kNoSegments, gdn::Room::kLeast}) {
+    p = gdn::plan_ws(B, T, Hqk, Hv, K, V, N, cu_seqlens != nullptr, use_qk_l2norm != 0, false,
+                     room);
+    if (p.total <= kNoAllocScratchBytes) break;
+  }
   if (p.total > kNoAllocScratchBytes)
     return gdn_host::fail(GDN_ERR_WORKSPACE,
                           "gdn_chunk_fwd_noalloc: the problem needs " + std::to_string(p.total) +
@@ -952,12 +955,10 @@ extern "C" int gdn_chunk_fwd_save(const void* q, const void* k, const void* v, c
   if (rc) return rc;
   if (N == 0 || ((long long)B * T == 0 && !ht)) return GDN_OK;  // nothing to compute
   gdn_host::launch_begin();
-  const gdn::WsPlan p = gdn::plan_ws(B, T, Hqk, Hv, K, V, N, cu_seqlens != nullptr,
-                                     use_qk_l2norm != 0, true);
-  if (!workspace || workspace_bytes < p.total)
-    return gdn_host::fail(GDN_ERR_WORKSPACE, "gdn_chunk_fwd_save: workspace needs " +
-                                                 std::to_string(p.total) + " bytes, got " +
-                                                 std::to_string(workspace_bytes));
+  gdn::WsPlan p;
+  rc = gdn_host::plan_for("gdn_chunk_fwd_save", B, T, Hqk, Hv, K, V, N, cu_seqlens != nullptr,
+                          use_qk_l2norm != 0, true, workspace, workspace_bytes, p);
+  if (rc) return rc;
   if (p.ncmax > (1LL << 30) || (long long)N * Hv * (V / 16) >= (1LL << 31))
     return gdn_host::fail(GDN_ERR_SHAPE, "gdn_chunk_fwd_save: problem too large");
   gdn::launch_chunk_fwd(static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),

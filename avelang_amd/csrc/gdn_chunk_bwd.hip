@@ -959,12 +959,10 @@ extern "C" int gdn_chunk_bwd(const void* q, const void* k, const void* v, const 
   }
   if (N == 0 || (tokens == 0 && !dh0)) return GDN_OK;
   gdn_host::launch_begin();
-  const gdn::WsPlan p = gdn::plan_ws(B, T, Hqk, Hv, K, V, N, cu_seqlens != nullptr,
-                                     use_qk_l2norm != 0, true);
-  if (!workspace || workspace_bytes < p.total)
-    return gdn_host::fail(GDN_ERR_WORKSPACE, "gdn_chunk_bwd: workspace needs " +
-                                                 std::to_string(p.total) + " bytes, got " +
-                                                 std::to_string(workspace_bytes));
+  gdn::WsPlan p;
+  rc = gdn_host::plan_for("gdn_chunk_bwd", B, T, Hqk, Hv, K, V, N, cu_seqlens != nullptr,
+                          use_qk_l2norm != 0, true, workspace, workspace_bytes, p);
+  if (rc) return rc;
   if (p.ncmax > (1LL << 30) || (long long)N * Hv * (V / 16) >= (1LL << 31) ||
       p.ncmax * (long long)Hqk >= (1LL << 30))
     return gdn_host::fail(GDN_ERR_SHAPE, "gdn_chunk_bwd: problem too large");

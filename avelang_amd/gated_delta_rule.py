@@ -248,8 +248,8 @@ def chunk_gated_delta_rule_bwd(
         if saved:
             raise ValueError(f"{name}: saved=True needs the training forward's workspace.")
         workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
-    elif workspace.numel() * workspace.element_size() < nbytes or workspace.device != dev:
-        raise ValueError(f"{name}: workspace must be >= {nbytes} bytes on {dev}.")
+    elif workspace.device != dev:   # (its size is checked by the entry point)
+        raise ValueError(f"{name}: workspace must be on {dev}.")
     rc = _native.lib().gdn_chunk_bwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(), _ptr(h0),
         do.data_ptr(), _ptr(dht),
@@ -367,9 +367,10 @@ def chunk_gated_delta_rule(
 
     Semantics of torch_chunk_gated_delta_rule (modeling_qwen3_next.py:374-453)
     with FLA's argument list.  Returns ``(o, final_state)``; ``final_state``
-    is ``None`` unless ``output_final_state``.  ``workspace`` (uint8, at least
-    ``chunk_workspace_bytes(...)``), ``out`` and ``final_state`` may be passed
-    to avoid allocation; ``final_state`` may be ``initial_state`` itself.
+    is ``None`` unless ``output_final_state``.  ``workspace`` (uint8, of
+    ``chunk_workspace_bytes(...)`` for this problem or any larger one),
+    ``out`` and ``final_state`` may be passed to avoid allocation;
+    ``final_state`` may be ``initial_state`` itself.
     With ``use_qk_l2norm_in_kernel`` q and k are L2-normalised (eps 1e-6)
     and rounded to bf16 before use, as FLA's separate l2norm pass does.
     The sequential state products run on fp16 operands (fp32 state and
@@ -438,8 +439,8 @@ def _chunk_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, cu_se
                                        use_qk_l2norm_in_kernel)
     if workspace is None:
         workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
-    elif workspace.numel() * workspace.element_size() < nbytes or workspace.device != dev:
-        raise ValueError(f"{name}: workspace must be >= {nbytes} bytes on {dev}.")
+    elif workspace.device != dev:   # (its size is checked by the entry point)
+        raise ValueError(f"{name}: workspace must be on {dev}.")
     if rows is not None:
         rc = _native.lib().gdn_chunk_fwd_rows(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), *rows,

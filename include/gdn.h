@@ -66,7 +66,10 @@ extern "C" {
  *       ht may equal h0 (in-place update); any other overlap is an error.
  *   use_qk_l2norm != 0: q and k are L2-normalised over K (eps 1e-6) and
  *       rounded to bf16 before use.
- *   workspace: device scratch of at least gdn_chunk_workspace_bytes(...).
+ *   workspace: device scratch of gdn_chunk_workspace_bytes(...) for these
+ *       sizes, or for others with B, T and N no smaller (where that is less
+ *       than these sizes' own, the call takes a form that needs no more and
+ *       agrees to rounding).
  * Precision: the sequential state products take fp16 operands (one MFMA
  * pass, fp32 accumulation and fp32 state), so q, k, the state and v-sized
  * intermediates must stay inside fp16's range (|x| < 65504); l2-normalised

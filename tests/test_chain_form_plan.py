@@ -1,5 +1,7 @@
 """Workspace of the segmented chain form (CPU): what gdn_chunk_fwd_noalloc refuses is still
 decided by the buffers without segments, and the backward's workspace covers the forward's."""
+import re
+
 import pytest
 
 from avelang_amd import _native
@@ -59,3 +61,37 @@ def test_segments_fill_the_gpu_once(Hv):
                _plain(T, Hv, Hv, 128, 0)) // (Hv * 10 * 128 * 128)   # segments that another follows
     assert buffers >= 1
     assert Hv * (2 * buffers - 1) <= 256
+
+
+def _least(lib, entry, B, T, Hqk, Hv, K, N, cu, l2):
+    """Bytes that a forward of these sizes cannot do without (from its refusal of none)."""
+    fake = [i << 40 for i in range(1, 6)] + [None, None, 6 << 40, (7 << 40) if cu else None]
+    assert entry(*fake, B, T, Hqk, Hv, K, K, N, 0.1, l2, None, 0, None) == -4
+    return int(re.search(r"workspace needs (\d+) bytes", lib.gdn_last_error().decode()).group(1))
+
+
+@pytest.mark.parametrize("cu", [0, 1])
+@pytest.mark.parametrize("l2", [0, 1])
+@pytest.mark.parametrize("save", [0, 1])
+@pytest.mark.parametrize("Hqk,Hv,K", [(2, 4, 128), (16, 32, 128), (4, 8, 64)])
+def test_a_buffer_for_the_largest_problem_holds_every_smaller_one(Hqk, Hv, K, save, l2, cu):
+    """The form that a call takes, and with it the workspace it takes at its best, changes with the
+    sizes; what it needs grows with B, T and N, up to what any larger problem's query gave."""
+    lib = _native.lib()
+    entry, query = ((lib.gdn_chunk_fwd_save, lib.gdn_chunk_bwd_workspace_bytes) if save else
+                    (lib.gdn_chunk_fwd, lib.gdn_chunk_workspace_bytes))
+    Ts = [1, 64, 500, 2048, 4352, 5184, 5248, 8192, 16384, 40000]
+    Ns = [1, 2, 3, 4, 8, 13, 64, 300]
+    seen = 0   # problems whose best is over a larger one's
+    for i, T in enumerate(Ts):
+        for j, N in enumerate(Ns):
+            dims = (1, T, Hqk, Hv, K, N) if cu else (N, T, Hqk, Hv, K, N)
+            least = _least(lib, entry, *dims, cu, l2)
+            best = query(dims[0], T, Hqk, Hv, K, K, N, cu, l2)
+            assert least <= best
+            for T2, N2 in ((T, Ns[j:]), (Ts[min(i + 1, len(Ts) - 1)], Ns[j:])):
+                for n in N2:
+                    size = query(1 if cu else n, T2, Hqk, Hv, K, K, n, cu, l2)
+                    assert least <= size, (T, N, T2, n)
+                    seen += best > size
+    assert seen or K == 64 or save or l2

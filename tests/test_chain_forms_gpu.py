@@ -283,3 +283,27 @@ def test_padding_leaves_the_state(rocm_device, what):
                                    initial_state=t["initial_state"])
     torch.cuda.synchronize()
     assert torch.equal(ht, t["initial_state"])
+
+
+@pytest.mark.parametrize("small,large", [
+    (dict(B=1, T=5184, Hqk=2, Hv=4), dict(B=1, T=5248, Hqk=2, Hv=4)),        # segments
+    (dict(B=2, T=700, Hqk=16, Hv=32), dict(B=4, T=700, Hqk=16, Hv=32))])     # two tiles, fp16 K
+def test_in_the_workspace_of_a_larger_problem(rocm_device, small, large):
+    """... whose form needs less, and in the least that the call takes: the same to rounding."""
+    from avelang_amd import chunk_workspace_bytes
+    size = lambda d: chunk_workspace_bytes(d["B"], d["T"], d["Hqk"], d["Hv"], 128, 128,  # noqa: E731
+                                           d["B"], False)
+    wl = W.make(**small, K=128, V=128, seed=31, h0_scale=0.05)
+    o, s = _run(wl, rocm_device)
+    n = -(-small["T"] // 64) * small["B"] * small["Hv"]
+    least = 512 + 256 * n + 2 * 6144 * n
+    for nbytes in (size(large), least):
+        assert least <= nbytes
+        ws = torch.full((nbytes + 4096,), 0x5a, dtype=torch.uint8, device=rocm_device)
+        o2, s2 = _run(wl, rocm_device, workspace=ws[:nbytes])
+        assert bool((ws[nbytes:] == 0x5a).all())
+        assert (s2 - s).norm() <= 8e-4 * s.norm()
+        assert (o2.float() - o.float()).norm() <= 2 ** -7 * o.float().norm()
+    assert least < size(small)
+    with pytest.raises(ValueError, match="workspace needs"):
+        _run(wl, rocm_device, workspace=ws[:least - 1])
