@@ -14,6 +14,8 @@ namespace gdn {
 // stated.  The backward-only buffers are NULL in a plain forward call.
 struct ChunkWs {
   int32_t* off;     // [N+1] first global chunk of each sequence
+  int32_t* longs;   // [1 + nlong] how many sequences take the state-wave form, then which
+                    // (WsPlan::longer, else NULL)
   int32_t* soff;    // [N+1] first segment of each sequence (cu_seqlens and segments)
   float* segs;      // [full segments][Hv][K][V] a segment's own contribution to the state, then
                     // the state after it
@@ -196,10 +198,15 @@ inline bool chain_reads_rows(bool bwd, bool l2, int N, int Hv, int V) {
 // Workspace plan (byte offsets into the caller's buffer).
 struct WsPlan {
   size_t off, status, gate, tfrag, pfrag, k16, q16, qn, kn, total;
-  size_t soff, segs, segm;
+  size_t longs, soff, segs, segm;
   // chunks per segment (0: none), segments of all sequences at most, and the full
   // ones among them, which another follows: these alone have buffers
   int seg, nseg, nfull;
+  // (cu_seqlens) a sequence of more than `cut` chunks is cut into segments; or,
+  // where one has more than `longer` (0: never), those of more than `member`
+  // chunks, nlong at most, take the state-wave form beside the others'
+  // whole-head form
+  int cut, longer, member, nlong;
   bool whole_head;   // the forward chain takes the whole-head form (gdn_chunk_head.hip)
   bool k16_copy, q16_copy;   // k16 / q16 planned (else the chains read the caller's rows)
   // backward only (0 when not planned)
@@ -242,12 +249,13 @@ namespace gdn {
 // Forward chain, state-wave form (gdn_chunk_chain.hip).  SAVE: the state at
 // every chunk start and the per-token deltas for the backward; OUT: o, ht.
 // qraw, kraw (a forward, OUT without SAVE, both non-null): K and Q from the
-// caller's bf16 rows instead of ws.k16 / ws.q16.
+// bf16 rows instead of ws.k16 / ws.q16.  nlong: of the sequences that ws.longs
+// that many at most.
 template <int K, bool SAVE, bool OUT>
 void launch_chain_sw(const uint16_t* v, const uint16_t* qraw, const uint16_t* kraw,
                      const float* h0, float* ht, uint16_t* o, const int32_t* cu, int N, int T,
                      int total, int Hqk, int Hv, int V, float scale, TokenStride ts,
-                     const ChunkWs& ws, hipStream_t st);
+                     const ChunkWs& ws, hipStream_t st, int nlong = 0);
 
 // Forward chain, whole-head form (gdn_chunk_head.hip), in segments where the
 // plan has them: the same results and buffers, K and Q from the caller's rows

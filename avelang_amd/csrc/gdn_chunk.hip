@@ -51,87 +51,107 @@ namespace gdn {
 // (cu[0] == 0, non-decreasing, cu[N] == total).  A violation is recorded in
 // *status and every sequence is then treated as empty (all offsets 0), so
 // that no later kernel reads or writes past the packed tokens; the caller's
-// outputs are zero-filled by zero_on_violation_kernel.
-__global__ __launch_bounds__(256) void chunk_table_kernel(const int32_t* __restrict__ cu,
-                                                          int N, int T, int total,
-                                                          int ncmax, int seg,
-                                                          int32_t* __restrict__ off,
-                                                          int32_t* __restrict__ soff,
-                                                          int32_t* __restrict__ status) {
-  __shared__ int part[257], spart[257];
-  __shared__ int bad;
-  const int tid = threadIdx.x;
+// outputs are zero-filled, o by the prep kernel's workgroups, which then have no
+// chunk, the gradients by zero_on_violation_kernel.
+// With segments also the first-segment offsets (WsPlan::cut), and with
+// WsPlan::longer the list of the sequences that take the state-wave form.
+// Latency-bound, one workgroup: the sums over the threads' sequences are wave
+// scans (5.4 us for 8 sequences, 10.1 with one thread adding 256 sums).
+__global__ __launch_bounds__(256) void chunk_table_kernel(
+    const int32_t* __restrict__ cu, int N, int T, int total, int ncmax, int seg, int cut,
+    int longer, int member, int nlong, int32_t* __restrict__ off, int32_t* __restrict__ soff,
+    int32_t* __restrict__ longs, int32_t* __restrict__ status) {
+  __shared__ int wave_sum[3][4];
+  const int tid = threadIdx.x, lane = tid % 64, w = tid / 64;
   const int per = (N + 255) / 256;
   const int a = min(tid * per, N), b = min(a + per, N);
-  if (tid == 0) bad = cu[0] != 0 ? 1 : (cu[N] != total ? 3 : 0);
-  __syncthreads();
-  for (int n = a; n < b; ++n)
-    if (cu[n + 1] < cu[n]) atomicMax(&bad, 2);
-  __syncthreads();
-  if (bad) {
+  int bad = cu[0] != 0 ? 1 : (cu[N] != total ? 3 : 0);
+  // chunks, segments and list members of this thread's sequences
+  int sum[3] = {0, 0, 0};
+  bool any = false;
+  for (int n = a; n < b; ++n) {
+    if (cu[n + 1] < cu[n] && bad < 2) bad = 2;
+    int s, e;
+    seq_bounds(cu, n, T, total, s, e);
+    const int nc = (e - s + kChunk - 1) / kChunk;
+    sum[0] += nc;
+    sum[1] += seg && nc > cut ? (nc + seg - 1) / seg : 1;
+    sum[2] += longer && nc > member;
+    any |= longer && nc > longer;
+  }
+  if (__syncthreads_or(bad)) {
+    bad = __syncthreads_or(bad == 3) ? 3 : __syncthreads_or(bad == 2) ? 2 : 1;
     for (int n = tid; n <= N; n += 256) {
       off[n] = 0;
       if (seg) soff[n] = n;
     }
-    if (tid == 0) *status = bad;
+    if (tid == 0) {
+      *status = bad;
+      if (longer) longs[0] = 0;
+    }
     return;
   }
-  if (tid == 0) *status = 0;
-  // (with segments of `seg` chunks also their first-segment offsets, at
-  // least one segment per sequence)
-  int sum = 0, ssum = 0;
-  for (int n = a; n < b; ++n) {
-    int s, e;
-    seq_bounds(cu, n, T, total, s, e);
-    const int nc = (e - s + kChunk - 1) / kChunk;
-    sum += nc;
-    if (seg) ssum += max(1, (nc + seg - 1) / seg);
+  any = __syncthreads_or(any);
+  int run[3], all[3];   // sums before this thread's sequences, and of all
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    int x = sum[i];
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+      const int y = __shfl_up(x, d);
+      if (lane >= d) x += y;
+    }
+    run[i] = x - sum[i];
+    if (lane == 63) wave_sum[i][w] = x;
   }
-  part[tid + 1] = sum;
-  spart[tid + 1] = ssum;
   __syncthreads();
-  if (tid == 0) {
-    part[0] = spart[0] = 0;
-    for (int i = 1; i <= 256; ++i) {
-      part[i] += part[i - 1];
-      spart[i] += spart[i - 1];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    all[i] = 0;
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+      if (y < w) run[i] += wave_sum[i][y];
+      all[i] += wave_sum[i][y];
     }
   }
-  __syncthreads();
-  int run = part[tid], srun = spart[tid];
   for (int n = a; n < b; ++n) {
-    off[n] = min(run, ncmax);
-    if (seg) soff[n] = srun;
+    off[n] = min(run[0], ncmax);
+    if (seg) soff[n] = run[1];
     int s, e;
     seq_bounds(cu, n, T, total, s, e);
     const int nc = (e - s + kChunk - 1) / kChunk;
-    run += nc;
-    if (seg) srun += max(1, (nc + seg - 1) / seg);
+    run[0] += nc;
+    run[1] += seg && nc > cut ? (nc + seg - 1) / seg : 1;
+    if (any && nc > member && run[2] < nlong) longs[1 + run[2]++] = n;
   }
-  if (tid == 255) {
-    off[N] = min(part[256], ncmax);
-    if (seg) soff[N] = spart[256];
+  if (tid == 0) {
+    *status = 0;
+    off[N] = min(all[0], ncmax);
+    if (seg) soff[N] = all[1];
+    if (longer) longs[0] = any ? min(all[2], nlong) : 0;
   }
+}
+
+// Zeroes n bytes at p as thread i of `threads`: 16-byte stores over the
+// 16-byte-aligned body, then the bytes before and after it.
+__device__ inline void zero_fill(void* ptr, size_t n, size_t i, size_t threads) {
+  unsigned char* p = static_cast<unsigned char*>(ptr);
+  const size_t head = (16 - ((uintptr_t)p & 15)) & 15;
+  const size_t h = head < n ? head : n;
+  const size_t body = (n - h) / 16;
+  for (size_t j = i; j < body; j += threads)
+    reinterpret_cast<uint4*>(p + h)[j] = uint4{0, 0, 0, 0};
+  for (size_t j = i; j < h + (n - h - 16 * body); j += threads)
+    p[j < h ? j : h + 16 * body + (j - h)] = 0;
 }
 
 __global__ __launch_bounds__(256) void zero_on_violation_kernel(const int32_t* __restrict__ status,
                                                                 ZeroList z) {
   if (*status == 0) return;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (int i = 0; i < 5; ++i) {
-    // 16-byte stores over the 16-byte-aligned body, then the tail bytes
-    unsigned char* p = static_cast<unsigned char*>(z.p[i]);
-    if (!p) continue;
-    const size_t n = z.bytes[i];
-    const size_t head = (16 - ((uintptr_t)p & 15)) & 15;
-    const size_t h = head < n ? head : n;
-    const size_t body = (n - h) / 16;
-    for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < body; j += stride)
-      reinterpret_cast<uint4*>(p + h)[j] = uint4{0, 0, 0, 0};
-    for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < h + (n - h - 16 * body);
-         j += stride)
-      p[j < h ? j : h + 16 * body + (j - h)] = 0;
-  }
+  for (int i = 0; i < 5; ++i)
+    if (z.p[i])
+      zero_fill(z.p[i], z.bytes[i], (size_t)blockIdx.x * blockDim.x + threadIdx.x,
+                (size_t)gridDim.x * blockDim.x);
 }
 
 void launch_zero_on_violation(const int32_t* status, const ZeroList& z, hipStream_t st) {
@@ -184,7 +204,7 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const float* __restrict__ g, const float* __restrict__ beta,
     const int32_t* __restrict__ cu, int N, int T, int total, int Hqk, int Hv, float scale,
-    ChunkWs ws, GateIn gate, TokenStride ts, int ncmax, int apart) {
+    ChunkWs ws, GateIn gate, TokenStride ts, int ncmax, int apart, uint16_t* o, size_t o_bytes) {
   constexpr int KB = K / 32;
   // strictly lower 16 x 16 blocks of A only (block (bi, m), m < bi, at
   // bi (bi - 1) / 2 + m; row stride 20 keeps float4 rows aligned and the 16
@@ -217,7 +237,14 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(
   int n, cfirst;
   if (cu) {
     const int32_t* off = ws.off;
-    if (ci >= off[N]) return;
+    if (ci >= off[N]) {
+      // no such chunk: none at all after a cu_seqlens violation, and then every
+      // (chunk, v-head) of the grid zeroes its share of o
+      if (OUT && *ws.status)
+        zero_fill(o, o_bytes, ((size_t)h * ncmax + ci) * 256 + threadIdx.x,
+                  (size_t)ncmax * Hv * 256);
+      return;
+    }
     // sequence owning chunk ci: largest n < N with off[n] <= ci
     int lo = 0, hi = N;
     while (hi - lo > 1) {
@@ -575,29 +602,59 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // passes over a segment (~3.5 us per chunk) against the serial combine (~1.4
 // us per segment; W = 4, T = 20011 25 segments 105 us, at 1.1 us 97, and 16
 // 106, 12 120).
-// With cu_seqlens nct is the mean; an unsegmented form still cuts a sequence
-// much longer than that, which would otherwise run on its own.
-static void chain_form(long long ncmax, long long nctotal, int N, int Hv, int K, int V,
-                       bool has_cu, bool segments, bool saving, WsPlan& p) {
-  p.seg = 0;
-  p.whole_head = false;
+// With cu_seqlens nct is the mean, and the device alone knows the lengths
+// (chunk_table_kernel).  Its measure is the load, the chunks that a compute
+// unit would have of an even batch: whole heads take 2.5 us per chunk of the
+// longest sequence, state waves 1.5 and 7.8 per load, so that a sequence of over
+// 3 to 4 loads in whole heads runs on among idle compute units.
+//  - From a load of 24 on such a sequence is cut into segments of one load (8 us
+//    per load and ~20).  32 heads, state waves / whole heads / this: one
+//    sequence of 16384 and 3, 7, 15 of 128 tokens 448 / 633 / 337, 453 / 639 /
+//    326, 464 / 651 / 341 us; of 65536 and 63 of 128 1739 / 2522 / 1221; 16384
+//    and 7 of 2048 538 / 717 / 443; 8 of 128 to 4096 349 / 248 / 258.
+//  - Under it there is too little to cut.  Under 3/4 of the compute units in
+//    chains (4 sequences of 32 heads gain 7 to 10 % of an even batch and lose as
+//    much of a random one, 5 nothing on average) state waves; from there on (6,
+//    7: 97.9 for 121, 121 for 161, 133 for 201 us, at worst 200 for 164) whole
+//    heads, but for the sequences of more than a load where one has over 4:
+//    these take state waves, in a launch of their own (4096 and 7 of 128 tokens
+//    126 / 178 / 124, 8192 and 7 of 128 224 / 328 / 223).
+// (Head sizes with 64, whose whole heads gain less: from 2 loads on; 16384 and
+// 7 of 128 316 / 388 / 202, 4096 and 7 of 128 89 / 117 / 79.)
+static void chain_form(long long ncmax, long long total, int N, int Hv, int K, int V,
+                       bool has_cu, Room room, bool saving, WsPlan& p) {
   if (N <= 0 || ncmax <= 0) return;
   const long long W = (long long)N * Hv, cus = device_cus();
   const long long nct = std::max(1LL, ncmax / N);
-  const bool square = K == V && segments;
+  const bool square = K == V && room == Room::kBest;
   const long long least = W > 8 ? std::max(72LL, 4 * W) : K == 128 ? 68 : 64;
   const long long least_saving = K == 128 && W > 8 ? std::min(8 * W, 256LL) : 0;
   if (square && 2 * W <= cus && nct >= (saving ? std::max(least, least_saving) : least)) {
     const long long fill = K == 128 ? (cus + 3 * W) / (2 * W) : cus / W;
     const double ns = std::min((double)fill, 1.5 * std::sqrt((double)nct));
-    p.seg = (int)std::ceil(nct / ns);
+    p.seg = p.cut = (int)std::ceil(nct / ns);
     p.whole_head = true;
     return;
   }
-  p.whole_head = W >= (K == 128 && V == 128 ? cus / 2 : cus);
-  if (p.whole_head && square && has_cu) {
-    const long long seg = std::max(64LL, 6 * nct);
-    if (nctotal > 2 * seg) p.seg = (int)seg;
+  const bool full = K == 128 && V == 128;
+  // (a sequence has half a chunk of padding on average)
+  const double load = (total / 64. + N / 2.) * Hv / cus;
+  p.whole_head = W >= (!full ? cus : has_cu && load < 24 ? 3 * cus / 4 : cus / 2);
+  if (!p.whole_head || !has_cu) return;
+  const long long most = (total + 63) / 64;   // chunks of a sequence
+  if (square && load >= 24) {
+    const int seg = (int)std::ceil(load), cut = (full ? 33 : 22) * seg / 10 + 10;
+    if (most > cut) {
+      p.seg = seg;
+      p.cut = cut;
+    }
+  } else if (room != Room::kLeast) {
+    const int longer = (int)std::max(8., (full ? 4 : 2) * load);
+    if (most > longer) {
+      p.longer = longer;
+      p.member = (int)std::max(4., load);
+      p.nlong = (int)std::min<long long>(N, ncmax / (p.member + 1));
+    }
   }
 }
 
@@ -607,7 +664,7 @@ WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, 
   const long long total = (long long)B * T;
   p.ncmax = has_cu ? (total + 63LL * N) / 64 : (long long)B * ((T + 63) / 64);
   const size_t nch = (size_t)p.ncmax * Hv;   // (chunk, v-head) pairs
-  chain_form(p.ncmax, (total + 63) / 64, N, Hv, K, V, has_cu, room == Room::kBest, bwd, p);
+  chain_form(p.ncmax, total, N, Hv, K, V, has_cu, room, bwd, p);
   size_t at = 0;
   auto take = [&](size_t bytes) {
     const size_t here = at;
@@ -643,6 +700,7 @@ WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, 
     p.dd = take(nch * 64 * V * 2);
     p.qtfrag = take((size_t)p.ncmax * Hqk * (K / 16) * 2 * 64 * 16);
   }
+  if (p.longer) p.longs = take((size_t)(p.nlong + 1) * 4);
   if (p.seg) {
     const long long per = std::max(1LL, ((T + 63LL) / 64 + p.seg - 1) / p.seg);
     p.nfull = (int)(has_cu ? p.ncmax / p.seg : N * (per - 1));
@@ -666,6 +724,7 @@ ChunkWs ws_pointers(const WsPlan& p, unsigned char* wsb) {
   ws.q16 = p.q16_copy ? reinterpret_cast<u16x8*>(wsb + p.q16) : nullptr;
   ws.qn = reinterpret_cast<uint16_t*>(wsb + p.qn);
   ws.kn = reinterpret_cast<uint16_t*>(wsb + p.kn);
+  if (p.longer) ws.longs = reinterpret_cast<int32_t*>(wsb + p.longs);
   if (p.seg) {
     ws.soff = reinterpret_cast<int32_t*>(wsb + p.soff);
     ws.segs = reinterpret_cast<float*>(wsb + p.segs);
@@ -692,7 +751,8 @@ static void launch_chunk(const uint16_t* q, const uint16_t* k, const uint16_t* v
   const int total = B * T;
   if (cu)
     hipLaunchKernelGGL(chunk_table_kernel, dim3(1), dim3(256), 0, st, cu, N, T, total,
-                       (int)p.ncmax, p.seg, ws.off, ws.soff, ws.status);
+                       (int)p.ncmax, p.seg, p.cut, p.longer, p.member, p.nlong, ws.off, ws.soff,
+                       ws.longs, ws.status);
   if (p.ncmax > 0) {
     const long long pairs = p.ncmax * (long long)Hqk;
     const int apart = (int)std::min(128LL, (pairs + 7) / 8 * 8);
@@ -700,29 +760,21 @@ static void launch_chunk(const uint16_t* q, const uint16_t* k, const uint16_t* v
     if (l2)
       hipLaunchKernelGGL((chunk_prep_kernel<K, BWD, OUT, true>), dim3(grid), dim3(256),
                          0, st, q, k, g, beta, cu, N, T, total, Hqk, Hv, scale, ws, gate, ts,
-                         (int)p.ncmax, apart);
+                         (int)p.ncmax, apart, o, (size_t)total * Hv * V * 2);
     else
       hipLaunchKernelGGL((chunk_prep_kernel<K, BWD, OUT, false>), dim3(grid), dim3(256),
                          0, st, q, k, g, beta, cu, N, T, total, Hqk, Hv, scale, ws, gate, ts,
-                         (int)p.ncmax, apart);
+                         (int)p.ncmax, apart, o, (size_t)total * Hv * V * 2);
   }
   // the chain reads K and Q as the prep kernel's fp16 copies where the plan
   // has them (normalised with use_qk_l2norm), else as the caller's bf16 rows
   if (p.whole_head)
     launch_chain_head<K, BWD, OUT>(q, k, v, h0, OUT ? ht : nullptr, OUT ? o : nullptr, cu, N, T,
                                    total, Hqk, Hv, V, scale, l2, ts, p, ws, st);
-  else
+  if (!p.whole_head || p.longer)
     launch_chain_sw<K, BWD, OUT>(v, ws.q16 ? nullptr : q, ws.k16 ? nullptr : k, h0,
-                               OUT ? ht : nullptr, OUT ? o : nullptr, cu, N, T, total, Hqk, Hv,
-                               V, scale, ts, ws, st);
-  // a cu_seqlens violation left every sequence empty: o is zero-filled (and
-  // ht = h0, written by the chain for an empty sequence)
-  if (cu && OUT) {
-    ZeroList z{};
-    z.p[0] = o;
-    z.bytes[0] = (size_t)total * Hv * V * 2;
-    launch_zero_on_violation(ws.status, z, st);
-  }
+                                 OUT ? ht : nullptr, OUT ? o : nullptr, cu, N, T, total, Hqk, Hv,
+                                 V, scale, ts, ws, st, p.nlong);
 }
 
 void launch_chunk_fwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, const float* g,

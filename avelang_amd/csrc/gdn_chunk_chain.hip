@@ -83,7 +83,8 @@ __global__ __launch_bounds__((chain_waves<SAVE, OUT, NS, RAWK>() * 64)) void
 chunk_chain_sw_kernel(const uint16_t* __restrict__ v, const uint16_t* __restrict__ qraw,
                       const uint16_t* __restrict__ kraw, const float* h0, float* ht,
                       uint16_t* __restrict__ o, const int32_t* __restrict__ cu, int N, int T,
-                      int total, int Hqk, int Hv, int V, float scale, TokenStride ts, ChunkWs ws) {
+                      int total, int Hqk, int Hv, int V, float scale, TokenStride ts, ChunkWs ws,
+                      const int32_t* longs) {
   static_assert(!RAWK || (OUT && !SAVE && NS == 1 && RAWQ), "RAWK is a plain forward");
   static_assert(!RAWQ || OUT, "RAWQ forms o");
   static_assert(!OUT || chain_split_out<SAVE, OUT, NS>(), "every form with o splits its output");
@@ -120,7 +121,11 @@ chunk_chain_sw_kernel(const uint16_t* __restrict__ v, const uint16_t* __restrict
   }
   const int vt0 = (bid % NVT) * NS;   // first V tile of this workgroup
   const int h = (bid / NVT) % Hv;
-  const int n = bid / NVT / Hv;
+  int n = bid / NVT / Hv;
+  if (longs) {   // the n-th of the list, if it has as many
+    if (n >= longs[0]) return;
+    n = longs[1 + n];
+  }
   const int hq = h / (Hv / Hqk);
 
   const int w = threadIdx.x / 64, lane = threadIdx.x % 64;
@@ -728,19 +733,19 @@ template <int K, bool SAVE, bool OUT>
 void launch_chain_sw(const uint16_t* v, const uint16_t* qraw, const uint16_t* kraw,
                      const float* h0, float* ht, uint16_t* o, const int32_t* cu, int N, int T,
                      int total, int Hqk, int Hv, int V, float scale, TokenStride ts,
-                     const ChunkWs& ws, hipStream_t st) {
+                     const ChunkWs& ws, hipStream_t st, int nlong) {
   // two V tiles per workgroup once the chains fill the GPU twice over: the
   // tiles share the stage and output waves' operand traffic, and every chain
   // still has a state wave of its own (not with both outputs, where a save
   // wave would make six waves; not with RAWK, see above)
-  const long long chains = (long long)N * Hv * (V / 16);
+  const long long chains = (long long)(nlong ? nlong : N) * Hv * (V / 16);
   const bool rawq = OUT && qraw;
   const bool rawk = OUT && !SAVE && rawq && kraw;
-  const bool two = !(SAVE && OUT) && !rawk && chain_two_tiles(N, Hv, V);
+  const bool two = !(SAVE && OUT) && !rawk && !nlong && chain_two_tiles(N, Hv, V);
   const dim3 grid((unsigned)(two ? chains / 2 : chains));
   auto go = [&](auto kern, int waves) {
     hipLaunchKernelGGL(kern, grid, dim3(waves * 64), 0, st, v, qraw, kraw, h0, ht, o, cu, N, T,
-                       total, Hqk, Hv, V, scale, ts, ws);
+                       total, Hqk, Hv, V, scale, ts, ws, nlong ? ws.longs : nullptr);
   };
   if constexpr (OUT) {
     if constexpr (!SAVE) {
@@ -766,7 +771,7 @@ void launch_chain_sw(const uint16_t* v, const uint16_t* qraw, const uint16_t* kr
   template void launch_chain_sw<K_, SAVE_, OUT_>(                                           \
       const uint16_t*, const uint16_t*, const uint16_t*, const float*, float*, uint16_t*,   \
       const int32_t*, int, int, int, int, int, int, float, TokenStride, const ChunkWs&,       \
-      hipStream_t);
+      hipStream_t, int);
 GDN_CHAIN_INST(64, false, true)
 GDN_CHAIN_INST(64, true, false)
 GDN_CHAIN_INST(64, true, true)

@@ -65,14 +65,15 @@ struct HeadArgs {
   int N, T, total, Hqk, Hv;
   float scale;
   int seg;      // chunks per segment (0: whole sequences)
+  int member;   // if ws.longs lists any, sequences of more chunks are (the state-wave form's)
   bool ht_in_segs;   // (segments, ht == h0) a cut sequence's final state goes to ws.segs
   TokenStride ts;
 };
 
 // Segments.  Sequence n's chunks are cut into segments of `seg` chunks (one
 // at least, also for an empty sequence); ws.soff[n] is its first segment's
-// global index with cu_seqlens (chunk_table_kernel), n times a constant
-// without.  Every segment but a sequence's last is full; ws.segs and ws.segm
+// global index with cu_seqlens (chunk_table_kernel, which leaves those of
+// `cut` chunks and less in one), n times a constant without.  Every segment but a sequence's last is full; ws.segs and ws.segm
 // hold the full ones alone, which the n last segments before are left out of:
 // segment j of sequence n is full segment first + j - n.
 __device__ __forceinline__ void seg_range(int n, int seg, const int32_t* cu, int T,
@@ -122,8 +123,8 @@ __device__ __forceinline__ SegPos seg_pos(int i, bool full, int seg, const int32
   const int c1 = cu ? ws.off[r.n + 1] : c0 + nct;
   r.first = j * seg;
   r.c_begin = c0 + r.first;
-  r.nc = seg ? min(seg, c1 - r.c_begin) : c1 - c0;
   r.last = j + 1 == cnt;
+  r.nc = r.last ? c1 - r.c_begin : seg;
   return r;
 }
 
@@ -242,6 +243,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
   // that another follows)
   const SegPos sp = seg_pos(bid / a.Hv, XFER, a.seg, a.cu, a.N, a.T, ws);
   if (sp.n < 0) return;
+  if (ws.longs && sp.nc > a.member && ws.longs[0] > 0) return;
   const int n = sp.n, full = sp.full;
   int s, e;
   seq_bounds(a.cu, n, a.T, a.total, s, e);
@@ -816,6 +818,7 @@ __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkW
   // time, a bit per thread.
   constexpr int NT = 4 * K;
   __shared__ unsigned long long many[NT / 64];
+  if (a.cu && ws.soff[a.N] == a.N) return;   // none is cut
   int seen = 0;
   for (int base = 0; base < a.N; base += NT) {
     int first = 0, count = 0;   // a sequence's segments
@@ -920,7 +923,8 @@ void launch_chain_head(const uint16_t* q, const uint16_t* k, const uint16_t* v, 
                        int Hv, int V, float scale, bool l2, TokenStride ts, const WsPlan& p,
                        const ChunkWs& ws, hipStream_t st) {
   const bool ht_in_segs = p.seg && p.nfull > 0 && ht && ht == h0;
-  const HeadArgs a{q, k, v, h0, ht, o, cu, N, T, total, Hqk, Hv, scale, p.seg, ht_in_segs, ts};
+  const HeadArgs a{q, k, v, h0, ht, o, cu, N, T, total, Hqk, Hv, scale, p.seg,
+                   p.member, ht_in_segs, ts};
   const unsigned grid = (unsigned)((p.seg ? p.nseg : N) * Hv);
   auto go = [&](auto kern, unsigned g) {
     hipLaunchKernelGGL(kern, dim3(g), dim3(4 * V), 0, st, a, ws);

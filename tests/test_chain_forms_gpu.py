@@ -69,15 +69,17 @@ def _cu(lens):
     return np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
 
 
-def _packed(dev, long=0):
-    """Sequences of 0 to 150 tokens (and one of `long`) over enough heads for the form."""
-    Hv = 8
+def _packed(dev, long=0, longs=(), K=128, l2norm=True):
+    """Sequences of 0 to 150 tokens (and one of `long`, or some of `longs`) over enough heads for
+    the form."""
+    Hv = 8 * 128 // K
     n = -(-_cus(dev) // Hv)
     rng = np.random.Generator(np.random.PCG64(5))
     lens = rng.integers(1, 151, size=n)
     lens[3], lens[n // 2] = 0, long or lens[n // 2]
+    lens[5:5 + 2 * len(longs):2] = longs
     cu = _cu(lens)
-    return W.make(1, int(cu[-1]), 4, Hv, 128, 128, seed=6, cu_seqlens=cu)
+    return W.make(1, int(cu[-1]), 4, Hv, K, K, seed=6, cu_seqlens=cu, l2norm=l2norm)
 
 
 def test_whole_head_packed(rocm_device):
@@ -85,8 +87,50 @@ def test_whole_head_packed(rocm_device):
 
 
 def test_whole_head_packed_with_one_long_sequence(rocm_device):
-    """A sequence far over the mean is cut into segments, the others stay whole."""
+    """A sequence far over the mean takes state waves, the others stay whole."""
     _check(_packed(rocm_device, long=6011), rocm_device, what="packed, one long")
+
+
+def _heavy(l2):
+    """32 heads: a sequence that is cut, in a batch that fills the GPU (load 24)."""
+    cu = _cu([9000, 0, 1, 3500])
+    return W.make(1, int(cu[-1]), 16, 32, 128, 128, seed=7, cu_seqlens=cu, l2norm=not l2)
+
+
+@pytest.mark.parametrize("l2", [False, True])
+def test_whole_head_packed_with_one_long_sequence_cut(rocm_device, l2):
+    """A sequence far over the load is cut into segments, the others stay whole."""
+    _check(_heavy(l2), rocm_device, l2, what="packed, one cut")
+
+
+# of a load of 3 to 13 chunks: under, at and over the 4 loads that are long, and over the one that
+# then takes state waves
+_LONGS = [(3000,), (1000, 500, 7, 1500), (3000, 2000), (3000, 2000, 7000), (9000, 4000, 9000, 250)]
+
+
+@pytest.mark.parametrize("K,l2", [(128, False), (128, True), (64, False)])
+@pytest.mark.parametrize("longs", _LONGS)
+def test_packed_with_long_sequences(rocm_device, longs, K, l2):
+    """Whole heads for the short sequences, state waves for the others."""
+    _check(_packed(rocm_device, longs=longs, K=K, l2norm=not l2), rocm_device, l2, str(longs))
+
+
+@pytest.mark.parametrize("l2", [False, True])
+@pytest.mark.parametrize("longs", _LONGS + ["cut"])
+def test_training_packed_with_long_sequences(rocm_device, longs, l2):
+    from avelang_amd import chunk_gated_delta_rule_bwd, chunk_gated_delta_rule_fwd_save
+    wl = _heavy(l2) if longs == "cut" else _packed(rocm_device, longs=longs, l2norm=not l2)
+    t = wl.torch(rocm_device)
+    o, s = _run(wl, rocm_device, l2)
+    o2, s2, ws = _run(wl, rocm_device, l2, fn=chunk_gated_delta_rule_fwd_save)
+    assert torch.equal(o, o2) and torch.equal(s, s2)
+    args = (t["q"], t["k"], t["v"], t["g"], t["beta"], torch.ones_like(t["v"]))
+    kw = dict(initial_state=t["initial_state"], cu_seqlens=t["cu_seqlens"],
+              use_qk_l2norm_in_kernel=l2)
+    got = chunk_gated_delta_rule_bwd(*args, workspace=ws, saved=True, **kw)
+    again = chunk_gated_delta_rule_bwd(*args, **kw)
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for x, y in zip(got, again))
 
 
 @pytest.mark.parametrize("B,T,Hqk,Hv,D,l2,decay", [
@@ -233,6 +277,8 @@ def _in_place_cases(dev):
         cu = _cu(lens)
         yield W.make(1, int(cu[-1]), 1, 2, 128, 128, seed=23, cu_seqlens=cu, decay=0.01,
                      h0_scale=0.05, l2norm=False), True
+    yield _packed(dev, longs=(3000, 2000, 7000)), False
+    yield _heavy(True), True
 
 
 def _save_workspace(wl, l2, dev):
