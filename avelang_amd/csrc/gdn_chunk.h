@@ -19,8 +19,10 @@ struct ChunkWs {
   int32_t* soff;    // [N+1] first segment of each sequence (cu_seqlens and segments)
   float* segs;      // [full segments][Hv][K][V] a segment's own contribution to the state, then
                     // the state after it
-  u16x8* segm;      // [full segments][Hv][part][K/16][K/32][64] a segment's transfer matrix M
-                    // as bf16 A-operand fragments of its three parts (rows in rho order)
+  u16x8* segm;      // [full segments][Hv][hi, lo][K/16][K/32][64] a segment's transfer matrix
+                    // less its decay on the diagonal, E = M - decay I, as bf16 A-operand
+                    // fragments, E = hi + lo (rows in rho order)
+  float* sdecay;    // [full segments][Hv] a segment's decay, e^(the sum of its g)
   int32_t* status;  // [1] 0, or the cu_seqlens violation the chunk table found
   float* gate;      // [NC][Hv][64]: G_i, the chunk-local cumulative log-decay
   u16x8* tfrag;     // [NC][Hv][6 slots][64 lanes] fp16 A-operand fragments of Tb,
@@ -198,7 +200,7 @@ inline bool chain_reads_rows(bool bwd, bool l2, int N, int Hv, int V) {
 // Workspace plan (byte offsets into the caller's buffer).
 struct WsPlan {
   size_t off, status, gate, tfrag, pfrag, k16, q16, qn, kn, total;
-  size_t longs, soff, segs, segm;
+  size_t longs, soff, segs, segm, sdecay;
   // chunks per segment (0: none), segments of all sequences at most, and the full
   // ones among them, which another follows: these alone have buffers
   int seg, nseg, nfull;

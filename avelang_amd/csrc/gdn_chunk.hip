@@ -599,9 +599,8 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // per compute unit, 64-wide heads' two; at W = 32, T = 8192 5 segments 138 us,
 // 4 155, 6 159, 8 152; a few workgroups over cost a second round: W = 24,
 // T = 32768 in 7 segments 519, in 6 440, W = 112 in 3 1837, in 2 1464), and balances the
-// passes over a segment (~3.5 us per chunk) against the serial combine (~1.4
-// us per segment; W = 4, T = 20011 25 segments 105 us, at 1.1 us 97, and 16
-// 106, 12 120).
+// passes over a segment (~3.5 us per chunk) against the serial combine (~1.2
+// us per segment; W = 4, T = 20011 25 segments 97 us, 16 106, 12 120).
 // With cu_seqlens nct is the mean, and the device alone knows the lengths
 // (chunk_table_kernel).  Its measure is the load, the chunks that a compute
 // unit would have of an even batch: whole heads take 2.5 us per chunk of the
@@ -707,7 +706,8 @@ WsPlan plan_ws(int B, int T, int Hqk, int Hv, int K, int V, int N, bool has_cu, 
     p.nseg = p.nfull + N;
     p.soff = take((size_t)(N + 1) * 4);
     p.segs = take((size_t)p.nfull * Hv * K * V * 4);
-    p.segm = take((size_t)p.nfull * Hv * K * K * 6);
+    p.segm = take((size_t)p.nfull * Hv * K * K * 4);
+    p.sdecay = take((size_t)p.nfull * Hv * 4);
   }
   p.total = at;
   return p;
@@ -729,6 +729,7 @@ ChunkWs ws_pointers(const WsPlan& p, unsigned char* wsb) {
     ws.soff = reinterpret_cast<int32_t*>(wsb + p.soff);
     ws.segs = reinterpret_cast<float*>(wsb + p.segs);
     ws.segm = reinterpret_cast<u16x8*>(wsb + p.segm);
+    ws.sdecay = reinterpret_cast<float*>(wsb + p.sdecay);
   }
   if (p.hs) {
     ws.tmat = reinterpret_cast<float*>(wsb + p.tmat);

@@ -418,6 +418,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
   auto lds4 = [&](int off) { return *reinterpret_cast<const f32x4*>(buf + off); };
   auto ldst = [&](int off) { return lds_tr16(reinterpret_cast<const uint16_t*>(buf + off)); };
 
+  float decay = 1.f;   // (XFER) of the state over the segment's chunks so far
   // What chunk j - 1 leaves for step j to finish: its output's Q S term
   // (scaled), vnew and P fragments.
   f32x4 O[2][4];
@@ -502,6 +503,7 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
       }
     };
     const float egl = *reinterpret_cast<const float*>(buf + (g_off - 32 * grp) + (kE - kG));
+    if constexpr (XFER) decay *= egl;
     read_blk(0);
     if constexpr (SAVE) {
       // the chunk's start state: hs[chunk][v-head] = S^T (bf16), row 32 w +
@@ -750,27 +752,29 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
     }
   }
   if (mpart) {
-    // M as three bf16 parts (split3_bf4), each as the combine's A fragments
-    // (row tile t, k-block w), transposed through this wave's share of the
-    // operand buffers
+    // E = M - decay I as hi + lo (bf16), the combine's A fragments (row tile t,
+    // k-block w), transposed through this wave's share of the operand buffers
     constexpr int LD = 20;
-    static_assert(3 * 32 * LD * 2 <= 4096 && 4096 * NW <= 2 * kBufStep, "a wave's share");
+    static_assert(2 * 32 * LD * 2 <= 4096 && 4096 * NW <= 2 * kBufStep, "a wave's share");
     uint16_t* X = reinterpret_cast<uint16_t*>(buf + 4096 * w);
-    u16x8* dst = ws.segm + ((size_t)full * a.Hv + h) * (3 * ST * KB * 64) + w * 64 + lane;
+    u16x8* dst = ws.segm + ((size_t)full * a.Hv + h) * (2 * ST * KB * 64) + w * 64 + lane;
+    if (threadIdx.x == 0) ws.sdecay[(size_t)full * a.Hv + h] = decay;
 #pragma unroll
     for (int t = 0; t < ST; ++t) {
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
-        u16x4 part[3];
-        split3_bf4(S[x][t], part);
+        f32x4 e = S[x][t];
 #pragma unroll
-        for (int y = 0; y < 3; ++y)
-          *reinterpret_cast<u16x4*>(X + (32 * y + 16 * x + r16) * LD + 4 * grp) = part[y];
+        for (int r = 0; r < 4; ++r)
+          if (rho_row(t, 4 * grp + r) == (int)lane_tile + 16 * x) e[r] -= decay;
+        u16x4 hi, lo;
+        split_bf4(e, hi, lo);
+        *reinterpret_cast<u16x4*>(X + (16 * x + r16) * LD + 4 * grp) = hi;
+        *reinterpret_cast<u16x4*>(X + (32 + 16 * x + r16) * LD + 4 * grp) = lo;
       }
       __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int y = 0; y < 3; ++y)
-        dst[(y * ST + t) * KB * 64] = lds_colfrag(X, LD, 32 * y, 0, lane);
+      dst[t * KB * 64] = lds_colfrag(X, LD, 0, 0, lane);
+      dst[(ST + t) * KB * 64] = lds_colfrag(X, LD, 32, 0, lane);
       __builtin_amdgcn_wave_barrier();
     }
     return;
@@ -795,20 +799,21 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
 
 // States at the segment starts: S_j = M_j S_(j-1) + B_j from the segments' own
 // contributions B (ws.segs; the first segment's is already the state after
-// it) and transfer matrices M (ws.segm), in place of B.  One workgroup per
-// (sequence, v-head, 16 value columns), wave w the state rows rho(16 w + m).
-// The state keeps its fp32: both operands of the product are split into three
-// bf16 parts, which hold all 24 bits (split3_bf4), and the six products of
-// 2^-17 and up are taken (M = I, a stretch of g = beta = 0, leaves every bit
-// of the state).  ~1.4 us per segment (T = 20011 of 4 heads, 25 segments:
-// 104.8 us per prefill; 97.0 with two parts and three products, which moved
-// the state by up to 2^-17 per segment).
-// The state passes between the waves through LDS, and a segment's M fragments
+// it) and transfer matrices M (ws.segm, ws.sdecay), in place of B.  One workgroup
+// per (sequence, v-head, 16 value columns), wave w the state rows rho(16 w + m).
+// M = decay I + E: the decay goes over the fp32 state in fp32, as within a
+// chunk (g = beta = 0 leaves every bit), and E S, what the segment's tokens
+// take out, is a product of bf16 hi + lo halves (three MFMA passes, ~2^-17
+// relative, where the chunks' own take fp16 operands, 2^-11).  Errors against
+// 64 bits are those of a chain in one piece to three digits.  ~1.2 us per
+// segment (25 of 4 heads 30.0 us, the call 98); M itself in three parts and six
+// products, exact too, took 37.0 and 105, on fp32 MFMA 42.
+// The state passes between the waves through LDS, and a segment's E fragments
 // are requested two segments ahead.
 template <int K>
 __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkWs ws) {
   constexpr int ST = K / 16, KB = K / 32;   // row tiles (waves), k-blocks
-  __shared__ __attribute__((aligned(16))) u16x8 St[2][3][KB][64];   // [parity][part]
+  __shared__ __attribute__((aligned(16))) u16x8 St[2][2][KB][64];   // [parity][hi, lo]
   const int h = blockIdx.x % a.Hv, vt = blockIdx.x / a.Hv;
   const int lane = threadIdx.x % 64;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -833,10 +838,10 @@ __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkW
         const int n = __builtin_amdgcn_readfirstlane(base + 64 * word + __builtin_ctzll(left));
         seg_range(n, a.seg, a.cu, a.T, ws, first, count);
         auto head = [&](int j) { return (size_t)(first - n + j) * a.Hv + h; };
-        auto load_m = [&](u16x8 (&m)[3][KB], int j) {
-          const u16x8* p = ws.segm + head(j) * (3 * ST * KB * 64) + w * KB * 64 + lane;
+        auto load_e = [&](u16x8 (&m)[2][KB], int j) {
+          const u16x8* p = ws.segm + head(j) * (2 * ST * KB * 64) + w * KB * 64 + lane;
 #pragma unroll
-          for (int y = 0; y < 3; ++y) {
+          for (int y = 0; y < 2; ++y) {
 #pragma unroll
             for (int b = 0; b < KB; ++b) m[y][b] = p[(y * ST * KB + b) * 64];
           }
@@ -851,45 +856,43 @@ __global__ __launch_bounds__(4 * K) void chunk_combine_kernel(HeadArgs a, ChunkW
           return f32x4{p[0], p[K], p[2 * K], p[3 * K]};
         };
         auto publish = [&](f32x4 x, int par) {
-          u16x4 part[3];
-          split3_bf4(x, part);
+          u16x4 part[2];
+          split_bf4(x, part[0], part[1]);
 #pragma unroll
-          for (int y = 0; y < 3; ++y)   // (a B fragment: tile w's half of k-block w / 2)
+          for (int y = 0; y < 2; ++y)   // (a B fragment: tile w's half of k-block w / 2)
             reinterpret_cast<u16x4*>(&St[par][y][w >> 1][lane])[w & 1] = part[y];
           lds_barrier();
         };
-        // segment j's M fragments and B tile in set j % 3
-        u16x8 m[3][3][KB];
+        // segment j's E fragments, decay and B tile in set j % 3
+        u16x8 m[3][2][KB];
         f32x4 bt[3];
-        load_m(m[1], 1);
-        bt[1] = load_b(1);
-        load_m(m[2], min(2, count - 2));
-        bt[2] = load_b(min(2, count - 2));
-        publish(load_b(0), 0);
+        float dec[3];
+        auto load = [&](auto set, int j) {
+          constexpr int c = decltype(set)::value;
+          load_e(m[c], j);
+          bt[c] = load_b(j);
+          dec[c] = ws.sdecay[head(j)];
+        };
+        load(std::integral_constant<int, 1>{}, 1);
+        load(std::integral_constant<int, 2>{}, min(2, count - 2));
+        f32x4 state = load_b(0);   // this wave's tile of the state after the segment before
+        publish(state, 0);
         auto step = [&](int j, auto jc) {
           constexpr int c = decltype(jc)::value;   // j % 3
-          const int jn = min(j + 2, count - 2);
-          load_m(m[(c + 2) % 3], jn);
-          bt[(c + 2) % 3] = load_b(jn);
-          f32x4 acc[3][3];   // [M part][state part], the largest six
+          load(std::integral_constant<int, (c + 2) % 3>{}, min(j + 2, count - 2));
+          f32x4 acc = zero4(), acc1 = zero4(), acc2 = zero4();
 #pragma unroll
           for (int b = 0; b < KB; ++b) {
-            const auto& sp = St[(j + 1) & 1];
-#pragma unroll
-            for (int z = 0; z < 3; ++z) {
-              const u16x8 part = sp[z][b][lane];
-#pragma unroll
-              for (int y = 0; y < 3 - z; ++y)
-                acc[y][z] = mfma16(m[c][y][b], part,
-                                   b ? acc[y][z] : (y || z ? zero4() : bt[c]));
-            }
+            const u16x8 hi = St[(j + 1) & 1][0][b][lane], lo = St[(j + 1) & 1][1][b][lane];
+            acc = mfma16(m[c][0][b], hi, acc);
+            acc1 = mfma16(m[c][0][b], lo, acc1);
+            acc2 = mfma16(m[c][1][b], hi, acc2);
           }
-          const f32x4 sum = acc[0][0] + ((acc[0][1] + acc[1][0]) +
-                                         ((acc[0][2] + acc[2][0]) + acc[1][1]));
+          state = dec[c] * state + (bt[c] + (acc + (acc1 + acc2)));
           float* o = tile_at(j);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) o[(size_t)r * K] = sum[r];
-          publish(sum, j & 1);
+          for (int r = 0; r < 4; ++r) o[(size_t)r * K] = state[r];
+          publish(state, j & 1);
         };
         for (int j = 1; j < count - 1;) {
           step(j++, std::integral_constant<int, 1>{});

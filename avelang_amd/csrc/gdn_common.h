@@ -63,16 +63,12 @@ typedef unsigned int u32x2p __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ u16x4 f2bf4(f32x4 x) {
   return __builtin_bit_cast(u16x4, __builtin_convertvector(x, bf16x4));
 }
-// x = part[0] + part[1] + part[2], exactly: each part rounds what is left to
-// bf16, whose 8 significand bits leave 16 and then 8 of fp32's 24.
-__device__ __forceinline__ void split3_bf4(f32x4 x, u16x4 (&part)[3]) {
-#pragma unroll
-  for (int y = 0; y < 3; ++y) {
-    const u32x2p p = __builtin_bit_cast(u32x2p, __builtin_convertvector(x, bf16x4));
-    part[y] = __builtin_bit_cast(u16x4, p);
-    x = x - f32x4{__uint_as_float(p[0] << 16), __uint_as_float(p[0] & 0xffff0000u),
-                  __uint_as_float(p[1] << 16), __uint_as_float(p[1] & 0xffff0000u)};
-  }
+__device__ __forceinline__ void split_bf4(f32x4 x, u16x4& hi, u16x4& lo) {
+  const u32x2p hp = __builtin_bit_cast(u32x2p, __builtin_convertvector(x, bf16x4));
+  const f32x4 hf = {__uint_as_float(hp[0] << 16), __uint_as_float(hp[0] & 0xffff0000u),
+                    __uint_as_float(hp[1] << 16), __uint_as_float(hp[1] & 0xffff0000u)};
+  hi = __builtin_bit_cast(u16x4, hp);
+  lo = f2bf4(x - hf);
 }
 
 __device__ __forceinline__ bf16x8 as_bf(u16x8 v) {

@@ -84,7 +84,7 @@ extern "C" {
  * the latter runs in segments (see there).
  * P = scale q.k e^(G_i - G_j) is rounded to fp16 in every form.  Few long
  * sequences (64 chunks and more) are run in segments, and so are those of a
- * packed batch that are far longer than its mean; their buffers (160 KiB per
+ * packed batch that are far longer than its mean; their buffers (128 KiB per
  * v-head at K = V = 128 and segment that another follows) are part of the
  * workspace.  The fp32 state crosses their borders as fp32.
  */

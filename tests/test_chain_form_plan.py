@@ -48,7 +48,7 @@ def test_packed_workspace_has_no_room_for_uncut_sequences(N, K):
     for T in (16384, 262144):
         plain = _plain(T, 16, 32, K, 0, N)
         got = lib.gdn_chunk_workspace_bytes(1, T, 16, 32, K, K, N, 1, 0)
-        assert plain <= got <= plain + 2 * 256 * 10 * K * K + 8 * (N + 1) + 4 * 256
+        assert plain <= got <= plain + 2 * 256 * (8 * K * K + 4) + 8 * (N + 1) + 5 * 256
 
 
 @pytest.mark.parametrize("Hv", list(range(2, 129, 2)))
@@ -58,7 +58,7 @@ def test_segments_fill_the_gpu_once(Hv):
     units (256 where no GPU is seen), beside which a few more would run alone."""
     T = 64 * 1024
     buffers = (_native.lib().gdn_chunk_workspace_bytes(1, T, Hv, Hv, 128, 128, 1, 0, 0) -
-               _plain(T, Hv, Hv, 128, 0)) // (Hv * 10 * 128 * 128)   # segments that another follows
+               _plain(T, Hv, Hv, 128, 0)) // (Hv * 8 * 128 * 128)   # segments that another follows
     assert buffers >= 1
     assert Hv * (2 * buffers - 1) <= 256
 
