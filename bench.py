@@ -516,7 +516,7 @@ def profile_pass(dev, reps=3, what="all"):
 
     1. one device-to-device copy of exactly 256 MiB (calibrates FETCH_SIZE /
        WRITE_SIZE against known bytes: 256 MiB read, 256 MiB written);
-    2. ``reps`` config-1 prefill calls (chunk_prep, chunk_chain);
+    2. ``reps`` config-1 prefill calls (chunk_prep, the chain's kernels);
     3. ``reps`` config-2 decode steps (recurrent_kernel<128,128>);
     4. ``reps`` calls of each layer operator at the Qwen3-Next layer shape;
     5. ``reps`` config-1 backward calls (gdn_chunk_bwd with its recomputation).
@@ -579,8 +579,9 @@ def pmc_summary(fetch_dir, write_dir, out_path):
     Each counter is averaged per kernel over its dispatches and scaled by
     what it reads for the pass's 256 MiB device copy (known bytes), so the
     figures are HBM bytes per launch.  Path totals: prefill = chunk_prep +
-    chunk_chain (forward instantiations), backward = the four launches of
-    gdn_chunk_bwd, decode = the recurrent kernel.
+    the forward chain (in segments: transfer pass, combine and outputs; else
+    one kernel), backward = the four launches of gdn_chunk_bwd, decode = the
+    recurrent kernel.
     """
     import csv
     import glob
@@ -614,12 +615,20 @@ def pmc_summary(fetch_dir, write_dir, out_path):
         # workgroup) do not change which launch of the path it is
         return any(k.startswith("gdn::" + p) and k[len("gdn::" + p)] in ",>" for p in prefixes)
 
+    # chunk_head_kernel<K, V, l2norm copies, saves, outputs, transfer pass>
+    def head(what):
+        return [f"chunk_head_kernel<128, 128, {copy}, {what}" for copy in ("false", "true")]
+
+    chain = ["chunk_chain_sw_kernel<128, false, true", *head("false, true, false")]
+    if not any(named(k, *chain) for k in kern):
+        raise SystemExit("pmc_summary: no kernel of the forward chain that writes the output")
     res = {
-        "prefill": total(lambda k: named(k, "chunk_prep_kernel<128, false",
-                                         "chunk_chain_sw_kernel<128, false, true")),
+        "prefill": total(lambda k: named(k, "chunk_prep_kernel<128, false", *chain,
+                                         *head("false, false, true"), "chunk_combine_kernel<128")),
         "decode": total(lambda k: "recurrent_kernel<128, 128" in k),
         "backward": total(lambda k: named(k, "chunk_prep_kernel<128, true",
                                           "chunk_chain_sw_kernel<128, true, false",
+                                          *head("true, false, false"),
                                           "chunk_rev_sw_kernel<128", "chunk_grad_kernel<128, 128")),
         "per_kernel": kern,
         "fetch_size_factor": round(ff, 4),
@@ -771,7 +780,8 @@ def main():
                      "unit": "TFLOP/s", "frac": round(tflops / BF16_PEAK_TFLOPS, 4),
                      "traffic": _load_traffic("prefill"),
                      "traffic_source": TRAFFIC_SOURCE,
-                     "kernel": "gdn_chunk_fwd = chunk_prep + chunk_chain (+ chunk_table with cu_seqlens)",
+                     "kernel": "gdn_chunk_fwd = chunk_prep + chunk_head (transfer pass) + "
+                               "chunk_combine + chunk_head (outputs)",
                      "algorithmic_flops_per_launch": flops,
                      "flops_per_token_per_vhead": 6 * C * pre["K"] + 4 * C * pre["V"] + 6 * pre["K"] * pre["V"]},
         "cpu_baseline": cpu_pre,

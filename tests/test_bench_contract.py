@@ -63,6 +63,33 @@ def test_pmc_summary_scales_by_the_copy_and_sums_dimensions(tmp_path):
     assert copy not in k
 
 
+def _counters(tmp_path, names):
+    for d, ctr in (("f", "FETCH_SIZE"), ("w", "WRITE_SIZE")):
+        _write_csv(str(tmp_path / d), [(1, "__amd_rocclr_copyBuffer", ctr, 256 * 1024)] +
+                   [(2 + i, f"void gdn::{n}(int)", ctr, 1024 << i) for i, n in enumerate(names)])
+    out = str(tmp_path / "traffic.json")
+    bench.pmc_summary(str(tmp_path / "f"), str(tmp_path / "w"), out)
+    return json.load(open(out))
+
+
+def test_pmc_summary_counts_every_kernel_of_a_chain_in_segments(tmp_path):
+    res = _counters(tmp_path, [
+        "chunk_prep_kernel<128, false, true, false>",                    # 1 MiB each way,
+        "chunk_head_kernel<128, 128, false, false, false, true>",        # 2, ...
+        "chunk_combine_kernel<128>", "chunk_head_kernel<128, 128, false, false, true, false>",
+        "chunk_prep_kernel<128, true, false, false>",
+        "chunk_head_kernel<128, 128, false, true, false, false>", "chunk_rev_sw_kernel<128>",
+        "chunk_head_kernel<128, 128, false, true, true, false>"])        # (a training forward)
+    assert res["prefill"] == 2 * (1 + 2 + 4 + 8) << 20
+    assert res["backward"] == 2 * (16 + 32 + 64) << 20
+
+
+def test_pmc_summary_refuses_a_pass_without_the_chain(tmp_path):
+    with pytest.raises(SystemExit):
+        _counters(tmp_path, ["chunk_prep_kernel<128, false, true, false>",
+                             "chunk_head_kernel<128, 128, false, false, false, true>"])
+
+
 def test_pmc_summary_needs_the_calibration_copy(tmp_path):
     _write_csv(str(tmp_path / "f"), [(1, "gdn::k(int)", "FETCH_SIZE", 1)])
     _write_csv(str(tmp_path / "w"), [(1, "gdn::k(int)", "WRITE_SIZE", 1)])
