@@ -16,12 +16,13 @@
 // a q outside fp16's range as the state-wave form's bf16 product).
 //
 // What bounds it: with a workgroup on every compute unit HBM (64 packed
-// sequences x 32 heads: 4.4 GB in 880 us, 5.0 TB/s; the state-wave form, whose
+// sequences x 32 heads: 3.9 GB in 876 us, 4.5 TB/s; the state-wave form, whose
 // eight workgroups per head each pull the chunk's 44 KiB of K, Q, Tb and P into
-// their compute units, ~1700 us); on its own ~1.9 us per chunk, instruction
-// issue: 120 MFMAs (1,920 cycles of the SIMD's matrix pipe), ~300 VALU and ~95
-// LDS instructions of the compute wave and ~200 of the helper wave beside it,
-// at the ~5 cycles a SIMD takes per VALU or MFMA instruction.  32 columns per
+// their compute units, ~1700 us); on its own 2.1 to 2.4 us per chunk (transfer
+// pass 1.3 to 1.5), instruction issue: per SIMD 120 MFMAs (1,920 cycles of its
+// matrix pipe), ~665 VALU and ~112 LDS instructions of its compute and its
+// helper wave, at the ~5 cycles a SIMD takes per VALU or MFMA instruction.  32
+// columns per
 // wave halve the LDS reads per product of 16 (one 1 KiB fragment, two MFMAs):
 // eight compute waves of 16 columns, staging themselves, took 2.5 us per
 // chunk, and a split into state and output waves 2.8.

@@ -86,7 +86,8 @@ extern "C" {
  * sequences (64 chunks and more) are run in segments, and so are those of a
  * packed batch that are far longer than its mean; their buffers (128 KiB per
  * v-head at K = V = 128 and segment that another follows) are part of the
- * workspace.  The fp32 state crosses their borders as fp32.
+ * workspace.  At their borders the fp32 state decays in fp32, and what a
+ * segment's tokens take out of it is a product of bf16 halves (2^-17).
  */
 int gdn_chunk_fwd(const void* q, const void* k, const void* v,
                   const float* g, const float* beta,
