@@ -475,13 +475,22 @@ __global__ __launch_bounds__(256) void conv1d_any_kernel(ConvArgs a) {
   }
 }
 
-// Rows with T == 0 still owe their final states (the initial states, or 0).
+// Final states by themselves, one lane per (b, d) row: for T == 0, and in place
+// of the initial ones, which other workgroups of the convolution read (input j
+// of a row's state is written after every read of it: inputs j and later).
 template <int DT, int W>
-__global__ __launch_bounds__(256) void conv1d_empty_final_kernel(ConvArgs a) {
-  const long long n = (long long)a.B * a.D * (W - 1);
+__global__ __launch_bounds__(256) void conv1d_final_kernel(ConvArgs a) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  ste<DT>(a.final_states, i, a.init ? lde<DT>(a.init, i) : 0.f);
+  if (i >= (long long)a.B * a.D) return;
+  const long long xr = i / a.D * a.x_sb + i % a.D * a.x_sd;
+#pragma unroll
+  for (int j = 0; j < W - 1; ++j) {
+    const int p = a.T - (W - 1) + j;
+    float v = 0.f;
+    if (p >= 0) v = lde<DT>(a.x, xr + p * a.x_st);
+    else if (a.init) v = lde<DT>(a.init, i * (W - 1) + (W - 1) + p);
+    ste<DT>(a.final_states, i * (W - 1) + j, v);
+  }
 }
 
 // ------------------------------------------------ causal conv1d update ----
@@ -778,20 +787,24 @@ int conv1d_cl_tile(long long rows, long long T) {
 }
 
 template <int DT, int W>
-int launch_conv(const gdn::ConvArgs& a, hipStream_t st) {
+int launch_conv(gdn::ConvArgs a, hipStream_t st) {
   const int N = vec_of(DT);
+  if (a.final_states && (a.T == 0 || a.final_states == a.init)) {
+    gdn::ConvArgs f = a;
+    if (a.T > 0) {
+      a.final_states = nullptr;
+      const int rc = launch_conv<DT, W>(a, st);
+      if (rc) return rc;
+    }
+    hipLaunchKernelGGL((gdn::conv1d_final_kernel<DT, W>),
+                       dim3((unsigned)(((long long)f.B * f.D + 255) / 256)), dim3(256), 0, st, f);
+    return gdn_host::check_launch("gdn_causal_conv1d_fwd");
+  }
   const bool vec_aligned_x = (reinterpret_cast<uintptr_t>(a.x) % 16) == 0;
   const bool vec_aligned_o = (reinterpret_cast<uintptr_t>(a.out) % 16) == 0;
   const bool vec_aligned_w = ((reinterpret_cast<uintptr_t>(a.weight) |
                                reinterpret_cast<uintptr_t>(a.bias)) % 16) == 0;
-  if (a.T == 0) {
-    if (a.final_states) {
-      const long long n = (long long)a.B * a.D * (W - 1);
-      hipLaunchKernelGGL((gdn::conv1d_empty_final_kernel<DT, W>), dim3(grid_for(n, 256)),
-                         dim3(256), 0, st, a);
-    }
-    return gdn_host::check_launch("gdn_causal_conv1d_fwd");
-  }
+  if (a.T == 0) return gdn_host::check_launch("gdn_causal_conv1d_fwd");
   if (a.x_sd == 1 && a.o_sd == 1 && a.D % N == 0 && a.x_sb % N == 0 && a.x_st % N == 0 &&
       a.o_sb % N == 0 && a.o_st % N == 0 && vec_aligned_x && vec_aligned_o && vec_aligned_w) {
     const int TT = conv1d_cl_tile((a.D / N + 255) / 256 * (long long)a.B, a.T);

@@ -90,7 +90,8 @@ int gdn_l2norm_fwd(const void* x, void* y, long long rows, int D, float eps, int
  *           only reads tokens with the same seq_idx (packed varlen).
  *   initial_states [B, D, W-1] nullable, final_states [B, D, W-1]
  *           nullable (contiguous, x's dtype; channel-last only): the W-1
- *           inputs before / at the end of each batch row.
+ *           inputs before / at the end of each batch row; they may be one
+ *           buffer (updated in place).
  */
 int gdn_causal_conv1d_fwd(const void* x, const void* weight, const void* bias,
                           const int32_t* seq_idx, const void* initial_states,

@@ -188,6 +188,24 @@ def test_conv_fn_time_tiles(rocm_device, B, T, given):
     _close_lowp(got, ref, f"conv B{B} T{T} {given}")
 
 
+@pytest.mark.parametrize("layout", ["channel_last", "strided"])
+@pytest.mark.parametrize("T", [1, 2, 3, 8, 9, 33, 64, 65, 200])
+def test_conv_fn_states_in_place(rocm_device, T, layout):
+    """final_states_out that is initial_states: the same bits as apart from it, over one time tile
+    and over several, whose first reads what the last one writes."""
+    x, w, bias = _conv_case(rocm_device, 3, 64, T, 4, torch.bfloat16, layout, seed=T)
+    init = _rand((3, 64, 3), rocm_device, seed=17)
+    want, fin = L.causal_conv1d_fn(x, w, bias, initial_states=init, return_final_states=True,
+                                   activation="silu")
+    state = init.clone()
+    out, same = L.causal_conv1d_fn(x, w, bias, initial_states=state, return_final_states=True,
+                                   final_states_out=state, activation="silu")
+    torch.cuda.synchronize()
+    assert same is state and torch.equal(out, want) and torch.equal(state, fin)
+    _, fref = LR.causal_conv1d(_np(x), _np(w), _np(bias), initial_states=_np(init), silu=True)
+    np.testing.assert_array_equal(_np(state), fref)
+
+
 def test_conv_fn_qwen3_next_shape(rocm_device):
     """Layer shape (conv_dim 8192, T 8192, channel-last bf16): oracle on 96 channels."""
     dev = rocm_device
