@@ -116,8 +116,9 @@ size_t gdn_chunk_workspace_bytes(int B, int T, int Hqk, int Hv, int K, int V,
  * The array is part of libgdn.so's device code object: every process that
  * loads the library holds those 32 MiB on every GPU it uses, until it ends,
  * whether or not it calls this entry point.
- * It never runs in segments (whose buffers would not fit), so that where
- * gdn_chunk_fwd does, the two agree to rounding, else bit for bit.
+ * It never runs in segments (whose buffers would not fit), nor in another
+ * form than its scratch holds, so that where gdn_chunk_fwd does, the two agree
+ * to rounding, else bit for bit.
  * Problems whose workspace without segments exceeds 32 MiB (about 5,300
  * tokens at 32 v-heads / 16 qk-heads, K = V = 128; about 2,300 with
  * use_qk_l2norm, whose chain reads fp16 copies of the normalised q, k rows

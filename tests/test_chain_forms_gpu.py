@@ -158,9 +158,10 @@ def test_segments_packed(rocm_device, lens):
                   h0_scale=0.05), rocm_device, what=str(lens))
 
 
-@pytest.mark.parametrize("T,Hv,n", [(9000, 2, 2), (400, 8, 64)])
+@pytest.mark.parametrize("T,Hv,n", [(9000, 2, 2), (400, 8, 64), (3000, 8, 32), (12500, 32, 4)])
 def test_violated_cu_seqlens(rocm_device, T, Hv, n):
-    """The device contract in both forms: o zero-filled, the final state the initial one."""
+    """The device contract in segments, whole heads, with long sequences listed and with long ones
+    cut: o zero-filled, the final state the initial one."""
     wl = W.make(1, T, 1, Hv, 128, 128, seed=3, cu_seqlens=_cu([T // n] * n))
     t = wl.torch(rocm_device)
     from avelang_amd import chunk_gated_delta_rule
@@ -353,3 +354,38 @@ def test_in_the_workspace_of_a_larger_problem(rocm_device, small, large):
     assert least < size(small)
     with pytest.raises(ValueError, match="workspace needs"):
         _run(wl, rocm_device, workspace=ws[:least - 1])
+
+
+@pytest.mark.parametrize("longs", [(), (3000,), (1000, 500, 7, 1500)])
+def test_noalloc_takes_the_same_form_of_a_packed_batch(rocm_device, longs):
+    """Long sequences in state waves beside whole heads, in the library's scratch: bit for bit."""
+    from avelang_amd import _native
+    wl = _packed(rocm_device, longs=longs)
+    d, t = wl.dims, wl.torch(rocm_device)
+    o, s = _run(wl, rocm_device)
+    o2, s2 = torch.full_like(o, 5.0), torch.full_like(s, 5.0)
+    rc = _native.lib().gdn_chunk_fwd_noalloc(
+        *(t[n].data_ptr() for n in ("q", "k", "v", "g", "beta", "initial_state")), s2.data_ptr(),
+        o2.data_ptr(), t["cu_seqlens"].data_ptr(),
+        *(d[n] for n in ("B", "T", "Hqk", "Hv", "K", "V", "N")), 128 ** -0.5, 0,
+        torch.cuda.current_stream(rocm_device).cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0, _native.last_error()
+    assert torch.equal(o, o2) and torch.equal(s, s2)
+
+
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 64), (128, 64), (64, 128)])
+def test_q_rows_of_many_magnitudes(rocm_device, K, V):
+    """Whole heads: every token's q times a power of two of its own (2^-6 to 2^6) gives its o times
+    that (to a bf16 rounding of each: P is rounded to fp16, whose subnormals the small rows reach)."""
+    from avelang_amd import chunk_gated_delta_rule
+    B = -(-_cus(rocm_device) // 4)
+    t = W.make(B, 130, 2, 4, K, V, seed=15, h0_scale=0.05, decay=0.01).torch(rocm_device)
+    gen = torch.Generator().manual_seed(1)
+    f = 2.0 ** torch.randint(-6, 7, (B, 130, 1, 1), generator=gen).to(rocm_device)
+    o, o2 = (chunk_gated_delta_rule((t["q"].float() * x).to(torch.bfloat16), t["k"], t["v"], t["g"],
+                                    t["beta"], initial_state=t["initial_state"])[0].float()
+             for x in (torch.ones_like(f), f))
+    torch.cuda.synchronize()
+    off = (o2 - f * o).norm(dim=-1) / (f * o).norm(dim=-1)
+    assert off.max() <= 2 ** -7, off.max()
