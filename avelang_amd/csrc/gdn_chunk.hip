@@ -574,7 +574,7 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 //
 // The state-wave form (a workgroup per 16 value columns) goes through a chunk
 // in ~0.86 us while W x 8 workgroups leave compute units free, the whole-head
-// form in ~1.9 us with an eighth of the operand traffic.  So the latter pays
+// form in 2.1 to 2.5 with an eighth of the operand traffic.  So the latter pays
 //  - unsegmented once W fills half the GPU: W = 128 (4 x 32 heads of T = 4096)
 //    276 -> 220 us per prefill, W = 256 (8 x 32 of 2048) 282 -> 187, 64 packed
 //    sequences x 32 heads 2346 -> 1500; at W = 64 it loses (128 -> 159).  With
@@ -598,9 +598,10 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // workgroups (two per segment, the first and last 1 and 0: W (2 ns - 3), one
 // per compute unit, 64-wide heads' two; at W = 32, T = 8192 5 segments 138 us,
 // 4 155, 6 159, 8 152; a few workgroups over cost a second round: W = 24,
-// T = 32768 in 7 segments 519, in 6 440, W = 112 in 3 1837, in 2 1464), and balances the
-// passes over a segment (~3.5 us per chunk) against the serial combine (~1.2
-// us per segment; W = 4, T = 20011 25 segments 97 us, 16 106, 12 120).
+// T = 32768 in 7 segments 519, in 6 440, W = 112 in 3 1837, in 2 1464), and
+// balances the passes over a segment (~3.5 us per chunk) against the serial
+// combine (~1.2 us per segment; W = 4, T = 20011 25 segments 97 us, 16 106, 12
+// 120).
 // With cu_seqlens nct is the mean, and the device alone knows the lengths
 // (chunk_table_kernel).  Its measure is the load, the chunks that a compute
 // unit would have of an even batch: whole heads take 2.5 us per chunk of the

@@ -74,9 +74,10 @@ struct HeadArgs {
 // Segments.  Sequence n's chunks are cut into segments of `seg` chunks (one
 // at least, also for an empty sequence); ws.soff[n] is its first segment's
 // global index with cu_seqlens (chunk_table_kernel, which leaves those of
-// `cut` chunks and less in one), n times a constant without.  Every segment but a sequence's last is full; ws.segs and ws.segm
-// hold the full ones alone, which the n last segments before are left out of:
-// segment j of sequence n is full segment first + j - n.
+// WsPlan::cut chunks and less in one), n times a constant without.  Every
+// segment but a sequence's last is full; ws.segs and ws.segm hold the full ones
+// alone, so without the last ones of the n sequences before: segment j of
+// sequence n is full segment first + j - n.
 __device__ __forceinline__ void seg_range(int n, int seg, const int32_t* cu, int T,
                                           const ChunkWs& ws, int& first, int& count) {
   if (cu) {
