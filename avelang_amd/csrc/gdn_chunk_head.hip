@@ -11,9 +11,8 @@
 // stands; so the compute waves exchange nothing and one barrier per chunk
 // hands the operand buffers over.  Every product takes fp16 operands rounded
 // from fp32 (K and V rows as fp16, exact in fp16's normal range; the caller's
-// Q rows times a power of two that brings the largest of 16 or 32 rows to
-// 2^14 .. 2^15, taken back from the output's factor: Q S is then as exact for
-// a q outside fp16's range as the state-wave form's bf16 product).
+// Q rows times a power of two, taken back from the output's factor: Q S is then
+// as exact for a q outside fp16's range as the state-wave form's bf16 product).
 //
 // What bounds it: with a workgroup on every compute unit HBM (64 packed
 // sequences x 32 heads: 3.9 GB in 876 us, 4.5 TB/s; the state-wave form, whose
@@ -22,10 +21,9 @@
 // pass 1.3 to 1.5), instruction issue: per SIMD 120 MFMAs (1,920 cycles of its
 // matrix pipe), ~665 VALU and ~112 LDS instructions of its compute and its
 // helper wave, at the ~5 cycles a SIMD takes per VALU or MFMA instruction.  32
-// columns per
-// wave halve the LDS reads per product of 16 (one 1 KiB fragment, two MFMAs):
-// eight compute waves of 16 columns, staging themselves, took 2.5 us per
-// chunk, and a split into state and output waves 2.8.
+// columns per wave halve the LDS reads per product of 16 (one 1 KiB fragment,
+// two MFMAs): eight compute waves of 16 columns, staging themselves, took 2.5
+// us per chunk, and a split into state and output waves 2.8.
 //
 // Staging: as many helper waves hold the next three chunks' K, Q and V units
 // and Tb / P fragments in registers (a load has two steps to land) and write
@@ -163,32 +161,12 @@ __device__ __forceinline__ u16x8 scale_h8(u16x8 x, float s) {
   return cat8(fma_h4(f32x4{f[0], f[1], f[2], f[3]}, s4, kNegZero4),
               fma_h4(f32x4{f[4], f[5], f[6], f[7]}, s4, kNegZero4));
 }
-// Biased exponent of the largest |x| of a wave's bf16 values, 15 at least (so
-// that 2^(141 - e) and its inverse are normal floats; 255: an inf or NaN).
-template <int N>
-__device__ __forceinline__ int q_exponent(const u32x4 (&x)[N]) {
-  float m = 0.f;
+// The larger of m and every |x| of eight bf16 values (NaN left out).
+__device__ __forceinline__ float max_abs8(u32x4 x, float m) {
 #pragma unroll
-  for (int i = 0; i < N; ++i) {
-#pragma unroll
-    for (int y = 0; y < 4; ++y)   // (both values of the word, sign bits ignored)
-      asm("v_max3_f32 %0, |%1|, |%2|, %0"
-          : "+v"(m) : "v"(x[i][y] << 16), "v"(x[i][y] & 0xffff0000u));
-  }
-  unsigned u = __float_as_uint(m);
-  auto ror = [&](auto n) {
-    u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x120 + decltype(n)::value, 0xf, 0xf,
-                                                     false));
-  };
-  ror(std::integral_constant<int, 8>{});
-  ror(std::integral_constant<int, 4>{});
-  ror(std::integral_constant<int, 2>{});
-  ror(std::integral_constant<int, 1>{});
-  unsigned top = 0;
-#pragma unroll
-  for (int row = 0; row < 4; ++row)
-    top = max(top, (unsigned)__builtin_amdgcn_readlane((int)u, 16 * row));
-  return max((int)(top >> 23), 15);
+  for (int y = 0; y < 4; ++y)
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(x[y] << 16), "v"(x[y] & 0xffff0000u));
+  return m;
 }
 
 // Workgroup bid of nb with a qk-head group's workgroups on one XCD (they read the
@@ -312,9 +290,6 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
     };
     auto stage = [&](const Regs& r, int j, int b) {
       unsigned char* bp = buf + b * kBufStep;
-      int qe = 141;   // biased exponent of this wave's Q rows, its scale 2^(141 - qe)
-      if constexpr (kRowsQ) qe = q_exponent(r.q);
-      const float qs = __int_as_float((268 - qe) << 23);
 #pragma unroll
       for (int i = 0; i < KPT; ++i) {
         const int x = tid + HT * i;
@@ -324,9 +299,6 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
         } else {
           *reinterpret_cast<u16x8*>(bp + KL::off(x / UPR, x % UPR)) =
               bf2h8(__builtin_bit_cast(u16x8, r.k[i]));
-          if constexpr (OUT)
-            *reinterpret_cast<u16x8*>(bp + kQ + qrow_off<K>(x / UPR, x % UPR)) =
-                scale_h8(__builtin_bit_cast(u16x8, r.q[i]), qs);
         }
       }
 #pragma unroll
@@ -339,11 +311,42 @@ __global__ __launch_bounds__(4 * V) void chunk_head_kernel(HeadArgs a, ChunkWs w
       for (int i = 0; i < SPW; ++i)
         if (hw + NW * i < NSL)
           *reinterpret_cast<u32x4*>(bp + kF + 1024 * (hw + NW * i) + 16 * lane) = r.f[i];
-      // the output's factor scale e^G of this wave's rows, the Q scale taken back
-      if constexpr (OUT) {
+      // Q rows as fp16 times a power of two, and the output's factor scale e^G with
+      // it taken back: 2^8 where this wave's rows are in range of it, else one for
+      // each row by its largest element
+      if constexpr (kRowsQ) {
+        float top = 0.f;
+#pragma unroll
+        for (int i = 0; i < KPT; ++i) top = max_abs8(r.q[i], top);
+        if (!__any(top >= 256.f) && __any(top >= 0x1p-13f)) {
+#pragma unroll
+          for (int i = 0; i < KPT; ++i) {
+            const int x = tid + HT * i;
+            *reinterpret_cast<u16x8*>(bp + kQ + qrow_off<K>(x / UPR, x % UPR)) =
+                scale_h8(__builtin_bit_cast(u16x8, r.q[i]), 256.f);
+          }
+          if (lane / (64 / UPR) % NW == hw)
+            *reinterpret_cast<float*>(bp + kO + 4 * lane) = a.scale * __expf(r.g) * 0x1p-8f;
+        } else {
+#pragma unroll
+          for (int i = 0; i < KPT; ++i) {
+            const int x = tid + HT * i, row = x / UPR;
+            unsigned m = __float_as_uint(max_abs8(r.q[i], 0.f));
+#pragma unroll
+            for (int d = 1; d < UPR; d *= 2) m = max(m, (unsigned)__shfl_xor((int)m, d));
+            // the largest element to 2^14 .. 2^15, both factors normal floats
+            const int e = max((int)(m >> 23), 15);
+            *reinterpret_cast<u16x8*>(bp + kQ + qrow_off<K>(row, x % UPR)) =
+                scale_h8(__builtin_bit_cast(u16x8, r.q[i]), __int_as_float((268 - e) << 23));
+            const float g = __shfl(r.g, row);
+            if (x % UPR == 0)
+              *reinterpret_cast<float*>(bp + kO + 4 * row) =
+                  a.scale * __expf(g) * __int_as_float((e - 14) << 23);
+          }
+        }
+      } else if constexpr (OUT) {
         if (lane / (64 / UPR) % NW == hw)
-          *reinterpret_cast<float*>(bp + kO + 4 * lane) =
-              a.scale * __expf(r.g) * __int_as_float((qe - 14) << 23);
+          *reinterpret_cast<float*>(bp + kO + 4 * lane) = a.scale * __expf(r.g);
       }
       if (hw == NW - 1) {
         const int L = min(kChunk, e - (s + j * kChunk));

@@ -78,8 +78,8 @@ extern "C" {
  * of the exact recurrence at any length.  Without use_qk_l2norm the output's
  * q.S term is, for few short chains, a bf16 MFMA product (q as given, the
  * state rounded to bf16), and for many or long chains an fp16 one (the state
- * as fp16, q times a power of two per group of rows, so that its own size does
- * not matter); with use_qk_l2norm it is an fp16 one (the normalised q as
+ * as fp16, q times a power of two, 2^8 or one per row, so that its own size
+ * does not matter); with use_qk_l2norm it is an fp16 one (the normalised q as
  * fp16); gdn_chunk_fwd_save gives the same o as gdn_chunk_fwd but where only
  * the latter runs in segments (see there).
  * P = scale q.k e^(G_i - G_j) is rounded to fp16 in every form.  Few long

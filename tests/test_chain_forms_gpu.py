@@ -376,16 +376,42 @@ def test_noalloc_takes_the_same_form_of_a_packed_batch(rocm_device, longs):
 
 @pytest.mark.parametrize("K,V", [(128, 128), (64, 64), (128, 64), (64, 128)])
 def test_q_rows_of_many_magnitudes(rocm_device, K, V):
-    """Whole heads: every token's q times a power of two of its own (2^-6 to 2^6) gives its o times
-    that (to a bf16 rounding of each: P is rounded to fp16, whose subnormals the small rows reach)."""
+    """Whole heads: every token's q times a power of two of its own (2^-6 to 2^6, and 2^-12 to 2^12:
+    under and over the 256 where each row takes a scale of its own) gives its o times that (to a
+    bf16 rounding of each: P is rounded to fp16, whose subnormals the small rows reach; the scale
+    keeps it between them and fp16's largest)."""
     from avelang_amd import chunk_gated_delta_rule
     B = -(-_cus(rocm_device) // 4)
     t = W.make(B, 130, 2, 4, K, V, seed=15, h0_scale=0.05, decay=0.01).torch(rocm_device)
     gen = torch.Generator().manual_seed(1)
-    f = 2.0 ** torch.randint(-6, 7, (B, 130, 1, 1), generator=gen).to(rocm_device)
-    o, o2 = (chunk_gated_delta_rule((t["q"].float() * x).to(torch.bfloat16), t["k"], t["v"], t["g"],
-                                    t["beta"], initial_state=t["initial_state"])[0].float()
-             for x in (torch.ones_like(f), f))
+    for top in (6, 12):
+        f = 2.0 ** torch.randint(-top, top + 1, (B, 130, 1, 1), generator=gen).to(rocm_device)
+        o, o2 = (chunk_gated_delta_rule((t["q"].float() * x).to(torch.bfloat16), t["k"], t["v"],
+                                        t["g"], t["beta"], scale=K ** -0.5 * 64,
+                                        initial_state=t["initial_state"])[0].float()
+                 for x in (torch.ones_like(f), f))
+        torch.cuda.synchronize()
+        off = (o2 - f * o).norm(dim=-1) / (f * o).norm(dim=-1)
+        assert off.max() <= 2 ** -7, (top, off.max())
+
+
+@pytest.mark.parametrize("what", ["state waves", "whole heads", "segments"])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan"), 2.0 ** 100])
+def test_a_token_of_q_out_of_range_leaves_the_others(rocm_device, what, bad):
+    """Without l2norm an inf, NaN or outlier in one token's q changes that token's o alone, in every
+    form (its neighbours share the helper wave that scales their rows)."""
+    from avelang_amd import chunk_gated_delta_rule
+    B = -(-_cus(rocm_device) // 4)
+    shape = {"state waves": (1, 200, 2, 4), "whole heads": (B, 130, 2, 4),
+             "segments": (1, 4400, 1, 2)}[what]
+    t = W.make(*shape, 128, 128, seed=16, h0_scale=0.05, decay=0.01).torch(rocm_device)
+    token = 70
+    q2 = t["q"].clone()
+    q2[:, token, :, 5] = bad
+    o, o2 = (chunk_gated_delta_rule(q, t["k"], t["v"], t["g"], t["beta"],
+                                    initial_state=t["initial_state"])[0] for q in (t["q"], q2))
     torch.cuda.synchronize()
-    off = (o2 - f * o).norm(dim=-1) / (f * o).norm(dim=-1)
-    assert off.max() <= 2 ** -7, off.max()
+    others = torch.arange(shape[1], device=rocm_device) != token
+    assert torch.equal(o[:, others], o2[:, others])
+    if bad == 2.0 ** 100:   # (finite in fp32 sums, out of fp16's P: inf or NaN, never plausible)
+        assert not torch.equal(o[:, token], o2[:, token])
